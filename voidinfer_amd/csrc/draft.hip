@@ -115,91 +115,152 @@ __global__ __launch_bounds__(kDraftLanes) void draft_choice_kernel(int lanes, in
 // over the unary scores decides instead (the selector's terms are not
 // calibrated as logits).
 //
-// One wave per lane, the rank-256 dot in registers: lane k holds ranks
-// 4k .. 4k + 3 of pred[anchor] * hidden[pos] and of every candidate's succ row
-// (8-byte loads, each candidate row read by the wave in one 512-byte sweep);
-// the 16 candidate sums are reduced across the wave with DPP in a fixed order.
-// The next anchor is one of this position's candidates, so their pred rows are
-// loaded with their succ rows and the chosen one is kept: no load waits on the
-// choice.  The order of the fp32 sums is this kernel's own; near ties may
-// therefore resolve differently from another order, within the sums'
-// rounding.
+// Bound: latency.  The chain is serial (a position's anchor is the one before's
+// choice), but everything it reads is known beforehand: position p's possible
+// anchors are position p - 1's candidates.  So one workgroup takes a lane and
+// requests a whole chunk of positions at once: the candidates' succ rows and the
+// hidden rows into registers, their pred rows on to LDS.  The serial part is then
+// one LDS read of the anchor's row, the dots, one barrier and a 16-lane maximum
+// per position.
+// Four waves, each four candidates (a CU has four SIMDs: more waves would repeat
+// the maximum on the same issue slots).  Lane k of a wave holds ranks
+// 4k .. 4k + 3; the candidate sums are reduced across the wave with DPP in a
+// fixed order.  That order is this kernel's own; near ties may therefore resolve
+// differently from another order, within the sums' rounding.  Measured, 8 lanes x
+// 16 positions over a 248,320-token codebook: 14.9 us per call, 47.4 with one wave per
+// lane loading each position after the one before.
 constexpr int kRank = 256;
-constexpr int kChainWaves = 4;                     // lanes per workgroup, one wave each
+constexpr int kChainWaves = 4;
 constexpr int kChainThreads = kChainWaves * kWave;
 constexpr int kRanksPerLane = kRank / kWave;       // 4
+constexpr int kChainMax = 16;                      // positions per chunk (the largest)
 static_assert(kRanksPerLane == 4, "four fp16 ranks = one 8-byte load");
+static_assert(kDraftK == 4 * kChainWaves, "four candidates per wave");
 
-// ranks 4k .. 4k + 3 of an fp16 row, as fp32
-__device__ __forceinline__ float4 rank4(const uint16_t* row, int k) {
-    const uint2 v = *reinterpret_cast<const uint2*>(row + kRanksPerLane * k);
+__device__ __forceinline__ float4 decode4(uint2 v) {
     return make_float4(Elem<VI_F16>::decode(v.x & 0xffffu), Elem<VI_F16>::decode(v.x >> 16),
                        Elem<VI_F16>::decode(v.y & 0xffffu), Elem<VI_F16>::decode(v.y >> 16));
 }
+// ranks 4k .. 4k + 3 of an fp16 row
+__device__ __forceinline__ uint2 rank4(const uint16_t* row, int k) {
+    return *reinterpret_cast<const uint2*>(row + kRanksPerLane * k);
+}
+// Index of the first maximum of 16 scores held one per lane in every 16-lane
+// row (score[0] wins if it is NaN; another NaN never wins): the serial rule
+// "replace when greater" as a maximum over order keys.
+__device__ __forceinline__ int first_max16_lanes(float score, int c) {
+    const uint32_t b = __builtin_bit_cast(uint32_t, score + 0.0f);   // -0 and +0 compare equal
+    const bool nan = (b & 0x7fffffffu) > 0x7f800000u;
+    const uint32_t key = nan ? (c == 0 ? 0xffffffffu : 0u) : ((b & 0x80000000u) ? ~b : (b | 0x80000000u));
+    uint32_t m = key;
+    m = max(m, lanes_xor_dpp<1>(m));
+    m = max(m, lanes_xor_dpp<2>(m));
+    m = max(m, lanes_xor_dpp<4>(m));
+    m = max(m, lanes_xor_dpp<8>(m));
+    return __builtin_ctzll(ballot(key == m));
+}
 
+template <int CH>   // positions per chunk
 __global__ __launch_bounds__(kChainThreads) void selector_chain_kernel(
-    int lanes, int positions, int vocabulary, const int64_t* anchors, const int64_t* candidates, const float* unary,
+    int positions, int vocabulary, const int64_t* anchors, const int64_t* candidates, const float* unary,
     const uint16_t* hidden, const uint16_t* pred_cb, const uint16_t* succ_cb, const vi_draft_sampling* sampling,
     int64_t* proposals) {
-    __shared__ float s_val[kChainWaves][kDraftK + 1], s_prob[kChainWaves][kDraftK + 1];
-    __shared__ int s_ord[kChainWaves][kDraftK + 1];
-    const int w = threadIdx.x / kWave, k = lane_id();
-    const int l = blockIdx.x * kChainWaves + w;
-    if (l >= lanes) return;   // (a whole wave)
+    __shared__ __attribute__((aligned(16))) uint16_t s_pred[CH][kDraftK][kRank];
+    __shared__ int s_cand[CH][kDraftK];
+    __shared__ float s_unary[CH][kDraftK];
+    __shared__ __attribute__((aligned(16))) float s_score[2][kDraftK];
+    __shared__ int s_valid[kChainWaves];
+    __shared__ float s_val[kDraftK], s_prob[kDraftK];
+    __shared__ int s_ord[kDraftK];
+    const int t = threadIdx.x, w = t / kWave, k = lane_id(), l = blockIdx.x;
     const int64_t seed_token = anchors[l];
-    const vi_draft_sampling smp = sampling ? sampling[l] : vi_draft_sampling{};
-    const bool sampled = sampling && smp.inv_temperature > 0.0f;
     int64_t* out = proposals + size_t(l) * positions;
-    bool bad = seed_token < 0 || seed_token >= vocabulary;
+    const int64_t* lane_cand = candidates + size_t(l) * positions * kDraftK;
+    const float* lane_unary = unary + size_t(l) * positions * kDraftK;
+    bool bad = seed_token < 0 || seed_token >= vocabulary;   // ends the chain (workgroup-uniform)
+    if (sampling && sampling[l].inv_temperature > 0.0f) {
+        // the coupled choice over the unary scores: serial, one wave
+        if (w != 0) return;
+        const vi_draft_sampling smp = sampling[l];
+        for (int pos = 0; pos < positions; ++pos) {
+            const int64_t* cd = lane_cand + size_t(pos) * kDraftK;
+            const int64_t mine = cd[k & (kDraftK - 1)];
+            bad = bad || ballot(mine < 0 || mine >= vocabulary) != 0;
+            if (k != 0) continue;
+            if (bad) { out[pos] = -1; continue; }
+            const int best = sampled_pick(smp, pos, vocabulary, lane_unary + size_t(pos) * kDraftK, cd, seed_token, out,
+                                          s_val, s_prob, s_ord);
+            out[pos] = cd[best];
+        }
+        return;
+    }
     // pred[anchor] of the current position (ranks 4k .. 4k + 3)
-    float4 pa = bad || sampled ? make_float4(0.f, 0.f, 0.f, 0.f) : rank4(pred_cb + size_t(seed_token) * kRank, k);
-    for (int pos = 0; pos < positions; ++pos) {
-        const size_t at = size_t(l) * positions + pos;
-        const int64_t* cd = candidates + at * kDraftK;
-        int64_t cand[kDraftK];
-#pragma unroll
-        for (int c = 0; c < kDraftK; ++c) {
-            cand[c] = cd[c];
-            bad = bad || cand[c] < 0 || cand[c] >= vocabulary;
+    uint2 pa = rank4(pred_cb + size_t(bad ? 0 : seed_token) * kRank, k);
+    for (int p0 = 0; p0 < positions; p0 += CH) {
+        // the chunk's candidates and unary scores, and the positions up to the
+        // first invalid candidate
+        const int n = min(CH, positions - p0);
+        int firstbad = CH;
+        for (int i = t; i < CH * kDraftK; i += kChainThreads) {
+            const int p = i / kDraftK, c = i % kDraftK;
+            const bool in = p < n;
+            const size_t at = size_t(p0 + (in ? p : n - 1)) * kDraftK + c;
+            const int64_t id = lane_cand[at];
+            const bool ok = id >= 0 && id < vocabulary;
+            if (in && !ok) firstbad = min(firstbad, p);
+            s_cand[p][c] = ok ? int(id) : 0;
+            s_unary[p][c] = lane_unary[at];
         }
-        if (bad) {   // an anchor or a candidate outside the codebooks: no proposal from here on
-            if (k == 0) out[pos] = -1;
-            continue;
-        }
-        int best = 0;
-        if (sampled) {
-            if (k == 0)
-                best = sampled_pick(smp, pos, vocabulary, unary + at * kDraftK, cd, seed_token, out, s_val[w],
-                                    s_prob[w], s_ord[w]);
-            best = __builtin_amdgcn_readfirstlane(best);
-        } else {
-            // every load of this position first: hidden, the candidates' succ rows
-            // and their pred rows (the next anchor's)
-            const float4 h = rank4(hidden + at * kRank, k);
-            float4 sv[kDraftK], pv[kDraftK];
 #pragma unroll
-            for (int c = 0; c < kDraftK; ++c) {
-                sv[c] = rank4(succ_cb + size_t(cand[c]) * kRank, k);
-                pv[c] = rank4(pred_cb + size_t(cand[c]) * kRank, k);
+        for (int m = 1; m < kWave; m <<= 1) firstbad = min(firstbad, __shfl_xor(firstbad, m, kWave));
+        if (k == 0) s_valid[w] = firstbad;
+        __syncthreads();   // (and the previous chunk's LDS rows are free)
+        int valid = bad ? 0 : n;
+#pragma unroll
+        for (int i = 0; i < kChainWaves; ++i) valid = min(valid, s_valid[i]);
+        valid = __builtin_amdgcn_readfirstlane(valid);
+        bad = bad || valid < n;
+        if (t >= valid && t < n) out[p0 + t] = -1;   // n <= the workgroup's threads
+        if (valid == 0) { __syncthreads(); continue; }
+        // every row of the chunk in flight (positions past the end repeat the last
+        // one's; never used)
+        uint2 h[CH], sv[CH][4], pv[CH][4];
+#pragma unroll
+        for (int p = 0; p < CH; ++p) {
+            const int q = min(p, valid - 1);
+            h[p] = rank4(hidden + (size_t(l) * positions + size_t(p0 + q)) * kRank, k);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const size_t id = size_t(s_cand[q][4 * w + j]);
+                sv[p][j] = rank4(succ_cb + id * kRank, k);
+                pv[p][j] = rank4(pred_cb + id * kRank, k);
             }
-            const float4 ah = make_float4(pa.x * h.x, pa.y * h.y, pa.z * h.z, pa.w * h.w);
-            float score[kDraftK];
-#pragma unroll
-            for (int c = 0; c < kDraftK; ++c) {
-                const float part = (ah.x * sv[c].x + ah.y * sv[c].y) + (ah.z * sv[c].z + ah.w * sv[c].w);
-                score[c] = unary[at * kDraftK + c] + wave_sum_f32(part);
-            }
-            // first maximum (NaN never replaces the incumbent); scores are wave-uniform
-            float bs = score[0];
-#pragma unroll
-            for (int c = 1; c < kDraftK; ++c)
-                if (score[c] > bs) { bs = score[c]; best = c; }
-            // the chosen candidate's pred row is the next position's anchor row
-#pragma unroll
-            for (int c = 0; c < kDraftK; ++c)
-                if (c == best) pa = pv[c];
         }
-        if (k == 0) out[pos] = cand[best];
+#pragma unroll
+        for (int p = 0; p < CH; ++p)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                *reinterpret_cast<uint2*>(&s_pred[p][4 * w + j][kRanksPerLane * k]) = pv[p][j];
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < CH; ++p) {
+            if (p >= valid) continue;   // (workgroup-uniform)
+            const float4 a = decode4(pa), hh = decode4(h[p]);
+            const float4 ah = make_float4(a.x * hh.x, a.y * hh.y, a.z * hh.z, a.w * hh.w);
+            float sc[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float4 s = decode4(sv[p][j]);
+                sc[j] = wave_sum_f32((ah.x * s.x + ah.y * s.y) + (ah.z * s.z + ah.w * s.w));
+            }
+            if (k == 0) *reinterpret_cast<float4*>(&s_score[p & 1][4 * w]) = make_float4(sc[0], sc[1], sc[2], sc[3]);
+            __syncthreads();
+            const int c = k & (kDraftK - 1);
+            const int best = first_max16_lanes(s_unary[p][c] + s_score[p & 1][c], c);
+            pa = *reinterpret_cast<const uint2*>(&s_pred[p][best][kRanksPerLane * k]);   // the next anchor's row
+            if (t == 0) out[p0 + p] = s_cand[p][best];
+        }
+        __syncthreads();   // the chunk's rows are read
     }
 }
 }  // namespace
@@ -216,11 +277,13 @@ vi_status launch_selector_chain(int lanes, int positions, int vocabulary, const 
                                 const int64_t* candidates, const float* unary, const void* hidden,
                                 const void* pred_codebook, const void* succ_codebook,
                                 const vi_draft_sampling* sampling, int64_t* proposals, hipStream_t stream) {
-    hipLaunchKernelGGL(selector_chain_kernel, dim3((lanes + kChainWaves - 1) / kChainWaves), dim3(kChainThreads), 0,
-                       stream, lanes, positions, vocabulary,
-                       anchors, candidates, unary, static_cast<const uint16_t*>(hidden),
-                       static_cast<const uint16_t*>(pred_codebook), static_cast<const uint16_t*>(succ_codebook),
-                       sampling, proposals);
+    // the smallest chunk that holds the chain: its rows are all requested at once
+    auto* kernel = positions <= 4 ? &selector_chain_kernel<4>
+                   : positions <= 8 ? &selector_chain_kernel<8>
+                                    : &selector_chain_kernel<kChainMax>;
+    hipLaunchKernelGGL(kernel, dim3(lanes), dim3(kChainThreads), 0, stream, positions, vocabulary, anchors, candidates,
+                       unary, static_cast<const uint16_t*>(hidden), static_cast<const uint16_t*>(pred_codebook),
+                       static_cast<const uint16_t*>(succ_codebook), sampling, proposals);
     return launch_status();
 }
 
