@@ -156,3 +156,51 @@ def test_scores_many_rows_and_rejects(orc, dev):
     assert lib.vi_sampled_scores(t.data_ptr(), 1, rows, vocab, vocab, C.byref(dcfg), 0, -1.0, 0, 0, 0, None, 0,
                                  None) == 1
     assert lib.vi_row_scores(t.data_ptr(), 1, rows, vocab, vocab - 1, 0, 0, 0, None, 0, None) == 1
+
+
+@pytest.mark.parametrize("presence", [0.0, 0.6, -0.75, 1e38])
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_sampled_scores_batched_scan(orc, dev, dtype, presence):
+    """The packet scan's batches: rows shorter and longer than a batch, ties past
+    the candidate pool, non-finite logits, logits past the dtype's penalty guard,
+    penalties that raise logits and one too large to batch."""
+    import voidinfer_amd as vi
+    first_key, cfg = 40, dict(temperature=0.7, top_k=0, top_p=0.9, min_p=0.01, seed=31)
+    for vocab in (7, 64, 2049, 40_003):
+        rng = np.random.default_rng(vocab * 4 + dtype)
+        rows = 9
+        x = (rng.standard_normal((rows, vocab)) * 1.5).astype(np.float32)
+        x[1] = 1.0                                            # every logit equal
+        x[2, ::3] = x[2].max()                                # ties past the pool
+        x[3, vocab // 2] = {0: 2e37, 1: 20000.0, 2: 2e37}[dtype]
+        x[4, 0], x[4, vocab - 1], x[4, vocab // 3] = np.nan, np.inf, -np.inf
+        x[5] = -np.abs(x[5]) - 3.0
+        bits = x if dtype == 2 else (x.astype(np.float16).view(np.uint16) if dtype == 1 else
+                                     torch.from_numpy(x).to(torch.bfloat16).view(torch.int16).numpy().view(np.uint16))
+        x32 = decode(bits, dtype)
+        top = np.argsort(-np.where(np.isfinite(x32), x32, -np.inf), axis=1, kind="stable")
+        fo = np.full(vocab, 0x7F7F7F7F, dtype=np.int32)
+        fo[top[:, 0]] = 10
+        fo[top[:, vocab // 2]] = 44                           # generated after some rows' keys
+        nxt = np.array([top[r, min(vocab - 1, r % 4)] for r in range(rows)], dtype=np.int64)
+        for temperature in (cfg["temperature"], 0.0):
+            args = (temperature, cfg["top_k"], cfg["top_p"], cfg["min_p"], cfg["seed"])
+            want_c, want_gap = orc.sampled_scores(bits, dtype, *args, nxt, first_key, 0.5, presence, fo)
+            c, gap = vi.sampled_scores(to_dev(bits, dtype, dev), torch.from_numpy(nxt), *args, first_key, 0.5, presence,
+                                       torch.from_numpy(fo).to(dev))
+            torch.cuda.synchronize()
+            c, gap = c.cpu().numpy(), gap.cpu().numpy()
+            for r in range(rows):
+                _, det = orc.sampled_packet(bits[r:r + 1], dtype, *args, presence, fo, first_key=first_key + r)
+                near = temperature > 0 and _near(det[0], cfg)
+                if c[r] != want_c[r]:
+                    assert near, (vocab, r, c[r], want_c[r])
+                elif np.isfinite(gap[r]) and np.isfinite(want_gap[r]):
+                    # perturbed values v/T + G subtracted in fp32: four roundings of up to |v/T| + 17
+                    bound = 2.0 ** -22 * (np.abs(x32[r][np.isfinite(x32[r])]).max() / 0.7 + abs(presence) + 17)
+                    assert abs(gap[r] - want_gap[r]) <= 1e-4 + bound or near, (vocab, r, gap[r], want_gap[r])
+                elif not (np.isnan(gap[r]) and np.isnan(want_gap[r])):
+                    boosted = x32[r:r + 1].copy()
+                    boosted[0, nxt[r]] = np.float32(boosted[0, nxt[r]] + np.float32(0.5))
+                    _, bd = orc.sampled_packet(boosted, 2, *args, presence, fo, first_key=first_key + r)
+                    assert gap[r] == want_gap[r] or near or _near(bd[0], cfg), (vocab, r, gap[r], want_gap[r])

@@ -101,3 +101,31 @@ def test_two_batch_slices(orc, dev, rng, k):
     x = rng.standard_normal((rows, vocab)).astype(np.float32) * 1.5
     x[np.arange(rows)[:, None], rng.integers(0, vocab, (rows, 6))] = rng.uniform(6, 10, (rows, 6))
     run(orc, dev, x.astype(np.float16).view(np.uint16), 1, k)
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("offset,vocab", [(1, 40_000), (3, 8191), (5, 100_003), (7, 63)])
+def test_rows_off_a_16_byte_boundary(orc, dev, rng, dtype, offset, vocab):
+    """Rows that start anywhere in a wider buffer (odd offsets and strides), for
+    the top-k, greedy and row-score scans: the same results as aligned rows."""
+    import voidinfer_amd as vi
+    rows = 6
+    x = rng.standard_normal((rows, offset + vocab + 2)).astype(np.float32)
+    x[:, :offset], x[:, offset + vocab:] = 9.0, 9.0          # outside the rows: never taken
+    x[2, offset + vocab // 2] = np.nan
+    x[3, offset + vocab - 1] = np.inf
+    bits = x if dtype == 2 else (x.astype(np.float16).view(np.uint16) if dtype == 1 else
+                                 (x.view(np.uint32) >> 16).astype(np.uint16))
+    view = to_dev(bits, dtype, dev)[:, offset:offset + vocab]
+    inner = np.ascontiguousarray(bits[:, offset:offset + vocab])
+    w_ids, w_vals, _, _ = orc.topk_rows(inner, dtype, 20)
+    ids, vals, _ = vi.topk_rows(view, 20, logprobs=True)
+    assert np.array_equal(ids.cpu().numpy(), w_ids)
+    fin = np.isfinite(w_vals)
+    assert np.array_equal(vals.cpu().numpy()[fin], w_vals[fin])
+    assert np.array_equal(vi.greedy_packet(view)["token"], orc.greedy_rows(inner, dtype)["token"])
+    nxt = np.arange(rows, dtype=np.int64)
+    g, gap = vi.row_scores(view, torch.from_numpy(nxt))
+    w_g, w_gap = orc.row_scores(inner, dtype, nxt)
+    assert np.array_equal(g.cpu().numpy(), w_g)
+    np.testing.assert_array_equal(gap.cpu().numpy(), w_gap)

@@ -251,3 +251,28 @@ def test_sampled_topk_mode_refuses_full_vocabulary_lanes(orc, dev):
     exempt = {l for l in keep if np.min(w[4][l]) < 1e-9} | set(refused)
     assert_same(g, w, exempt)
     assert len(exempt) <= len(refused) + 1
+
+
+@pytest.mark.parametrize("tdt", [0, 1, 2])
+@pytest.mark.parametrize("ddt", [0, 1, 2])
+@pytest.mark.parametrize("vocab", [4096, 10_007])
+def test_sampled_lists_every_dtype_pair(orc, dev, rng, tdt, ddt, vocab):
+    """The one-launch list path over every pair of logit types, on rows that
+    start on and off a 16-byte boundary."""
+    import voidinfer_amd as vi
+    from voidinfer_amd import workloads as W
+    lanes, drafts = 5, 4
+    enc = {0: "bf16", 1: "f16", 2: "f32"}
+    d = W.gaussian_zipf(lanes * drafts, vocab, 2.0, 11)
+    t = np.repeat(d.reshape(lanes, drafts, vocab)[:, list(range(drafts)) + [drafts - 1]], 1, axis=1).copy()
+    t += rng.standard_normal(t.shape).astype(np.float32) * 0.5
+    tb, db = W.encode(t.reshape(-1, vocab), enc[tdt]), W.encode(d, enc[ddt])
+    p = W.config4(lanes=lanes, drafts=drafts, vocab=256)[3]
+    p["top_k"] = [1, 20, 50, 64, 20]
+    p["temperature"][4] = 0.0
+    drafted = np.array([[rng.choice(np.argsort(-d[l * drafts + j])[:4]) for j in range(drafts)] for l in range(lanes)],
+                       dtype=np.int32)
+    g = vi.verify_rows(1, to_dev(tb, tdt, dev), torch.from_numpy(drafted).to(dev), lanes, drafts,
+                       draft=to_dev(db, ddt, dev), params=p)
+    w = orc.verify_rows(1, tb, tdt, db, ddt, lanes, drafts, drafted, p, ())
+    assert_same(g, w, {l for l in range(lanes) if np.min(w[4][l]) < 1e-9})

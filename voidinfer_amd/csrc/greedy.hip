@@ -57,7 +57,7 @@ __device__ __forceinline__ void greedy_write(const void* row, int r, int vocabul
     }
 }
 
-template <int DT, bool VEC, bool SCORE>
+template <int DT, bool SCORE>
 __global__ __launch_bounds__(kGreedyThreads) void greedy_kernel(
     const void* logits, int vocabulary, int64_t stride, int slice_len, uint64_t serial,
     vi_greedy_row* out, GreedyPartial* partials, uint32_t* arrivals, const int64_t* next, int64_t* greedy,
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(kGreedyThreads) void greedy_kernel(
     // within a vector free of non-finite values the first maximum is taken only
     // if it beats the running best strictly; a vector holding one goes element
     // by element.
-    scan_slice_vec<DT, VEC, kGreedyThreads>(
+    scan_slice_vec<DT, kGreedyThreads>(
         row, begin, end, [](const auto&, const auto&) {},
         [&](const uint4& dv, int id0, bool ok) {
             constexpr int P = Elem<DT>::kPerVec;
@@ -188,15 +188,14 @@ vi_status launch_greedy_kind(const void* logits, int dtype, int rows, int vocabu
         partials = c.take<GreedyPartial>(size_t(rows) * p.slices);
         if (!c.ok) return VI_ERR_WORKSPACE;
     }
-    const bool vec = (reinterpret_cast<uintptr_t>(logits) % 16 == 0) && ((stride * elem_size(dtype)) % 16 == 0);
     const dim3 grid(p.slices, rows), block(kGreedyThreads);
-#define VI_GREEDY_LAUNCH(DT, V)                                                                          \
-    hipLaunchKernelGGL((greedy_kernel<DT, V, SCORE>), grid, block, 0, stream, logits, vocabulary, stride, \
+#define VI_GREEDY_LAUNCH(DT)                                                                          \
+    hipLaunchKernelGGL((greedy_kernel<DT, SCORE>), grid, block, 0, stream, logits, vocabulary, stride, \
                        p.slice_len, serial, out, partials, arrivals, next, greedy, gap)
     switch (dtype) {
-        case VI_BF16: if (vec) VI_GREEDY_LAUNCH(VI_BF16, true); else VI_GREEDY_LAUNCH(VI_BF16, false); break;
-        case VI_F16: if (vec) VI_GREEDY_LAUNCH(VI_F16, true); else VI_GREEDY_LAUNCH(VI_F16, false); break;
-        default: if (vec) VI_GREEDY_LAUNCH(VI_F32, true); else VI_GREEDY_LAUNCH(VI_F32, false); break;
+        case VI_BF16: VI_GREEDY_LAUNCH(VI_BF16); break;
+        case VI_F16: VI_GREEDY_LAUNCH(VI_F16); break;
+        default: VI_GREEDY_LAUNCH(VI_F32); break;
     }
 #undef VI_GREEDY_LAUNCH
     return launch_status();

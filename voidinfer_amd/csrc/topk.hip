@@ -106,12 +106,9 @@ struct TopkArgs {
     uint32_t* lvalid;       // [rows]
     uint32_t* lflags;       // [rows]
     int skip_unlisted;      // rows of lanes without a top-k list are left to the full-vocabulary path
-    // kModeVerify with the decisions taken as the rows finish: decide == 1 over
-    // the draft rows (each position's decision, each lane's chain), decide == 2
-    // over the target rows (the bonus rows' draws); in the paired launch
-    // decide == 3 (target rows) and 4 (draft rows): each position's later row
-    // decides.  larr: the lanes' arrival counters, zero between calls
-    int decide;
+    // the decisions are taken as the rows finish, each position's by the later
+    // of its two rows.  dv.larr: the lanes' arrival counters, zero between calls
+    int target_side;        // target rows, else draft rows
     VerifyDecideArgs dv;
     int pair_rows;          // (the paired launch: rows of the target half)
 };
@@ -305,52 +302,57 @@ __device__ __forceinline__ int packet_support(const vi_device_sampling& cfg, int
     return support < 1 ? 1 : support;
 }
 
-// Coupled draw over the sorted candidates (sampled_select.cuh:79-116): the
-// selected index; value[0..support) receives the perturbed values l/T + G.
-__device__ __forceinline__ int packet_draw(const vi_device_sampling& cfg, int key, int cap, const float* cand_val,
-                           const int* cand_idx, float* value, float* prob, int* support_out) {
-    if (!(cfg.temperature > 0.0f)) {
-        value[0] = cand_val[0];
-        *support_out = 1;
-        return 0;
-    }
+// Coupled draw over the sorted candidates (sampled_select.cuh:79-116), by one
+// wave: lane j holds candidate j (value cv, id ci).  The weights and the
+// perturbed values l/T + G are taken on their own lanes; the one
+// order-dependent chain, the running fp32 sums of the weights, is added lane by
+// lane in candidate order, and the cuts and the draw (the first maximum: NaN
+// never replaces the incumbent) are the serial rule's, found by ballots.
+// Returns the selected index; value: the lane's perturbed value.
+__device__ __forceinline__ int packet_draw_wave(const vi_device_sampling& cfg, int key, int cap, float cv, int ci,
+                                                float& value, int& support) {
+    const int lane = lane_id();
+    support = 1;
+    value = cv;
+    if (!(cfg.temperature > 0.0f)) return 0;
+    const bool in = lane < cap;
     const float inv_temp = 1.0f / cfg.temperature;
-    const int support = packet_support(cfg, cap, cand_val, prob);
-    int best = 0;
-    for (int j = 0; j < support; ++j) {
-        value[j] = fmaf(cand_val[j], inv_temp, gumbel(cfg.seed, key, cand_idx[j]));
-        if (j > 0 && value[j] > value[best]) best = j;
+    const float m = readlane_f(cv, 0) * inv_temp;
+    const float prob = in ? expf(fmaf(cv, inv_temp, -m)) : 0.0f;
+    float run = 0.0f, cum = 0.0f;
+    for (int j = 0; j < cap; ++j) {
+        run += readlane_f(prob, j);
+        cum = lane == j ? run : cum;
     }
-    *support_out = support;
-    return best;
+    const float min_p_thresh = cfg.min_p > 0.0f ? cfg.min_p * readlane_f(prob, 0) : -1.0f;
+    const float top_p_target = cfg.top_p * run;
+    const uint64_t fm = ballot(in && min_p_thresh >= 0.0f && prob < min_p_thresh);
+    const uint64_t hm = ballot(in && cfg.top_p < 1.0f && cum >= top_p_target);
+    const int jf = fm ? __builtin_ctzll(fm) : cap, jh = hm ? __builtin_ctzll(hm) : cap;
+    support = jf <= jh ? jf : jh + 1;
+    if (support < 1) support = 1;
+    value = fmaf(cv, inv_temp, gumbel(cfg.seed, key, ci));
+    const uint32_t b = __builtin_bit_cast(uint32_t, value + 0.0f);   // (-0 and +0 compare equal)
+    const bool nan = (b & 0x7fffffffu) > 0x7f800000u;
+    uint32_t k = nan ? (lane == 0 ? 0xffffffffu : 0u) : ((b & 0x80000000u) ? ~b : (b | 0x80000000u));
+    if (lane >= support) k = 0u;
+    uint32_t top = k;
+    top = max(top, lanes_xor_dpp<1>(top));
+    top = max(top, lanes_xor_dpp<2>(top));
+    top = max(top, lanes_xor_dpp<4>(top));
+    top = max(top, lanes_xor_dpp<8>(top));
+    top = max(top, lanes_xor_dpp<16>(top));
+    top = max(top, lanes_xor_dpp<32>(top));
+    return __builtin_ctzll(ballot(k == top));
 }
 
-// VeriCache sampled gap (exl3_sampled_score_kernel, sampled_select.cuh:300-360):
-// how far, in logit units, next trails the selected token.  In the support:
-// T times the perturbed-value gap.  Outside it: infinite, unless raising next's
-// logit by `tolerance` re-ranks it into the support of the same sampler; then
-// the gap is taken against the best other support entry.  A next at or past
-// the vocabulary end is infinite.
-template <int DT>
-__device__ __forceinline__ float sampled_gap(const vi_device_sampling& cfg, int key, const void* row, int vocabulary,
-                             float tolerance, int64_t want, int selected, int support, const float* cand_val,
-                             const int* cand_idx, const float* value, float* prob, float* v2, int* i2) {
-    const int token = cand_idx[selected];
-    if (want < 0 || want == token) return 0.0f;
-    if (want >= vocabulary) return kInfF;
-    if (!(cfg.temperature > 0.0f)) {
-        float own = Elem<DT>::decode(static_cast<const typename Elem<DT>::Bits*>(row)[want]);
-        if (cfg.presence_penalty != 0.0f && cfg.first_occurrence && cfg.first_occurrence[want] < key)
-            own -= cfg.presence_penalty;
-        return fmaxf(0.0f, cand_val[selected] - own);
-    }
-    int cap = 20;
-    if (cfg.top_k > 0 && cfg.top_k < cap) cap = cfg.top_k;
-    int rank = -1;
-    for (int j = 0; j < cap; ++j)
-        if (cand_idx[j] == want) { rank = j; break; }
-    if (rank >= 0 && rank < support) return (value[selected] - value[rank]) * cfg.temperature;
-    if (rank < 0 || !(tolerance > 0.0f)) return kInfF;
+// VeriCache sampled gap (exl3_sampled_score_kernel, sampled_select.cuh:300-360)
+// of a candidate `rank` outside the support: infinite, unless raising its logit
+// by `tolerance` re-ranks it into the support of the same sampler; then the gap
+// is taken against the best other support entry.  One lane, its arrays in LDS.
+__device__ __forceinline__ float raised_gap(const vi_device_sampling& cfg, int key, float tolerance, int want,
+                                            int rank, int cap, const float* cand_val, const int* cand_idx,
+                                            float* prob, float* v2, int* i2) {
     const float boosted = cand_val[rank] + tolerance;
     int at = 0;
     for (int j = 0; j < cap; ++j) {
@@ -362,14 +364,14 @@ __device__ __forceinline__ float sampled_gap(const vi_device_sampling& cfg, int 
     int pos = at;
     while (pos > 0 && boosted > v2[pos - 1]) { v2[pos] = v2[pos - 1]; i2[pos] = i2[pos - 1]; --pos; }
     v2[pos] = boosted;
-    i2[pos] = int(want);
+    i2[pos] = want;
     const int s2 = packet_support(cfg, cap, v2, prob);
     if (pos >= s2) return kInfF;
     const float inv_temp = 1.0f / cfg.temperature;
     float best = -kInfF;
     for (int j = 0; j < s2; ++j)
         if (j != pos) best = fmaxf(best, fmaf(v2[j], inv_temp, gumbel(cfg.seed, key, i2[j])));
-    const float own = fmaf(cand_val[rank], inv_temp, gumbel(cfg.seed, key, int(want)));
+    const float own = fmaf(cand_val[rank], inv_temp, gumbel(cfg.seed, key, want));
     return fmaxf(0.0f, (best - own) * cfg.temperature);
 }
 
@@ -436,9 +438,12 @@ __device__ __forceinline__ void sample_finish(const vi_row_params& p, int cap, c
 
 // ------------------------------------------------------------------- the kernel
 // The work of one workgroup: slice `slice` of `slices` of row r.
-template <int DT, bool VEC, int MODE>
+template <int DT, int MODE>
 __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, const int slices, const int r) {
-    constexpr bool kD = MODE == kModeSample;   // DPP lane exchanges in the list merges
+    constexpr bool kD = MODE == kModeSample || MODE == kModePacket;   // DPP lane exchanges in the list merges
+    // modes whose candidates' values are looked up (penalties): the batched scan
+    // with the looked-up gate
+    constexpr bool kPen = MODE == kModeSample || MODE == kModePacket;
     const int lane = lane_id(), wave = threadIdx.x / kWave;
     const void* row = static_cast<const unsigned char*>(a.logits) + size_t(r) * size_t(a.stride) * sizeof(typename Elem<DT>::Bits);
     const int begin = slice * a.slice_len, end = min(a.vocabulary, begin + a.slice_len);
@@ -463,6 +468,7 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
             path[path_count++] = a.keys.input[r];
         }
         slack = a.cfg.presence_penalty < 0.0f ? -a.cfg.presence_penalty : 0.0f;
+        lookups = a.cfg.presence_penalty != 0.0f && (a.cfg.first_occurrence || path_count > 0);
     } else if constexpr (MODE == kModeVerify) {
         p = a.params[r / a.params_div];
         // a sampled lane whose top_k lies outside [1, 64] has no list here: its
@@ -509,17 +515,15 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
         if (lookups && a.hist_counts) {
             // the slice's first batch of logits requested before the counting
             // (its latency and the history's overlap)
-            if constexpr (VEC) {
-                constexpr int P = Elem<DT>::kPerVec;
-                const int nvec = (end - begin) / P;
-                const unsigned char* base = static_cast<const unsigned char*>(row) + size_t(begin) * (16 / P);
+            constexpr int P = Elem<DT>::kPerVec;
+            const int nvec = (end - begin) / P;
+            const unsigned char* base = static_cast<const unsigned char*>(row) + size_t(begin) * (16 / P);
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int v = u * kTopkThreads + int(threadIdx.x);
-                    pre[u] = v < nvec ? load16(base + size_t(v) * 16) : make_uint4(0, 0, 0, 0);
-                }
-                have_pre = nvec > 0;
+            for (int u = 0; u < 4; ++u) {
+                const int v = u * kTopkThreads + int(threadIdx.x);
+                pre[u] = v < nvec ? load16(base + size_t(v) * 16) : make_uint4(0, 0, 0, 0);
             }
+            have_pre = nvec > 0;
             // the slice's tokens' counts in the lane's history, in LDS; the
             // history checked as the hash builder checks it
             uint32_t* cnt = s_dyn;
@@ -580,6 +584,11 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     // bitmap says the token is absent)
     auto count_of = [&](int id) -> uint32_t {
         if (!lookups) return 0u;
+        if constexpr (MODE == kModePacket) {   // (generated before the key, or drafted on the row's path)
+            bool seen = a.cfg.first_occurrence && a.cfg.first_occurrence[id] < key;
+            for (int j = 0; j < path_count && !seen; ++j) seen = path[j] == id;
+            return seen ? 1u : 0u;
+        }
         if (hcnt) return hcnt[id - begin];
         if (pres) {
             const int o = id - begin;
@@ -865,11 +874,7 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
             if (ok && !finite) flags |= kSliceNonfinite;
             bool cand = ok && finite && better(x + slack, id, L.kv, L.ki);
             float v = x;
-            if (cand && a.cfg.presence_penalty != 0.0f) {
-                bool seen = a.cfg.first_occurrence && a.cfg.first_occurrence[id] < key;
-                for (int j = 0; j < path_count && !seen; ++j) seen = path[j] == id;
-                if (seen) v = x - a.cfg.presence_penalty;
-            }
+            if (cand && count_of(id)) v = x - a.cfg.presence_penalty;
             list_offer(L, K, cand, v, id);
         } else if constexpr (MODE == kModeVerify) {
             if (ok && !finite) flags |= kSliceNonfinite;
@@ -903,7 +908,7 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
             list_offer(L, K, cand, v, id);
         }
     };
-    // ---- sample mode, batches.  A row qualifies when its penalties only lower a
+    // ---- sample and packet modes, batches.  A sample row qualifies when its penalties only lower a
     // logit and cannot carry one with |x| below the overflow guard out of the
     // dtype's range (guard * repetition + frequency * history length + presence
     // under half the largest finite value): then, as in elem_fn, only elements
@@ -914,8 +919,16 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     // through elem_fn.  Other rows take elem_fn throughout, and a row whose
     // penalties fail the range check has every element looked up (a penalty
     // could then turn a finite logit that no gate would look at non-finite,
-    // which the row's finite count and flags must see).
+    // which the row's finite count and flags must see).  A packet row qualifies
+    // unless its presence penalty could carry a logit under the guard out of
+    // fp32's range (the penalized value is not stored in the logits' dtype); a
+    // negative penalty raises logits, by `slack` at most, so a raw value plus the
+    // slack is what has to reach the gate.  (Sampled scores of 16 x 248,320 fp16
+    // rows: 21.8 us per call; 55.2 with every element offered to the wave's list
+    // and the draw taken by one lane.)
     bool batched = false;
+    if constexpr (MODE == kModePacket)
+        batched = !lookups || double(overflow_guard<DT>()) + fabs(double(a.cfg.presence_penalty)) < 1.0e38;
     if constexpr (MODE == kModeSample) {
         if (!lookups) {
             batched = true;
@@ -933,6 +946,10 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     // counts given)
     auto penalized = [&](uint32_t bits, uint32_t c, float& v) -> bool {
         const float x = Elem<DT>::decode(bits);
+        if constexpr (MODE == kModePacket) {
+            v = c ? x - a.cfg.presence_penalty : x;
+            return true;
+        }
         v = p.temperature > 0.0f ? x * inv_t : x;
         if (c) {
             const uint32_t pb = penalize_bits<DT>(bits, c, p);
@@ -1037,6 +1054,7 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
             if (p.temperature > 0.0f) b = b || !isfinite(mx * inv_t) || !isfinite(mn * inv_t);
             bad |= okv[u] && b;
             vm[u] = okv[u] ? (p.temperature > 0.0f ? mx * inv_t : mx) : -kInfF;
+            if constexpr (MODE == kModePacket) vm[u] += slack;
         }
         if (ballot(bad) != 0) {
             // (one call per vector with a constant index, each a rolled loop over
@@ -1064,7 +1082,8 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
             for (int j = 0; j < P; ++j) {
                 const uint32_t bits = vec_bits<DT>(dvu, j);
                 const float x = Elem<DT>::decode(bits);
-                const bool want = ok && (p.temperature > 0.0f ? x * inv_t : x) >= gate;
+                const bool want =
+                    ok && (MODE == kModePacket ? x + slack : p.temperature > 0.0f ? x * inv_t : x) >= gate;
                 if (ballot(want) == 0) continue;
                 float v = -kInfF;
                 const bool c = want && penalized(bits, want ? count_of(id0 + j) : 0u, v) && v >= gate;
@@ -1111,7 +1130,7 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     };
     // (16-bit vector rows; bf16 rows in top-k mode keep the batch scan: their
     // held scan with the log-sum-exp does not fit 128 registers)
-    constexpr bool kHeldMode = VEC && (DT == VI_F16 || (DT == VI_BF16 && MODE == kModeVerify));
+    constexpr bool kHeldMode = DT == VI_F16 || (DT == VI_BF16 && MODE == kModeVerify);
     auto held_scan = [&](int nvec) {
       if constexpr (kHeldMode) {
         constexpr int P = Elem<DT>::kPerVec;
@@ -1367,38 +1386,18 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     };
     if constexpr (MODE == kModeTopk || MODE == kModeVerify) {
         if (held_fits()) held_then_tail();
-        else scan_slice_batches<DT, VEC, kTopkThreads>(row, begin, end, first_fn, batch_fn, elem_fn);
-    } else if constexpr (MODE == kModeSample) {
+        else scan_slice_batches<DT, kTopkThreads>(row, begin, end, first_fn, batch_fn, elem_fn);
+    } else {
         if (batched) {
             if (threadIdx.x == 0) s_np = 0;   // (ordered by the first batch's barrier)
-            scan_slice_batches_from<DT, VEC, kTopkThreads>(row, begin, end, pre, have_pre, first_sample, sample_batch,
+            scan_slice_batches_from<DT, kTopkThreads>(row, begin, end, pre, have_pre, first_sample, sample_batch,
                                                            elem_fn);
             sample_pool_finish();
         } else {
-            scan_slice<DT, VEC, kTopkThreads>(row, begin, end, elem_fn);
+            scan_slice<DT, kTopkThreads>(row, begin, end, elem_fn);
         }
-    } else {
-        scan_slice<DT, VEC, kTopkThreads>(row, begin, end, elem_fn);
     }
 
-    // Verification with decisions over the draft rows: the position's target
-    // list (entries, finite count, flags), loaded by wave 0 as early as the row's
-    // last workgroup is known
-    float tl_v = -kInfF;
-    int tl_i = kInvalidId;
-    uint32_t tl_valid = 0, tl_flags = 0;
-    bool tl_have = false;
-    auto tl_fetch = [&]() {
-        if constexpr (MODE == kModeVerify) {
-            const int l = r / a.dv.drafts, j = r - l * a.dv.drafts;
-            const size_t tr = size_t(l) * a.dv.target_rows + j;
-            tl_v = a.dv.tlval[tr * kMaxK + lane];
-            tl_i = a.dv.tlidx[tr * kMaxK + lane];
-            tl_valid = a.dv.tlvalid[tr];
-            tl_flags = a.dv.tlflags[tr];
-            tl_have = true;
-        }
-    };
     // ---- merge the wave lists in LDS
     __shared__ float s_val[kTopkWaves][kMaxK];
     __shared__ int s_idx[kTopkWaves][kMaxK];
@@ -1445,9 +1444,6 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
         __syncthreads();
         if (!s_last) return;
         handoff_acquire();
-        if constexpr (MODE == kModeVerify) {   // (the target row's list, loaded under the merge below)
-            if (a.decide == 1 && wave == 0) tl_fetch();
-        }
         // the headers (wave 0, lane sl holds slice sl's; slices <= 64), loaded
         // now so that their latency overlaps the list loads and merges
         // (loads unconditional, at clamped in-bounds addresses, and selected
@@ -1476,7 +1472,7 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
                     s_pi[t] = get_agent(&a.pidx[src]);
                 }
                 __syncthreads();
-            } else if (MODE == kModeSample && n <= kMergeHeld * kTopkThreads) {
+            } else if (kPen && n <= kMergeHeld * kTopkThreads) {
                 // this thread's entries (loads at clamped addresses, selected after)
                 float ev[kMergeHeld];
                 int ei[kMergeHeld];
@@ -1616,32 +1612,54 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
         }
         if (lane == 0 && (f & kSliceNonfinite) && a.nonfinite_flag) atomicOr(a.nonfinite_flag, 1u);
     } else if constexpr (MODE == kModePacket) {
-        __shared__ float s_tail[3][20];
+        __shared__ float s_tail[2][20];
         __shared__ int s_tail_i[20];
-        if (lane == 0) {
-            int support = 1;
-            const int sel = packet_draw(a.cfg, key, K, s_val[0], s_idx[0], s_tail[0], s_tail[1], &support);
-            if (a.score) {
-                a.chosen[r] = s_idx[0][sel];
-                a.score_gap[r] = sampled_gap<DT>(a.cfg, key, row, a.vocabulary, a.tolerance, a.next[r], sel, support,
-                                                 s_val[0], s_idx[0], s_tail[0], s_tail[1], s_tail[2], s_tail_i);
-            } else {
-                a.out_rows[r].serial = a.serial;
-                a.out_rows[r].token = s_idx[0][sel];
-                a.out_rows[r].nonfinite = (f & kSliceNonfinite) ? 1u : 0u;
+        float value;
+        int support;
+        const int sel = packet_draw_wave(a.cfg, key, K, L.v, L.i, value, support);
+        const int token = readlane_i(L.i, sel);
+        if (a.score) {
+            // how far, in logit units, next trails the selected token: in the
+            // support T times the perturbed-value gap (a next at or past the
+            // vocabulary end is infinite)
+            const int64_t want = a.next[r];
+            float gap = 0.0f;
+            if (want >= a.vocabulary && want != token) {
+                gap = kInfF;
+            } else if (want >= 0 && want != token && !(a.cfg.temperature > 0.0f)) {
+                float own = Elem<DT>::decode(load_bits<DT>(row, want));
+                if (a.cfg.presence_penalty != 0.0f && a.cfg.first_occurrence && a.cfg.first_occurrence[want] < key)
+                    own -= a.cfg.presence_penalty;
+                gap = fmaxf(0.0f, readlane_f(L.v, sel) - own);
+            } else if (want >= 0 && want != token) {
+                int cap = 20;
+                if (a.cfg.top_k > 0 && a.cfg.top_k < cap) cap = a.cfg.top_k;
+                const uint64_t wm = ballot(lane < cap && L.i == int(want));
+                const int rank = wm ? __builtin_ctzll(wm) : -1;
+                if (rank >= 0 && rank < support)
+                    gap = (readlane_f(value, sel) - readlane_f(value, rank)) * a.cfg.temperature;
+                else if (rank < 0 || !(a.tolerance > 0.0f))
+                    gap = kInfF;
+                else if (lane == 0)
+                    gap = raised_gap(a.cfg, key, a.tolerance, int(want), rank, cap, s_val[0], s_idx[0], s_tail[0],
+                                     s_tail[1], s_tail_i);
             }
+            if (lane == 0) {
+                a.chosen[r] = token;
+                a.score_gap[r] = gap;
+            }
+        } else if (lane == 0) {
+            a.out_rows[r].serial = a.serial;
+            a.out_rows[r].token = token;
+            a.out_rows[r].nonfinite = (f & kSliceNonfinite) ? 1u : 0u;
         }
     } else if constexpr (MODE == kModeVerify) {
         const bool refused = verify_list_refused(p);
         const uint32_t rvalid = refused ? 0u : c;
         const uint32_t rflags = ((f & kSliceNonfinite) ? VI_FLAG_NONFINITE : 0u) | (refused ? VI_FLAG_ERROR : 0u);
-        if (a.decide >= 3) {   // (read by the position's other row, in this launch)
-            if (lane < K) { put_agent(&a.lval[size_t(r) * kMaxK + lane], L.v); put_agent(&a.lidx[size_t(r) * kMaxK + lane], L.i); }
-            if (lane == 0) { put_agent(&a.lvalid[r], rvalid); put_agent(&a.lflags[r], rflags); }
-        } else {
-            if (lane < K) { a.lval[size_t(r) * kMaxK + lane] = L.v; a.lidx[size_t(r) * kMaxK + lane] = L.i; }
-            if (lane == 0) { a.lvalid[r] = rvalid; a.lflags[r] = rflags; }
-        }
+        // (read by the position's other row, in this launch)
+        if (lane < K) { put_agent(&a.lval[size_t(r) * kMaxK + lane], L.v); put_agent(&a.lidx[size_t(r) * kMaxK + lane], L.i); }
+        if (lane == 0) { put_agent(&a.lvalid[r], rvalid); put_agent(&a.lflags[r], rflags); }
         // the lane's decided positions counted; its last walks the chain
         auto lane_arrive = [&](int l, uint32_t total) {
             uint32_t old = 0;
@@ -1658,11 +1676,11 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
                             a.dv.accepted, a.dv.committed, a.dv.committed_count, a.dv.lane_flags);
             if (lane == 0) put_agent(&a.dv.larr[l], 0u);
         };
-        if (a.decide >= 3) {
-            // paired launch: target row (l, j) or draft row (l, j); the later of
+        {
+            // target row (l, j) or draft row (l, j); the later of
             // the two takes position j's decision with the other's list read back
             // (a bonus row decides alone)
-            const bool tside = a.decide == 3;
+            const bool tside = a.target_side != 0;
             const int per = tside ? a.dv.target_rows : a.dv.drafts;
             const int l = r / per, j = r - l * per;
             const bool bonus = tside && j == a.dv.drafts;
@@ -1702,29 +1720,6 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
                 }
                 lane_arrive(l, uint32_t(a.dv.drafts + (a.dv.target_rows == a.dv.drafts + 1 ? 1 : 0)));
             }
-        } else if (a.decide == 2) {
-            // target row r: position j of lane l; a bonus row draws the lane's
-            // bonus token from its own list (in LDS)
-            const int l = r / a.dv.target_rows, j = r - l * a.dv.target_rows;
-            if (j == a.dv.drafts)
-                position_decision(p, j, l, a.dv.drafts, a.dv.target_rows, s_val[0], s_idx[0], rvalid, rflags,
-                                  nullptr, nullptr, 0u, 0u, a.dv.drafted, a.vocabulary, 0, a.dv.dec);
-        } else if (a.decide == 1) {
-            // draft row r is position j of lane l: its decision, from the target
-            // row's list (in LDS) and this row's (in LDS; entries past K are never
-            // read); the lane's last position to finish walks the chain (the
-            // bonus draw is the target launch's; agent-scope hand-off of the
-            // decisions, the lane's counter reset for the next call)
-            const int l = r / a.dv.drafts, j = r - l * a.dv.drafts;
-            if (!tl_have) tl_fetch();
-            __shared__ float s_tv[kMaxK];
-            __shared__ int s_ti[kMaxK];
-            s_tv[lane] = tl_v;
-            s_ti[lane] = tl_i;
-            wave_sync();
-            position_decision(p, j, l, a.dv.drafts, a.dv.target_rows, s_tv, s_ti, tl_valid, tl_flags, s_val[0],
-                              s_idx[0], rvalid, rflags, a.dv.drafted, a.vocabulary, 0, a.dv.dec);
-            lane_arrive(l, uint32_t(a.dv.drafts));
         }
     } else {
         // the candidates' fp64 weights, one per lane (into LDS for the running sums)
@@ -1762,18 +1757,19 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     }
 }
 
-template <int DT, bool VEC, int MODE>
+template <int DT, int MODE>
 __global__ __launch_bounds__(kTopkThreads, 4) void topk_kernel(TopkArgs a) {
-    topk_body<DT, VEC, MODE>(a, int(blockIdx.x), int(gridDim.x), int(blockIdx.y));
+    topk_body<DT, MODE>(a, int(blockIdx.x), int(gridDim.x), int(blockIdx.y));
 }
 
 // Verification's target rows (first t.pair_rows rows of the grid) and draft
-// rows in one launch.
+// rows in one launch, `slices` workgroups per row (one grid dimension: the two
+// row sets together may pass the limit of the second).
 template <int DTT, int DTD>
-__global__ __launch_bounds__(kTopkThreads, 4) void verify_pair_kernel(TopkArgs t, TopkArgs d) {
-    const int y = int(blockIdx.y);
-    if (y < t.pair_rows) topk_body<DTT, true, kModeVerify>(t, int(blockIdx.x), int(gridDim.x), y);
-    else topk_body<DTD, true, kModeVerify>(d, int(blockIdx.x), int(gridDim.x), y - t.pair_rows);
+__global__ __launch_bounds__(kTopkThreads, 4) void verify_pair_kernel(TopkArgs t, TopkArgs d, int slices) {
+    const int y = int(blockIdx.x) / slices, slice = int(blockIdx.x) - y * slices;
+    if (y < t.pair_rows) topk_body<DTT, kModeVerify>(t, slice, slices, y);
+    else topk_body<DTD, kModeVerify>(d, slice, slices, y - t.pair_rows);
 }
 
 // History hash builder: one workgroup per row.  Each history token is
@@ -1834,22 +1830,18 @@ __global__ __launch_bounds__(kHashThreads) void history_hash_kernel(
 }
 
 template <int MODE>
-vi_status launch_mode(const TopkArgs& args, int dtype, bool vec, int rows, int slices, hipStream_t stream) {
+vi_status launch_mode(const TopkArgs& args, int dtype, int rows, int slices, hipStream_t stream) {
     if (slices < 1 || slices > 64) return VI_ERR_INVALID;   // the merge reads one slice header per lane
     const dim3 grid(slices, rows), block(kTopkThreads);
     const size_t dyn = size_t(args.pres_words) * 4;
-#define VI_TOPK_LAUNCH(DT, V) hipLaunchKernelGGL((topk_kernel<DT, V, MODE>), grid, block, dyn, stream, args)
+#define VI_TOPK_LAUNCH(DT) hipLaunchKernelGGL((topk_kernel<DT, MODE>), grid, block, dyn, stream, args)
     switch (dtype) {
-        case VI_BF16: if (vec) VI_TOPK_LAUNCH(VI_BF16, true); else VI_TOPK_LAUNCH(VI_BF16, false); break;
-        case VI_F16: if (vec) VI_TOPK_LAUNCH(VI_F16, true); else VI_TOPK_LAUNCH(VI_F16, false); break;
-        default: if (vec) VI_TOPK_LAUNCH(VI_F32, true); else VI_TOPK_LAUNCH(VI_F32, false); break;
+        case VI_BF16: VI_TOPK_LAUNCH(VI_BF16); break;
+        case VI_F16: VI_TOPK_LAUNCH(VI_F16); break;
+        default: VI_TOPK_LAUNCH(VI_F32); break;
     }
 #undef VI_TOPK_LAUNCH
     return launch_status();
-}
-
-bool aligned16(const void* p, int64_t stride, int dtype) {
-    return (reinterpret_cast<uintptr_t>(p) % 16 == 0) && ((stride * elem_size(dtype)) % 16 == 0);
 }
 
 struct Partials {
@@ -1903,7 +1895,7 @@ vi_status launch_topk_rows(const void* logits, int dtype, int rows, int vocabula
     a.logits = logits; a.vocabulary = vocabulary; a.stride = stride; a.slice_len = plan.slice_len;
     a.pval = part.pval; a.pidx = part.pidx; a.phdr = part.phdr; a.arrivals = part.arrivals;
     a.k = k; a.ids = ids; a.values = values; a.logprobs = logprobs; a.nonfinite_flag = nonfinite_flag;
-    return launch_mode<kModeTopk>(a, dtype, aligned16(logits, stride, dtype), rows, plan.slices, stream);
+    return launch_mode<kModeTopk>(a, dtype, rows, plan.slices, stream);
 }
 
 vi_status launch_packet(const void* scores, int dtype, int rows, int vocabulary, int64_t stride,
@@ -1917,7 +1909,7 @@ vi_status launch_packet(const void* scores, int dtype, int rows, int vocabulary,
     a.logits = scores; a.vocabulary = vocabulary; a.stride = stride; a.slice_len = plan.slice_len;
     a.pval = part.pval; a.pidx = part.pidx; a.phdr = part.phdr; a.arrivals = part.arrivals;
     a.cfg = cfg; a.keys = keys; a.serial = serial; a.out_rows = out;
-    return launch_mode<kModePacket>(a, dtype, aligned16(scores, stride, dtype), rows, plan.slices, stream);
+    return launch_mode<kModePacket>(a, dtype, rows, plan.slices, stream);
 }
 
 vi_status launch_sampled_scores(const void* scores, int dtype, int rows, int vocabulary, int64_t stride,
@@ -1933,36 +1925,7 @@ vi_status launch_sampled_scores(const void* scores, int dtype, int rows, int voc
     a.pval = part.pval; a.pidx = part.pidx; a.phdr = part.phdr; a.arrivals = part.arrivals;
     a.cfg = cfg; a.keys.first = first_key; a.score = 1; a.tolerance = tolerance;
     a.next = next; a.chosen = chosen; a.score_gap = gap;
-    return launch_mode<kModePacket>(a, dtype, aligned16(scores, stride, dtype), rows, plan.slices, stream);
-}
-
-vi_status launch_verify_lists(const void* logits, int dtype, int rows, int layout_rows, int layout_slices,
-                              int vocabulary, int64_t stride, const vi_row_params* params, int params_div,
-                              float* lval, int* lidx, uint32_t* lvalid, uint32_t* lflags, int skip_unlisted,
-                              void* ws, size_t ws_bytes, hipStream_t stream, const VerifyDecideArgs* decide,
-                              int decide_mode) {
-    // Partials carved for (layout_rows, layout_slices) so that launches over
-    // different row counts share one counter layout in one workspace.
-    const TopkPlan plan = topk_plan(rows, vocabulary);
-    if (rows > layout_rows || plan.slices > layout_slices) return VI_ERR_WORKSPACE;
-    Carver c(ws, ws_bytes);
-    const Partials part = carve_partials(c, layout_rows, layout_slices);
-    if (!c.ok) return VI_ERR_WORKSPACE;
-    TopkArgs a{};
-    a.logits = logits; a.vocabulary = vocabulary; a.stride = stride; a.slice_len = plan.slice_len;
-    a.pval = part.pval; a.pidx = part.pidx; a.phdr = part.phdr; a.arrivals = part.arrivals;
-    a.params = params; a.params_div = params_div;
-    a.lval = lval; a.lidx = lidx; a.lvalid = lvalid; a.lflags = lflags; a.skip_unlisted = skip_unlisted;
-    if (decide) { a.decide = decide_mode; a.dv = *decide; }
-    return launch_mode<kModeVerify>(a, dtype, aligned16(logits, stride, dtype), rows, plan.slices, stream);
-}
-
-bool verify_pair_supported(const void* target, int target_dtype, int64_t target_stride, const void* draft,
-                           int draft_dtype, int64_t draft_stride) {
-    auto ok = [](const void* p, int dt, int64_t stride) {
-        return (dt == VI_BF16 || dt == VI_F16) && aligned16(p, stride, dt);
-    };
-    return ok(target, target_dtype, target_stride) && ok(draft, draft_dtype, draft_stride);
+    return launch_mode<kModePacket>(a, dtype, rows, plan.slices, stream);
 }
 
 vi_status launch_verify_pair(const void* target, int target_dtype, int64_t target_stride, const void* draft,
@@ -1971,8 +1934,6 @@ vi_status launch_verify_pair(const void* target, int target_dtype, int64_t targe
                              uint32_t* tvalid, uint32_t* tflags, float* dval, int* didx, uint32_t* dvalid,
                              uint32_t* dflags, const VerifyDecideArgs& decide, void* ws, size_t ws_bytes,
                              hipStream_t stream, int skip_unlisted) {
-    if (!verify_pair_supported(target, target_dtype, target_stride, draft, draft_dtype, draft_stride))
-        return VI_ERR_UNSUPPORTED;
     const int trows = lanes * decide.target_rows, drows = lanes * decide.drafts;
     // one slicing for both halves, about 1,024 workgroups for the two row sets
     // together (one round at four per CU; a slice of up to two held batches)
@@ -1989,7 +1950,7 @@ vi_status launch_verify_pair(const void* target, int target_dtype, int64_t targe
     t.pval = part.pval; t.pidx = part.pidx; t.phdr = part.phdr; t.arrivals = part.arrivals;
     t.params = params; t.params_div = decide.target_rows;
     t.lval = tval; t.lidx = tidx; t.lvalid = tvalid; t.lflags = tflags;
-    t.decide = 3; t.dv = decide; t.pair_rows = trows; t.skip_unlisted = skip_unlisted;
+    t.target_side = 1; t.dv = decide; t.pair_rows = trows; t.skip_unlisted = skip_unlisted;
     TopkArgs d = t;   // (the draft half: its rows' partials after the target half's)
     const size_t off = size_t(trows) * plan.slices;
     d.logits = draft; d.stride = draft_stride;
@@ -1997,14 +1958,21 @@ vi_status launch_verify_pair(const void* target, int target_dtype, int64_t targe
     d.arrivals = part.arrivals + trows;
     d.params_div = decide.drafts;
     d.lval = dval; d.lidx = didx; d.lvalid = dvalid; d.lflags = dflags;
-    d.decide = 4;
-    const dim3 grid(plan.slices, trows + drows), block(kTopkThreads);
-#define VI_PAIR(A, B) hipLaunchKernelGGL((verify_pair_kernel<A, B>), grid, block, 0, stream, t, d)
-    if (target_dtype == VI_BF16) {
-        if (draft_dtype == VI_BF16) VI_PAIR(VI_BF16, VI_BF16); else VI_PAIR(VI_BF16, VI_F16);
-    } else {
-        if (draft_dtype == VI_BF16) VI_PAIR(VI_F16, VI_BF16); else VI_PAIR(VI_F16, VI_F16);
+    d.target_side = 0;
+    const dim3 grid(unsigned(plan.slices) * unsigned(trows + drows)), block(kTopkThreads);
+#define VI_PAIR(A, B) hipLaunchKernelGGL((verify_pair_kernel<A, B>), grid, block, 0, stream, t, d, plan.slices)
+#define VI_PAIR_D(A)                              \
+    switch (draft_dtype) {                        \
+        case VI_BF16: VI_PAIR(A, VI_BF16); break; \
+        case VI_F16: VI_PAIR(A, VI_F16); break;   \
+        default: VI_PAIR(A, VI_F32); break;       \
     }
+    switch (target_dtype) {
+        case VI_BF16: VI_PAIR_D(VI_BF16); break;
+        case VI_F16: VI_PAIR_D(VI_F16); break;
+        default: VI_PAIR_D(VI_F32); break;
+    }
+#undef VI_PAIR_D
 #undef VI_PAIR
     return launch_status();
 }
@@ -2092,7 +2060,7 @@ vi_status launch_sample(const SampleArgs& s, void* ws, size_t ws_bytes, hipStrea
         a.stats = s.stats;
         // fp32 logits / unaligned rows: full-route rows fail loudly in the top-k launch
         a.full_rows_unsupported = (full_ok && (s.route_mask & VI_ROUTE_FULL)) ? 0 : (full_ok ? 0 : 1);
-        st = launch_mode<kModeSample>(a, s.dtype, aligned16(s.logits, s.stride, s.dtype), s.rows, plan.slices,
+        st = launch_mode<kModeSample>(a, s.dtype, s.rows, plan.slices,
                                       topk_stream);
         if (st != VI_OK && !side) return st;
     }

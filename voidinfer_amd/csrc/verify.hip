@@ -61,40 +61,6 @@ __global__ void verify_greedy_kernel(const vi_greedy_row* rows, int lanes, int d
     if (lane_flags) lane_flags[l] = flags;
 }
 
-// Every position of every lane at once; with `arrivals` (list lanes only) the
-// last position of a lane to finish runs its chain (agent-scope hand-off of the
-// decisions, the lane's counter reset for the next call), else
-// verify_chain_kernel does after the full-vocabulary kernels.
-__global__ __launch_bounds__(kFinalizeThreads) void verify_position_kernel(
-    const float* tval, const int* tidx, const uint32_t* tvalid, const uint32_t* tflags, const float* dval,
-    const int* didx, const uint32_t* dvalid, const uint32_t* dflags, int drafts, int target_rows,
-    const int32_t* drafted, const vi_row_params* params, int vocabulary, int full_ok, PosDecision* dec,
-    uint32_t* arrivals, const int64_t* terminal, int n_terminal, int32_t* accepted, int32_t* committed,
-    int32_t* committed_count, uint32_t* lane_flags) {
-    const int j = blockIdx.x, l = blockIdx.y;
-    // (position `drafts` is the bonus row's, which has no draft row, and exists
-    // only when target_rows == drafts + 1)
-    const bool has_t = j < target_rows, has_d = j < drafts;
-    const size_t tr = has_t ? size_t(l) * target_rows + j : 0, dr = has_d ? size_t(l) * drafts + j : 0;
-    position_decision(params[l], j, l, drafts, target_rows, tval + tr * kMaxK, tidx + tr * kMaxK,
-                      has_t ? tvalid[tr] : 0u, has_t ? tflags[tr] : 0u, dval + dr * kMaxK, didx + dr * kMaxK,
-                      has_d ? dvalid[dr] : 0u, has_d ? dflags[dr] : 0u, drafted, vocabulary, full_ok, dec);
-    if (!arrivals) return;
-    uint32_t old = 0;
-    if (threadIdx.x == 0) {
-        handoff_stores_done();
-        old = __hip_atomic_fetch_add(&arrivals[l], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (__builtin_amdgcn_readfirstlane(old) != uint32_t(drafts)) return;   // (drafts + 1 positions per lane)
-    handoff_acquire();
-    const PosDecision* D = dec + size_t(l) * (drafts + 1);
-    lane_chain_wave(l, [&](int q) {
-        return PosDecision{get_agent(&D[q].token), get_agent(&D[q].flags), get_agent(&D[q].accept), 0};
-    }, drafts, target_rows, drafted, params, terminal, n_terminal, full_ok, accepted, committed, committed_count,
-                    lane_flags);
-    if (threadIdx.x == 0) put_agent(&arrivals[l], 0u);
-}
-
 // The accept chains after the full-vocabulary kernels (one thread per lane).
 __global__ void verify_chain_kernel(const PosDecision* dec, int lanes, int drafts, int target_rows,
                                     const int32_t* drafted, const vi_row_params* params, const int64_t* terminal,
@@ -639,11 +605,6 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
     const int full_ok = (a.mode == VI_VERIFY_SAMPLED &&
                          full_path_ok(a.target, a.target_dtype, a.vocabulary, a.target_stride) &&
                          full_path_ok(a.draft, a.draft_dtype, a.vocabulary, a.draft_stride)) ? 1 : 0;
-    // every lane listed: the target rows' scan draws the bonus tokens as its
-    // bonus rows finish, the draft rows' scan takes each position's decision as
-    // its row finishes, and each lane's last position walks the chain (two
-    // launches in all)
-    const bool fused = !full_ok;
     VerifyDecideArgs dv{};
     dv.drafts = a.drafts; dv.target_rows = a.target_rows;
     dv.tlval = tval; dv.tlidx = tidx; dv.tlvalid = tvalid; dv.tlflags = tflags;
@@ -652,101 +613,77 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
     dv.terminal = a.terminal; dv.n_terminal = a.n_terminal;
     dv.accepted = a.accepted; dv.committed = a.committed; dv.committed_count = a.committed_count;
     dv.lane_flags = a.lane_flags;
-    const bool paired = verify_pair_supported(a.target, a.target_dtype, a.target_stride, a.draft, a.draft_dtype,
-                                              a.draft_stride);
-    if (paired) {
-        // both row sets in one launch: each listed position decided by its later
-        // row, each listed lane's chain walked by its last position (the lanes
-        // without a list, when the full path runs, are left to it)
-        st = launch_verify_pair(a.target, a.target_dtype, a.target_stride, a.draft, a.draft_dtype, a.draft_stride,
-                                a.lanes, a.vocabulary, a.params, v.lrows, v.lslices, tval, tidx, tvalid, tflags, dval,
-                                didx, dvalid, dflags, dv, lws, lbytes, stream, full_ok);
-        if (st != VI_OK || !full_ok) return st;
-    } else {
-    st = launch_verify_lists(a.target, a.target_dtype, trows, v.lrows, v.lslices, a.vocabulary, a.target_stride,
-                             a.params, a.target_rows, tval, tidx, tvalid, tflags, full_ok, lws, lbytes, stream,
-                             fused ? &dv : nullptr, 2);
+    // both row sets in one launch: each listed position decided by its later
+    // row, each listed lane's chain walked by its last position (the lanes
+    // without a list, when the full path runs, are left to it)
+    st = launch_verify_pair(a.target, a.target_dtype, a.target_stride, a.draft, a.draft_dtype, a.draft_stride, a.lanes,
+                            a.vocabulary, a.params, v.lrows, v.lslices, tval, tidx, tvalid, tflags, dval, didx, dvalid,
+                            dflags, dv, lws, lbytes, stream, full_ok);
+    if (st != VI_OK || !full_ok) return st;
+    const size_t tn = size_t(trows), dn = size_t(drows);
+    vi_row_params* tpar = c.take<vi_row_params>(tn);
+    vi_row_params* dpar = c.take<vi_row_params>(dn);
+    FullBound* tb = c.take<FullBound>(tn);
+    FullBound* db = c.take<FullBound>(dn);
+    uint32_t* tbase = c.take<uint32_t>(tn * kFullBaseSlots);
+    uint32_t* dbase = c.take<uint32_t>(dn * kFullBaseSlots);
+    vi_sample_stats* tst = c.take<vi_sample_stats>(tn);
+    vi_sample_stats* dst = c.take<vi_sample_stats>(dn);
+    int32_t* ttok = c.take<int32_t>(tn);
+    int32_t* dtok = c.take<int32_t>(dn);
+    const int ranges = full_ranges(a.vocabulary);
+    double* rsum = c.take<double>(size_t(a.lanes) * ranges * 2);
+    int* rlast = c.take<int>(size_t(a.lanes) * ranges * 2);
+    const size_t fbytes = full_sampler_bytes(v.trows, a.vocabulary);
+    const size_t dbytes = full_sampler_bytes(a.lanes * a.drafts, a.vocabulary);
+    unsigned char* fws = c.take<unsigned char>(fbytes);
+    unsigned char* dws = c.take<unsigned char>(dbytes);
+    if (!c.ok) return VI_ERR_WORKSPACE;
+    hipLaunchKernelGGL(verify_row_params_kernel, dim3((trows + drows + 255) / 256), dim3(256), 0, stream,
+                       a.params, a.lanes, a.target_rows, tpar, a.drafts, dpar);
+    // the rows' filtered distributions (and the target rows' draws) from the
+    // full-vocabulary sampler, each row set in its own workspace: the draft
+    // rows on the side stream beside the target rows on the caller's, joined
+    // back before the accept launch
+    auto sample = [&](const void* logits, int dtype, int rows, int64_t stride, const vi_row_params* par,
+                      int32_t* tok, vi_sample_stats* stats, const FullOut* out, unsigned char* w, size_t wb,
+                      hipStream_t on) {
+        SampleArgs s{};
+        s.logits = logits; s.dtype = dtype; s.rows = rows; s.vocabulary = a.vocabulary; s.stride = stride;
+        s.params = par; s.tokens = tok; s.stats = stats; s.route_mask = VI_ROUTE_FULL; s.full_out = out;
+        return dtype == VI_F32 ? launch_wide(s, w, wb, nullptr, 0, 0, nullptr, on) : launch_full(s, w, wb, on);
+    };
+    const FullOut tout{tb, tbase}, dout{db, dbase};
+    SideStream* side = drows > 0 ? side_stream() : nullptr;
+    if (side && (hipEventRecord(side->fork, stream) != hipSuccess ||
+                 hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess)) {
+        (void)hipGetLastError();
+        side = nullptr;
+    }
+    st = sample(a.draft, a.draft_dtype, drows, a.draft_stride, dpar, dtok, dst, &dout, dws, dbytes,
+                side ? side->stream : stream);
+    if (st == VI_OK)
+        st = sample(a.target, a.target_dtype, trows, a.target_stride, tpar, ttok, tst, &tout, fws, fbytes, stream);
+    // joined also when a launch failed: the side work uses the caller's workspace
+    if (side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
+                 hipStreamWaitEvent(stream, side->join, 0) != hipSuccess))
+        return VI_ERR_LAUNCH;
     if (st != VI_OK) return st;
-    if (fused)
-        return launch_verify_lists(a.draft, a.draft_dtype, drows, v.lrows, v.lslices, a.vocabulary, a.draft_stride,
-                                   a.params, a.drafts, dval, didx, dvalid, dflags, 0, lws, lbytes, stream, &dv, 1);
-    st = launch_verify_lists(a.draft, a.draft_dtype, drows, v.lrows, v.lslices, a.vocabulary, a.draft_stride,
-                             a.params, a.drafts, dval, didx, dvalid, dflags, full_ok, lws, lbytes, stream);
-    if (st != VI_OK) return st;
-    hipLaunchKernelGGL(verify_position_kernel, dim3(a.drafts + 1, a.lanes), dim3(kFinalizeThreads), 0, stream, tval,
-                       tidx, tvalid, tflags, dval, didx, dvalid, dflags, a.drafts, a.target_rows, a.drafted, a.params,
-                       a.vocabulary, full_ok, dec, full_ok ? nullptr : larr, a.terminal, a.n_terminal, a.accepted,
-                       a.committed, a.committed_count, a.lane_flags);
+    FullVerifyArgs f{};
+    f.t = FullRows{a.target, a.target_dtype, a.target_stride, tb, tbase, tst,
+                   a.target_dtype == VI_F32 ? kFullSlice32 : kFullSlice16};
+    f.d = FullRows{a.draft, a.draft_dtype, a.draft_stride, db, dbase, dst,
+                   a.draft_dtype == VI_F32 ? kFullSlice32 : kFullSlice16};
+    f.ttok = ttok; f.lanes = a.lanes; f.drafts = a.drafts; f.target_rows = a.target_rows;
+    f.vocabulary = a.vocabulary; f.drafted = a.drafted; f.params = a.params; f.terminal = a.terminal;
+    f.n_terminal = a.n_terminal; f.dec = dec; f.rsum = rsum; f.rlast = rlast; f.ranges = ranges;
+    switch (a.target_dtype) {
+        case VI_BF16: launch_full_verify_d<VI_BF16>(f, stream); break;
+        case VI_F16: launch_full_verify_d<VI_F16>(f, stream); break;
+        default: launch_full_verify_d<VI_F32>(f, stream); break;
+    }
     st = launch_status();
     if (st != VI_OK) return st;
-    }
-    if (full_ok) {
-        const size_t tn = size_t(trows), dn = size_t(drows);
-        vi_row_params* tpar = c.take<vi_row_params>(tn);
-        vi_row_params* dpar = c.take<vi_row_params>(dn);
-        FullBound* tb = c.take<FullBound>(tn);
-        FullBound* db = c.take<FullBound>(dn);
-        uint32_t* tbase = c.take<uint32_t>(tn * kFullBaseSlots);
-        uint32_t* dbase = c.take<uint32_t>(dn * kFullBaseSlots);
-        vi_sample_stats* tst = c.take<vi_sample_stats>(tn);
-        vi_sample_stats* dst = c.take<vi_sample_stats>(dn);
-        int32_t* ttok = c.take<int32_t>(tn);
-        int32_t* dtok = c.take<int32_t>(dn);
-        const int ranges = full_ranges(a.vocabulary);
-        double* rsum = c.take<double>(size_t(a.lanes) * ranges * 2);
-        int* rlast = c.take<int>(size_t(a.lanes) * ranges * 2);
-        const size_t fbytes = full_sampler_bytes(v.trows, a.vocabulary);
-        const size_t dbytes = full_sampler_bytes(a.lanes * a.drafts, a.vocabulary);
-        unsigned char* fws = c.take<unsigned char>(fbytes);
-        unsigned char* dws = c.take<unsigned char>(dbytes);
-        if (!c.ok) return VI_ERR_WORKSPACE;
-        hipLaunchKernelGGL(verify_row_params_kernel, dim3((trows + drows + 255) / 256), dim3(256), 0, stream,
-                           a.params, a.lanes, a.target_rows, tpar, a.drafts, dpar);
-        // the rows' filtered distributions (and the target rows' draws) from the
-        // full-vocabulary sampler, each row set in its own workspace: the draft
-        // rows on the side stream beside the target rows on the caller's, joined
-        // back before the accept launch
-        auto sample = [&](const void* logits, int dtype, int rows, int64_t stride, const vi_row_params* par,
-                          int32_t* tok, vi_sample_stats* stats, const FullOut* out, unsigned char* w, size_t wb,
-                          hipStream_t on) {
-            SampleArgs s{};
-            s.logits = logits; s.dtype = dtype; s.rows = rows; s.vocabulary = a.vocabulary; s.stride = stride;
-            s.params = par; s.tokens = tok; s.stats = stats; s.route_mask = VI_ROUTE_FULL; s.full_out = out;
-            return dtype == VI_F32 ? launch_wide(s, w, wb, nullptr, 0, 0, nullptr, on) : launch_full(s, w, wb, on);
-        };
-        const FullOut tout{tb, tbase}, dout{db, dbase};
-        SideStream* side = drows > 0 ? side_stream() : nullptr;
-        if (side && (hipEventRecord(side->fork, stream) != hipSuccess ||
-                     hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess)) {
-            (void)hipGetLastError();
-            side = nullptr;
-        }
-        st = sample(a.draft, a.draft_dtype, drows, a.draft_stride, dpar, dtok, dst, &dout, dws, dbytes,
-                    side ? side->stream : stream);
-        if (st == VI_OK)
-            st = sample(a.target, a.target_dtype, trows, a.target_stride, tpar, ttok, tst, &tout, fws, fbytes, stream);
-        // joined also when a launch failed: the side work uses the caller's workspace
-        if (side && (hipEventRecord(side->join, side->stream) != hipSuccess ||
-                     hipStreamWaitEvent(stream, side->join, 0) != hipSuccess))
-            return VI_ERR_LAUNCH;
-        if (st != VI_OK) return st;
-        FullVerifyArgs f{};
-        f.t = FullRows{a.target, a.target_dtype, a.target_stride, tb, tbase, tst,
-                       a.target_dtype == VI_F32 ? kFullSlice32 : kFullSlice16};
-        f.d = FullRows{a.draft, a.draft_dtype, a.draft_stride, db, dbase, dst,
-                       a.draft_dtype == VI_F32 ? kFullSlice32 : kFullSlice16};
-        f.ttok = ttok; f.lanes = a.lanes; f.drafts = a.drafts; f.target_rows = a.target_rows;
-        f.vocabulary = a.vocabulary; f.drafted = a.drafted; f.params = a.params; f.terminal = a.terminal;
-        f.n_terminal = a.n_terminal; f.dec = dec; f.rsum = rsum; f.rlast = rlast; f.ranges = ranges;
-        switch (a.target_dtype) {
-            case VI_BF16: launch_full_verify_d<VI_BF16>(f, stream); break;
-            case VI_F16: launch_full_verify_d<VI_F16>(f, stream); break;
-            default: launch_full_verify_d<VI_F32>(f, stream); break;
-        }
-        st = launch_status();
-        if (st != VI_OK) return st;
-    }
-    if (!full_ok) return VI_OK;   // (the position launch ran every lane's chain)
     hipLaunchKernelGGL(verify_chain_kernel, dim3(blocks), dim3(threads), 0, stream, dec, a.lanes, a.drafts,
                        a.target_rows, a.drafted, a.params, a.terminal, a.n_terminal, full_ok, a.accepted, a.committed,
                        a.committed_count, a.lane_flags);

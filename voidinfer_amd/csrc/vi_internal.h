@@ -109,23 +109,16 @@ struct VerifyDecideArgs {
     int32_t* committed_count;
     uint32_t* lane_flags;
 };
-vi_status launch_verify_lists(const void* logits, int dtype, int rows, int layout_rows, int layout_slices,
-                              int vocabulary, int64_t stride, const vi_row_params* params, int params_div,
-                              float* lval, int* lidx, uint32_t* lvalid, uint32_t* lflags, int skip_unlisted,
-                              void* ws, size_t ws_bytes, hipStream_t stream, const VerifyDecideArgs* decide = nullptr,
-                              int decide_mode = 0);
-// Target and draft rows of sampled verification in one launch (both row sets
-// 16-byte aligned 16-bit logits, every lane listed): each position's decision
-// is taken by the later of its two rows to finish (a bonus row decides alone),
-// and each lane's last decided position walks the chain.
+// Target and draft rows of sampled verification over top-k lists in one launch:
+// each position's decision is taken by the later of its two rows to finish (a
+// bonus row decides alone), and each lane's last decided position walks the
+// chain.
 vi_status launch_verify_pair(const void* target, int target_dtype, int64_t target_stride, const void* draft,
                              int draft_dtype, int64_t draft_stride, int lanes, int vocabulary,
                              const vi_row_params* params, int layout_rows, int layout_slices, float* tval, int* tidx,
                              uint32_t* tvalid, uint32_t* tflags, float* dval, int* didx, uint32_t* dvalid,
                              uint32_t* dflags, const VerifyDecideArgs& decide, void* ws, size_t ws_bytes,
                              hipStream_t stream, int skip_unlisted);
-bool verify_pair_supported(const void* target, int target_dtype, int64_t target_stride, const void* draft,
-                           int draft_dtype, int64_t draft_stride);
 size_t topk_partials_bytes_slices(int rows, int slices);
 
 // History hash (token -> count) per row for the top-k sampler route.
