@@ -233,3 +233,26 @@ def test_stream_config5_all_rows(orc, dev):
             assert g_st["flags"][r] == w_stats["flags"][r] and g_st["finite"][r] == w_stats["finite"][r], (name, r)
             np.testing.assert_allclose(g_st["support_mass"][r], w_stats["support_mass"][r], rtol=1e-6)
         assert exempt <= 2, (name, exempt)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("rows,vocab", [(3, 200_000), (9, 24_576 * 4 + 8), (1, 12_288 * 2)])
+def test_stream_many_groups_and_top_key(orc, dev, rng, dtype, rows, vocab):
+    """Rows whose logits spread over every exponent (more occupied groups than
+    the merge keeps), and rows whose largest valid key is hard to find: negative
+    logits only, signed zeros only, the highest groups holding nothing valid."""
+    x = rng.standard_normal((9, vocab)).astype(np.float32) * np.exp2(rng.uniform(-14, 4, (9, vocab))).astype(np.float32)
+    x[1] = -np.abs(x[1]) - np.float32(1e-3)
+    x[2] = np.where(rng.random(vocab) < 0.5, 0.0, -0.0)
+    x[3] = np.where(rng.random(vocab) < 0.9, -np.abs(x[3]), -0.0)
+    bits = x.astype(np.float16).view(np.uint16) if dtype else (x.view(np.uint32) >> 16).astype(np.uint16)
+    inf_ = 0x7C00 if dtype else 0x7F80
+    big = 0x7BFF if dtype else 0x7F00
+    bits[1, ::9] = inf_                                  # nothing valid above the negative keys
+    bits[4, ::5] = big                                   # finite patterns whose z overflows (T 1e-36)
+    bits[4, 3] = inf_ + 1
+    bits = bits[:rows] if rows > 1 else bits[4:5]
+    t = np.array([0.7, 0.9, 1.0, 0.5, 1e-36, 0.8, 1.2, 0.6, 0.7], np.float32)
+    p = params(rows, rng, temperature=t[:rows] if rows > 1 else t[4:5], top_k=rng.choice([0, 0, 300], rows),
+               top_p=rng.choice([0.9, 0.95, 1.0], rows), min_p=rng.choice([0.0, 0.01], rows))
+    stream(orc, dev, np.ascontiguousarray(bits), dtype, p, label=f"groups-{dtype}-{rows}-{vocab}")

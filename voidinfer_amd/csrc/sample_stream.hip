@@ -28,8 +28,8 @@
 // once (the repeat list) are corrected at the end of the part: one count moves
 // from the count-1 pattern to the count-c one.  Each thread then owns 32
 // histogram words (a group: 32 positive and 32 negative keys); the non-empty
-// groups are stored at their place in the part's table, with an occupancy
-// bitmap and the part's highest valid key, and the words are cleared.
+// groups are stored at their place in the part's table, with occupancy bitmaps
+// of the groups holding positive and negative patterns, and the words are cleared.
 //
 // Merge launch (merge_kernel, one workgroup per row, on the XCD whose L2 holds
 // the row's tables).  The row's occupied groups are summed over its parts per
@@ -65,7 +65,13 @@ constexpr int kXcds = 8;
 constexpr int kRepPF = 2;                // repeat-list entries prefetched per thread
 constexpr int kMaxParts = 16;            // parts per row
 constexpr int kMaxPartLen = 65504;       // tokens per part (a multiple of 32 below 65,536)
-constexpr int kPub = 32;                 // words per part header: the occupancy bitmap
+constexpr int kPub = 64;                 // words per part header: the occupancy bitmaps, by sign
+// Place of group g in an occupancy bitmap of 32 words: byte g & 127, bit g >> 7
+// (the order in which a publishing thread meets its groups).
+struct GroupBit {
+    uint32_t word, shift;
+};
+__device__ __forceinline__ GroupBit group_bit(uint32_t g) { return GroupBit{(g & 127u) >> 2, ((g & 3u) << 3) | (g >> 7)}; }
 constexpr uint32_t kTakeAll = 0xffffffffu;
 constexpr double kFix = 0x1p40;          // fixed-point scale of the masses (w <= 1, counts <= 2^20)
 
@@ -83,8 +89,8 @@ static_assert(kLds == 155648, "LDS map");
 // what the fixed arrays leave (more groups than that are summed again from the
 // parts' tables when needed).
 constexpr int kOffMBits = 0;                          // u32[kMaxParts][32]: each part's occupied groups
-constexpr int kOffMOcc = kOffMBits + 4 * 32 * kMaxParts;   // u32[32]: occupied in any part
-constexpr int kOffMSlot = kOffMOcc + 128;             // u16[1024]: slot of group g
+constexpr int kOffMOcc = kOffMBits + 4 * 32 * kMaxParts;   // u32[3][32]: occupied in any part, by sign too
+constexpr int kOffMSlot = kOffMOcc + 384;             // u16[1024]: slot of group g
 constexpr int kOffMGroupOf = kOffMSlot + 2048;        // u16[1024]: group of slot s
 constexpr int kOffMBcnt = kOffMGroupOf + 2048;        // u32[2048]: logits per 32-key block
 constexpr int kOffMBmass = kOffMBcnt + 8192;          // u64[2048]: block masses, fixed point
@@ -275,8 +281,8 @@ constexpr int kMaxItems = 1024;          // parts one workgroup can take
 struct StreamShared {
     int items[kMaxItems];                // the workgroup's parts (indices among its XCD's), in order
     uint32_t scan[kW + 1];
-    // the part's occupied groups: byte q * 16 + wave, bit i -> group q * 128 + wave * 8 + i
-    unsigned char occb[kGroups / 8];
+    // the part's groups holding positive and negative patterns (GroupBit's order)
+    unsigned char occb[2][kGroups / 8];
 };
 
 // The presence bytes (one per vector) of a row from token s0: the lane
@@ -525,27 +531,28 @@ __global__ __launch_bounds__(kT) void stream_kernel(StreamArgs a) {
             uint4* dst = a.pwords + pi * (kGroups * kGW / 4);
             const int t = opaque_tid();
             uint4* H4 = reinterpret_cast<uint4*>(H);
+            uint32_t occ_p = 0u, occ_n = 0u;   // bit q: the thread's group of round q
 #pragma unroll
             for (int q = 0; q < kHW / 4 / kT; ++q) {
                 const int c = q * kT + t;            // 16-byte chunk c: words 4c .. 4c + 3 of group c / 8
                 const uint4 d = H4[c];
                 H4[c] = make_uint4(0u, 0u, 0u, 0u);
-                const uint64_t bm = ballot((d.x | d.y | d.z | d.w) != 0u);
-                // bit 8i of sm: group i of the wave's eight is occupied
-                uint64_t sm = bm | (bm >> 4);
-                sm |= sm >> 2;
-                sm |= sm >> 1;
-                sm &= 0x0101010101010101ull;
-                const uint64_t lanes = (sm << 8) - sm;   // the occupied groups' lanes
-                const uint32_t half = lane < 32 ? uint32_t(lanes) : uint32_t(lanes >> 32);
-                if ((half >> (lane & 31)) & 1u) dst[c] = d;
-                if (lane == 0) {
-                    const uint32_t lo = uint32_t(sm), hi = uint32_t(sm >> 32);
-                    sh.occb[q * kW + wave] = uint8_t((((lo * 0x00204081u) >> 21) & 0xfu) | ((((hi * 0x00204081u) >> 21) & 0xfu) << 4));
-                }
+                // the halves any word of the group holds: over its eight lanes, lane
+                // ^ 1, ^ 2, then the mirrored half row (uniform quads by then)
+                uint32_t any = (d.x | d.y) | (d.z | d.w);
+                any |= dpp_u32<0xb1, 0xf, false>(any);
+                any |= dpp_u32<0x4e, 0xf, false>(any);
+                any |= dpp_u32<0x141, 0xf, false>(any);
+                if (any) dst[c] = d;
+                occ_p |= min(any & 0xffffu, 1u) << q;
+                occ_n |= min(any >> 16, 1u) << q;
+            }
+            if ((lane & 7) == 0) {   // groups q * 128 + wave * 8 + lane / 8
+                sh.occb[0][tid >> 3] = uint8_t(occ_p);
+                sh.occb[1][tid >> 3] = uint8_t(occ_n);
             }
             lds_barrier();
-            if (tid < 32) a.ppub[pi * kPub + tid] = reinterpret_cast<const uint32_t*>(sh.occb)[tid];
+            if (tid < kPub) a.ppub[pi * kPub + tid] = reinterpret_cast<const uint32_t*>(sh.occb)[tid];
             // Stores and loads share one counter and may complete out of order:
             // with a store outstanding every wait on a load would have to drain
             // the counter.  Drain it once here instead.
@@ -632,7 +639,14 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     const float inv_t = 1.0f / p.temperature;
 
     // ---- 0. the parts' occupancy bitmaps; the valid key range
-    for (int i = tid; i < P * 32; i += kT) pbits[i] = a.ppub[(pi0 + i / 32) * kPub + i % 32];
+    if (tid < 96) occ[tid] = 0u;
+    uint32_t pub[2] = {0u, 0u};   // (thread i: word i % 32 of part i / 32; at most 512 words)
+    static_assert(kMaxParts * 32 <= kT, "one bitmap word per thread");
+    if (tid < P * 32) {
+        pub[0] = a.ppub[(pi0 + tid / 32) * kPub + tid % 32];
+        pub[1] = a.ppub[(pi0 + tid / 32) * kPub + 32 + tid % 32];
+        pbits[tid] = pub[0] | pub[1];
+    }
     // The first repeat entries (two per thread), requested now (reads within
     // the list whatever it holds); their logits are gathered once the owner
     // part is known, for the entries inside it only.
@@ -652,15 +666,16 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     for (int i = tid; i < 2048; i += kT) { bcnt[i] = 0u; bmass[i] = 0ull; }
     if (tid == 0) { sh.flags = pv.flags; sh.token = -1; sh.ok = 1u; sh.z0key = 0u; }
     lds_barrier();
-    if (tid < 32) {
-        uint32_t o = 0u;
-        for (int pp = 0; pp < P; ++pp) o |= pbits[pp * 32 + tid];
-        occ[tid] = o;
+    if (tid < P * 32) {
+        atomicOr(&occ[tid % 32], pub[0] | pub[1]);
+        atomicOr(&occ[32 + tid % 32], pub[0]);
+        atomicOr(&occ[64 + tid % 32], pub[1]);
     }
     lds_barrier();
     // a slot per occupied group
     {
-        const uint32_t o = (occ[tid >> 5] >> (tid & 31)) & 1u;
+        const GroupBit gb = group_bit(uint32_t(tid));
+        const uint32_t o = (occ[gb.word] >> gb.shift) & 1u;
         uint32_t n = 0u;
         const uint32_t e = block_scan_lds(o, sh.scan, &n);
         if (o) { slot_of[tid] = uint16_t(e); group_of[e] = uint16_t(tid); }
@@ -676,6 +691,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     // lo1, hi1); the parts' loads four at a time.
     auto sum_pair = [&](uint32_t g, uint32_t q) -> uint4 {
         uint4 c = make_uint4(0u, 0u, 0u, 0u);
+        const GroupBit gb = group_bit(g);
         const uint64_t* src = reinterpret_cast<const uint64_t*>(a.pwords);
         for (int p0 = 0; p0 < P; p0 += 4) {
             uint64_t w2[4];
@@ -683,7 +699,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             for (int k = 0; k < 4; ++k) {
                 const int pp = p0 + k;
                 w2[k] = 0ull;
-                if (pp < P && ((pbits[pp * 32 + (g >> 5)] >> (g & 31u)) & 1u))
+                if (pp < P && ((pbits[pp * 32 + gb.word] >> gb.shift) & 1u))
                     w2[k] = src[((pi0 + pp) * kGroups + g) * 16 + q];
             }
 #pragma unroll
@@ -695,107 +711,163 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         if (g == 0u && q == 0u) { c.x += c.y; c.y = 0u; }   // -0 is +0
         return c;
     };
-    // ---- 1. per-key counts summed over the parts (a task: two words of a
-    // group; two tasks per thread, their loads issued together) and the
-    // highest valid key present, z0's.  Past kSlotCap occupied groups the
-    // counts are not kept: a second pass adds them to the block sums.
-    const uint32_t ntask = nslots * 16u;
-    auto task_keys = [&](uint32_t t) { return uint32_t(group_of[t >> 4]) * kGW + 2u * (t & 15u); };
-    auto top_of = [&](uint32_t t, uint4 c) -> uint32_t {
-        const uint32_t w0 = task_keys(t);
-        uint32_t m = 0u;
-        auto consider = [&](uint32_t k, uint32_t n) {
-            if (n && key_valid<DT>(k, kmin, kmax)) m = max(m, k);
-        };
-        consider(0x8000u + w0, c.x); consider(0x7fffu - w0, c.y); consider(0x8001u + w0, c.z); consider(0x7ffeu - w0, c.w);
-        return m;
+    // ---- 1. the highest valid key present, z0's, by the last wave: the highest
+    // group holding a positive pattern (the lowest holding a negative one) is
+    // known from the bitmaps, so one read of its 32 words finds the key
+    auto word_or = [&](uint32_t g) -> uint32_t {   // (lanes 0..31: word `lane` of group g, any part's halves)
+        uint32_t w = 0u;
+        const GroupBit gb = group_bit(g);
+        const uint32_t* src = reinterpret_cast<const uint32_t*>(a.pwords);
+        for (int p0 = 0; p0 < P; p0 += 4) {
+            uint32_t w4[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int pp = min(p0 + k, P - 1);
+                w4[k] = src[((pi0 + pp) * kGroups + g) * kGW + uint32_t(lane & 31)];
+                if (!((pbits[pp * 32 + gb.word] >> gb.shift) & 1u)) w4[k] = 0u;
+            }
+            w |= (w4[0] | w4[1]) | (w4[2] | w4[3]);
+        }
+        return lane < 32 ? w : 0u;
     };
-    {
-        uint32_t top = 0u;
-        for (uint32_t t0 = 0; t0 < ntask; t0 += 2 * kT) {
-            const uint32_t ta = t0 + uint32_t(tid), tb = ta + kT;
-            const bool va = ta < ntask, vb = tb < ntask;
-            const uint4 ca = va ? sum_pair(group_of[ta >> 4], ta & 15u) : make_uint4(0u, 0u, 0u, 0u);
-            const uint4 cb = vb ? sum_pair(group_of[tb >> 4], tb & 15u) : make_uint4(0u, 0u, 0u, 0u);
-            if (store_keys) {
-                if (va) keys[ta] = ca;
-                if (vb) keys[tb] = cb;
-            }
-            if (va) top = max(top, top_of(ta, ca));
-            if (vb) top = max(top, top_of(tb, cb));
-        }
+    auto find_top = [&]() -> uint32_t {
+        if (kmin > kmax) return 0u;
+        // (byte j of word `lane`: bit q is group q * 128 + 4 * lane + j)
+        uint32_t m = lane < 32 ? occ[32 + lane] : 0u;   // groups of positive patterns, highest first
+        while (ballot(m != 0u)) {
+            uint32_t g = 0u;
 #pragma unroll
-        for (int o = 32; o; o >>= 1) top = max(top, uint32_t(__shfl_xor(int(top), o, kWave)));
-        if (lane == 0 && top) atomicMax(&sh.z0key, top);
-    }
-    lds_barrier();
-    const uint32_t z0key = sh.z0key;
-    const double z0 = double(key_z<DT>(z0key, inv_t));
-    if (!store_keys) {   // (block sums straight from the counts)
-        auto add = [&](uint32_t k, uint32_t c) {
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t b = (m >> (8u * j)) & 0xffu;
+                if (b) g = max(g, ((31u - uint32_t(__builtin_clz(b))) << 7) | (4u * uint32_t(lane) + j));
+            }
+#pragma unroll
+            for (int o = 32; o; o >>= 1) g = max(g, uint32_t(__shfl_xor(int(g), o, kWave)));
+            const GroupBit gb = group_bit(g);
+            if (uint32_t(lane) == gb.word) m &= ~(1u << gb.shift);
+            if (0x8000u + 32u * g > kmax) continue;
+            const uint64_t h = ballot((word_or(g) & 0xffffu) && 0x8000u + 32u * g + uint32_t(lane) <= kmax);
+            if (h) return 0x8000u + 32u * g + 63u - uint32_t(__builtin_clzll(h));
+        }
+        m = lane < 32 ? occ[64 + lane] : 0u;            // negative patterns, lowest first (-0 is +0)
+        while (ballot(m != 0u)) {
+            uint32_t g = kGroups;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t b = (m >> (8u * j)) & 0xffu;
+                if (b) g = min(g, (uint32_t(__builtin_ctz(b)) << 7) | (4u * uint32_t(lane) + j));
+            }
+#pragma unroll
+            for (int o = 32; o; o >>= 1) g = min(g, uint32_t(__shfl_xor(int(g), o, kWave)));
+            const GroupBit gb = group_bit(g);
+            if (uint32_t(lane) == gb.word) m &= ~(1u << gb.shift);
+            const uint32_t wd = 32u * g + uint32_t(lane & 31);
+            const uint64_t h = ballot((word_or(g) >> 16) && (wd == 0u || 0x7fffu - wd >= kmin));
+            if (h) {
+                const uint32_t w0 = 32u * g + uint32_t(__builtin_ctzll(h));
+                return w0 == 0u ? 0x8000u : 0x7fffu - w0;
+            }
+        }
+        return 0u;
+    };
+    // ---- 2. per-key counts summed over the parts and the block sums in one
+    // pass (a task: four words of a group, 16 bytes per part; two tasks per
+    // thread, their loads issued together, the first pair's while the last wave
+    // finds z0).  A 32-key block's sums are the eight lanes' of its group and
+    // sign.  Counts of the first kSlotCap occupied groups are kept for the
+    // decisions (past it they are summed again there).  (With z0 found from the
+    // counts, rows of more groups than the LDS keeps took two passes and an
+    // atomic per key: fp16 N(0, 1.4), 81 x 168,896, merge
+    // 48.6 us then, 31.8 now.)
+    const uint32_t ntask = nslots * 8u;
+    auto sum_quad = [&](uint32_t t, uint32_t (&lo)[4], uint32_t (&hi)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lo[i] = hi[i] = 0u;
+        if (t >= ntask) return;
+        const uint32_t g = group_of[t >> 3], q = t & 7u;
+        const GroupBit gb = group_bit(g);
+        for (int p0 = 0; p0 < P; p0 += 4) {
+            uint4 w4[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int pp = p0 + k;
+                w4[k] = make_uint4(0u, 0u, 0u, 0u);
+                if (pp < P && ((pbits[pp * 32 + gb.word] >> gb.shift) & 1u))
+                    w4[k] = a.pwords[((pi0 + pp) * kGroups + g) * (kGW / 4) + q];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                lo[0] += w4[k].x & 0xffffu; hi[0] += w4[k].x >> 16;
+                lo[1] += w4[k].y & 0xffffu; hi[1] += w4[k].y >> 16;
+                lo[2] += w4[k].z & 0xffffu; hi[2] += w4[k].z >> 16;
+                lo[3] += w4[k].w & 0xffffu; hi[3] += w4[k].w >> 16;
+            }
+        }
+        if (g == 0u && q == 0u) { lo[0] += hi[0]; hi[0] = 0u; }   // -0 is +0
+    };
+    double z0 = 0.0;
+    uint32_t z0key = 0u;
+    bool invalid = false;
+    auto add_quad = [&](uint32_t t, const uint32_t (&lo)[4], const uint32_t (&hi)[4]) {
+        const uint32_t s = min(t, ntask - 1u) >> 3, g = group_of[s], q = t & 7u, w0 = g * kGW + 4u * q;
+        if (store_keys && t < ntask) {
+            keys[s * 16u + 2u * q] = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+            keys[s * 16u + 2u * q + 1u] = make_uint4(lo[2], hi[2], lo[3], hi[3]);
+        }
+        uint32_t cp = 0u, cn = 0u;
+        uint64_t mp = 0ull, mn = 0ull;
+        auto add = [&](uint32_t k, uint32_t c, uint32_t& cs, uint64_t& ms) {
             if (!c) return;
-            if (!key_valid<DT>(k, kmin, kmax)) { atomicOr(&sh.flags, uint32_t(VI_FLAG_NONFINITE)); return; }
-            atomicAdd(&bcnt[k >> 5], c);
-            atomicAdd(reinterpret_cast<unsigned long long*>(&bmass[k >> 5]),
-                      (unsigned long long)fixed_mass(c, key_weight<DT>(k, inv_t, z0)));
+            if (!key_valid<DT>(k, kmin, kmax)) { invalid = true; return; }
+            cs += c;
+            ms += fixed_mass(c, key_weight<DT>(k, inv_t, z0));
         };
-        auto add4 = [&](uint32_t t, uint4 c) {
-            const uint32_t w0 = task_keys(t);
-            add(0x8000u + w0, c.x); add(0x7fffu - w0, c.y); add(0x8001u + w0, c.z); add(0x7ffeu - w0, c.w);
-        };
-        for (uint32_t t0 = 0; t0 < ntask; t0 += 2 * kT) {
-            const uint32_t ta = t0 + uint32_t(tid), tb = ta + kT;
-            const bool va = ta < ntask, vb = tb < ntask;
-            const uint4 ca = va ? sum_pair(group_of[ta >> 4], ta & 15u) : make_uint4(0u, 0u, 0u, 0u);
-            const uint4 cb = vb ? sum_pair(group_of[tb >> 4], tb & 15u) : make_uint4(0u, 0u, 0u, 0u);
-            if (va) add4(ta, ca);
-            if (vb) add4(tb, cb);
-        }
-        lds_barrier();
-    }
-    // ---- 2. block sums: four threads per 32-key block, eight keys each
-    if (store_keys) {
-        const uint32_t nunits = nslots * 8u;
-        for (uint32_t u0 = 0; u0 < nunits; u0 += kT) {
-            const uint32_t u = u0 + uint32_t(tid);
-            uint32_t c8 = 0u, blk = 0u;
-            uint64_t m8 = 0ull;
-            bool bad = false;
-            if (u < nunits) {
-                const uint32_t s = u >> 3, neg = (u >> 2) & 1u, qq = u & 3u, g = group_of[s];
 #pragma unroll
-                for (int i = 0; i < 8; i += 2) {
-                    const uint4 c2 = keys[s * 16u + 4u * qq + uint32_t(i) / 2u];
-                    const uint32_t wd = g * kGW + 8u * qq + uint32_t(i);
-                    const uint32_t ca = neg ? c2.y : c2.x, cb = neg ? c2.w : c2.z;
-                    const uint32_t ka = neg ? 0x7fffu - wd : 0x8000u + wd, kb = neg ? 0x7ffeu - wd : 0x8001u + wd;
-                    if (ca) {
-                        if (key_valid<DT>(ka, kmin, kmax)) { c8 += ca; m8 += fixed_mass(ca, key_weight<DT>(ka, inv_t, z0)); }
-                        else bad = true;
-                    }
-                    if (cb) {
-                        if (key_valid<DT>(kb, kmin, kmax)) { c8 += cb; m8 += fixed_mass(cb, key_weight<DT>(kb, inv_t, z0)); }
-                        else bad = true;
-                    }
-                }
-                blk = neg ? 1023u - g : 1024u + g;
-            }
-            // the four quarters of a block are lanes 4i .. 4i + 3
-            c8 += dpp_u32<0xb1, 0xf, false>(c8);   // quad_perm [1,0,3,2]
-            c8 += dpp_u32<0x4e, 0xf, false>(c8);   // quad_perm [2,3,0,1]
-            {
-                const uint64_t o1 = uint64_t(dpp_u32<0xb1, 0xf, false>(uint32_t(m8))) |
-                                    (uint64_t(dpp_u32<0xb1, 0xf, false>(uint32_t(m8 >> 32))) << 32);
-                m8 += o1;
-                const uint64_t o2 = uint64_t(dpp_u32<0x4e, 0xf, false>(uint32_t(m8))) |
-                                    (uint64_t(dpp_u32<0x4e, 0xf, false>(uint32_t(m8 >> 32))) << 32);
-                m8 += o2;
-            }
-            if (u < nunits && (u & 3u) == 0u) { bcnt[blk] = c8; bmass[blk] = m8; }
-            if (ballot(bad) && lane == 0) atomicOr(&sh.flags, uint32_t(VI_FLAG_NONFINITE));
+        for (int i = 0; i < 4; ++i) {
+            add(0x8000u + w0 + uint32_t(i), lo[i], cp, mp);
+            add(0x7fffu - w0 - uint32_t(i), hi[i], cn, mn);
         }
-        lds_barrier();
+        // over the group's eight lanes: lane ^ 1, ^ 2, then the mirrored half row
+        // (uniform quads by then)
+        auto dpp64 = [](uint64_t v, auto dpp) {
+            return uint64_t(dpp(uint32_t(v))) | (uint64_t(dpp(uint32_t(v >> 32))) << 32);
+        };
+        auto step = [&](auto dpp) {
+            cp += dpp(cp);
+            cn += dpp(cn);
+            mp += dpp64(mp, dpp);
+            mn += dpp64(mn, dpp);
+        };
+        step([](uint32_t u) { return dpp_u32<0xb1, 0xf, false>(u); });
+        step([](uint32_t u) { return dpp_u32<0x4e, 0xf, false>(u); });
+        step([](uint32_t u) { return dpp_u32<0x141, 0xf, false>(u); });
+        if (t < ntask && q == 0u) {
+            bcnt[1024u + g] = cp;
+            bmass[1024u + g] = mp;
+            bcnt[1023u - g] = cn;
+            bmass[1023u - g] = mn;
+        }
+    };
+    for (uint32_t t0 = 0; t0 < ntask || t0 == 0u; t0 += 2 * kT) {   // (uniform; the first turn always: z0)
+        uint32_t la[4], ha[4], lb[4], hb[4];
+        const uint32_t ta = t0 + uint32_t(tid), tb = ta + kT;
+        if (t0 == 0u && wave == kW - 1) {
+            const uint32_t top = find_top();
+            if (lane == 0) sh.z0key = top;
+        }
+        sum_quad(ta, la, ha);
+        sum_quad(tb, lb, hb);
+        if (t0 == 0u) {
+            lds_barrier();
+            z0key = sh.z0key;
+            z0 = double(key_z<DT>(z0key, inv_t));
+            if (ntask == 0u) break;
+        }
+        add_quad(ta, la, ha);
+        if (t0 + kT < ntask) add_quad(tb, lb, hb);   // (uniform)
     }
+    if (ballot(invalid) && lane == 0) atomicOr(&sh.flags, uint32_t(VI_FLAG_NONFINITE));
+    lds_barrier();
     // ---- 3. descending prefix sums over the 2048 blocks (thread t: blocks
     // 2047 - 2t and 2046 - 2t)
     {
@@ -842,7 +914,8 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         const uint32_t k = 32u * b + 31u - uint32_t(lane & 31);
         if (lane >= 32 || !key_valid<DT>(k, kmin, kmax)) return 0u;
         const KeyLoc kl = key_loc(k);
-        if (!((occ[kl.group >> 5] >> (kl.group & 31u)) & 1u)) return 0u;
+        const GroupBit gb = group_bit(kl.group);
+        if (!((occ[gb.word] >> gb.shift) & 1u)) return 0u;
         const uint4 c = store_keys ? keys[uint32_t(slot_of[kl.group]) * 16u + (kl.word >> 1)]
                                    : sum_pair(kl.group, kl.word >> 1);
         const uint32_t lo = (kl.word & 1u) ? c.z : c.x, hi = (kl.word & 1u) ? c.w : c.y;
@@ -1024,8 +1097,9 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     if (wave == 0 && sh.ok) {
         const uint32_t dk = sh.draw_key;
         const KeyLoc kl = key_loc(dk);
+        const GroupBit gb = group_bit(kl.group);
         uint32_t c = 0u;
-        if (lane < P && ((pbits[lane * 32 + (kl.group >> 5)] >> (kl.group & 31u)) & 1u)) {
+        if (lane < P && ((pbits[lane * 32 + gb.word] >> gb.shift) & 1u)) {
             const uint64_t* src = reinterpret_cast<const uint64_t*>(a.pwords) + ((pi0 + lane) * kGroups + kl.group) * 16;
             const uint64_t w2 = src[kl.word >> 1];
             const uint32_t wd = (kl.word & 1u) ? uint32_t(w2 >> 32) : uint32_t(w2);
@@ -1368,11 +1442,18 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
 struct StreamPlan {
     int parts, part_len;
 };
-static StreamPlan stream_plan(int rows, int vocabulary) {
+static StreamPlan stream_plan(int rows, int vocabulary, int dtype) {
     const int cus = device_cus();
     int parts = (vocabulary + kMaxPartLen - 1) / kMaxPartLen;
     const int fill = (cus + std::max(rows, 1) - 1) / std::max(rows, 1);   // parts that give every CU one
-    parts = std::max(parts, std::min(kMaxParts, fill));
+    // Few rows: as many parts as the CUs take, but none so short that the merge,
+    // one workgroup per row that reads every part's table, loses more than the
+    // stream wins.  fp16 rows spread over some hundred groups a part, bf16 rows
+    // over a few dozen.  Stream + merge, us, with 16 / 8 / 4 parts: fp16 2 x
+    // 162,880 8.8 + 43.2 / 10.5 + 34.1 / 12.8 + 30.6; bf16 8 x 248,320 9.5 + 19.8 /
+    // 11.0 + 19.8 / 15.0 + 20.1; bf16 3 x 45,568 6.4 + 16.9 / 6.3 + 15.8 / 6.4 + 14.7.
+    const int shortest = dtype == VI_F16 ? 24576 : 12288;
+    parts = std::max(parts, std::min({kMaxParts, fill, vocabulary / shortest}));
     // a multiple of 32 tokens: every part's presence bytes start 4-byte aligned
     const int len = ((vocabulary + parts - 1) / parts + 31) / 32 * 32;
     return {(vocabulary + len - 1) / len, len};
@@ -1405,7 +1486,7 @@ bool stream_supported(const SampleArgs& s) {
     if (s.vocabulary <= 0 || s.vocabulary % 8 || s.vocabulary > kMaxParts * kMaxPartLen) return false;
     if (s.stride < s.vocabulary || s.stride % 8 || reinterpret_cast<uintptr_t>(s.logits) % 16) return false;
     if (int64_t(s.rows) * kMaxParts > (int64_t(1) << 30)) return false;
-    if (stream_grid(s.rows, stream_plan(s.rows, s.vocabulary).parts).per_wg > kMaxItems) return false;
+    if (stream_grid(s.rows, stream_plan(s.rows, s.vocabulary, s.dtype).parts).per_wg > kMaxItems) return false;
     const bool hist = !s.pstate && s.histories && s.offsets && s.max_history > 0;
     if (hist && !hist_fits(s.vocabulary, s.max_history)) return false;
     return true;
@@ -1413,8 +1494,8 @@ bool stream_supported(const SampleArgs& s) {
 
 size_t stream_workspace(int rows, int vocabulary, int64_t max_history) {
     if (rows <= 0 || vocabulary <= 0 || vocabulary % 8 || vocabulary > kMaxParts * kMaxPartLen) return 0;
-    const StreamPlan pl = stream_plan(rows, vocabulary);
-    const size_t np = size_t(rows) * pl.parts;
+    // (bf16 rows take the most parts)
+    const size_t np = size_t(rows) * stream_plan(rows, vocabulary, VI_BF16).parts;
     size_t b = align_up(np * kPub * 4, 256) + align_up(np * kGroups * kGW * 4, 256);
     if (max_history > 0 && hist_fits(vocabulary, max_history))
         b += align_up(size_t(rows) * hist_words(vocabulary) * 4, 256) +
@@ -1424,7 +1505,7 @@ size_t stream_workspace(int rows, int vocabulary, int64_t max_history) {
 
 vi_status launch_stream(const SampleArgs& s, unsigned char* ws, size_t ws_bytes, hipStream_t stream) {
     if (!stream_supported(s)) return VI_ERR_UNSUPPORTED;
-    const StreamPlan pl = stream_plan(s.rows, s.vocabulary);
+    const StreamPlan pl = stream_plan(s.rows, s.vocabulary, s.dtype);
     StreamArgs a{};
     a.logits = s.logits; a.rows = s.rows; a.vocabulary = s.vocabulary; a.stride = s.stride;
     a.parts = pl.parts; a.part_len = pl.part_len;
