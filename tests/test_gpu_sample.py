@@ -456,3 +456,34 @@ def test_presence_table_kernels(orc, dev, rng):
     vi.presence_truncate(table, 12)
     t = table.cpu().numpy()
     assert t[5] == 10 and t[7] == 11 and t[9999] == 0x7F7F7F7F and t[3] == 0x7F7F7F7F
+
+
+@pytest.mark.parametrize("vocab", [1, 3, 16_386, 32_769, 70_001])
+def test_full_route_fp32_slice_edges_and_long_chains(orc, dev, rng, vocab):
+    """fp32 rows whose last slice has no whole vector, near-flat rows whose cap,
+    cuts and draw share crowded bins, anchors past 2^120, top_k caps below and
+    inside the deep bin; penalties from histories and from states whose hashes
+    are loaded enough for probe chains past the first four slots."""
+    import voidinfer_amd as vi
+    rows = 8
+    x = make_rows(rng, rows, vocab, std=0.1, dtype=2, zipf=False)
+    x[1] = -2e37 * (1.0 + np.abs(x[1]))                      # |z| past 2^120, every row bin wide
+    x[2] *= 1000.0
+    x[3, ::2] += 5.0
+    x[4] = np.round(x[4] * 8) / 8                            # few distinct values
+    p = params(rows, rng, temperature=np.array([0.7, 1.0, 0.5, 1.2, 0.9, 0.3, 0.8, 1.0], np.float32),
+               top_k=np.array([0, 0, 700, 0, 100, 9000, 65, 0]), top_p=np.array([.95, .9, .99, .5, 1, .9, 1, .95], np.float32),
+               min_p=np.array([0, 0, 0, .2, 0, .5, .01, 1.0], np.float32), repetition_penalty=1.1, frequency_penalty=0.02,
+               presence_penalty=0.1)
+    n = min(500, vocab)
+    h = [np.repeat(rng.choice(vocab, n, replace=False), rng.integers(1, 4, n)).astype(np.int32) for _ in range(rows)]
+    offs = np.concatenate([[0], np.cumsum([len(v) for v in h])]).astype(np.int64)
+    hist = np.concatenate(h)
+    g, w = run_both(orc, dev, x, 2, p, hist, offs)
+    compare(g, w, p, f"fp32-{vocab}")
+    state = vi.PenaltyState(rows, vocab, slots=512, device=dev)   # up to 500 tokens in 512 slots
+    state.update(torch.from_numpy(hist).to(dev), torch.from_numpy(offs).to(dev))
+    out = vi.sample_rows_state(to_dev(x, 2, dev), p, state, want_probs=True)
+    assert np.array_equal(out.tokens.cpu().numpy(), g["tokens"])
+    assert np.array_equal(vi.stats_numpy(out.stats), g["stats"])
+    assert np.array_equal(out.probs.cpu().numpy(), g["probs"])

@@ -137,9 +137,9 @@ __device__ __forceinline__ uint4 load16(const void* p) {
     const u32x4_t v = __builtin_nontemporal_load(static_cast<const u32x4_any_t*>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
 }
-// Ordinary (cached) 16-byte load.
+// Ordinary (cached) 16-byte load, from any address.
 __device__ __forceinline__ uint4 load16_cached(const void* p) {
-    const u32x4_t v = *static_cast<const u32x4_t*>(p);
+    const u32x4_t v = *static_cast<const u32x4_any_t*>(p);
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
