@@ -213,7 +213,7 @@ def latency(args):
         "warmup": args.warmup, "ms_per_step": s_lat["gpu_us_p50"] / 1e3, "higher_is_better": False,
         "scaling": "weak", "vs_baseline": None, "dtype": "fp32" if dtype == vi.F32 else "bf16", "data": "synthetic",
         "config": {"workload": workload, "rows": int(rows), "vocabulary": int(V), "history": max_h,
-                   "routes": int(routes), "kernel": "vi_sample_rows (topk.hip / sample_slices.hip routes)"},
+                   "routes": int(routes), "kernel": "vi_sample_rows (topk.hip / sample_stream.hip routes)"},
         "latency": {"sampled": s_lat, "greedy": g_lat},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_GBPS, "unit": "GB/s",
                      "frac": achieved / PEAK_GBPS, "traffic": None, "bytes_per_launch": bytes_per_call,

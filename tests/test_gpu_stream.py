@@ -1,11 +1,9 @@
 """GPU full-vocabulary rows in one launch (csrc/sample_stream.hip) vs the CPU oracle.
 
 The stream route serves the 16-bit full-route rows (temperature > 0, top_k 0 or
-> 64) of vi_sample_rows / vi_sample_rows_state when no probabilities are
-wanted and the rows are 16-byte aligned with a vocabulary that is a multiple of
-8; these tests call the sampler that way.  Bar (north star): token ids equal
-to the oracle's except where a cumulative-mass boundary lies within 1e-6 of
-the drawn uniform or of a cut; support sizes, finite counts and flags equal
+> 64) of vi_sample_rows / vi_sample_rows_state.  Bar: token ids equal to the
+oracle's except where a cumulative-mass boundary lies within 1e-6 of the drawn
+uniform or of a cut; support sizes, finite counts and flags equal
 outside exempt rows; Philox uniforms bit-exact; support mass within 1e-6.
 Cases: vocabularies from 64 to 248,320 and part boundaries (65,528 tokens),
 one to 128 rows (one to sixteen parts per row), caps above 64, min-p, top-p,
@@ -256,3 +254,39 @@ def test_stream_many_groups_and_top_key(orc, dev, rng, dtype, rows, vocab):
     p = params(rows, rng, temperature=t[:rows] if rows > 1 else t[4:5], top_k=rng.choice([0, 0, 300], rows),
                top_p=rng.choice([0.9, 0.95, 1.0], rows), min_p=rng.choice([0.0, 0.01], rows))
     stream(orc, dev, np.ascontiguousarray(bits), dtype, p, label=f"groups-{dtype}-{rows}-{vocab}")
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("vocab", [1, 7, 13, 4_099, 65_505, 131_015, 500_001])
+def test_stream_odd_rows_and_probabilities(orc, dev, rng, dtype, vocab):
+    """Rows off a 16-byte boundary, logits past the last whole vector (a last part
+    of one logit at 65,505), supports that cut the logits of their last key, the
+    distribution's tokens seen once and more than once; at 500,001 tokens the
+    history view's bitmaps and counts exceed the LDS."""
+    rows, L = 9, 24_000 if vocab > 400_000 else 600
+    bits = make_rows(rng, rows, vocab, std=1.0, dtype=dtype)
+    bits[1::4] &= 0xFFC0 if dtype == 0 else 0xFE00        # few values: many ties at every cut
+    bits[2, -1] = bits[2].max() if vocab < 8 else 0x4380   # the row's last logit is drawn
+    p = params(rows, rng, temperature=rng.uniform(0.5, 1.2, rows), top_k=rng.choice([0, 70, 1000], rows),
+               top_p=rng.choice([0.8, 0.95, 1.0], rows), min_p=rng.choice([0.0, 0.0, 0.02], rows),
+               repetition_penalty=rng.uniform(1.0, 1.2, rows), presence_penalty=0.1, frequency_penalty=0.03)
+    p["repetition_penalty"][3], p["presence_penalty"][3], p["frequency_penalty"][3] = 1.0, 0.0, 0.0
+    hist = rng.integers(0, vocab, (rows, L)).astype(np.int32)
+    hist[:, :40] = rng.integers(max(0, vocab - 9), vocab, (rows, 40))   # the tail's tokens, repeated
+    offs = np.arange(rows + 1, dtype=np.int64) * L
+    compare(*run_both(orc, dev, bits, dtype, p, hist.reshape(-1), offs, want_probs=True), p, f"odd-{dtype}-{vocab}")
+
+
+def test_stream_more_rows_than_one_launch(orc, dev, rng):
+    """32,777 rows: two launches over the same tables, the second of nine rows."""
+    import voidinfer_amd as vi
+    rows, vocab = 32_777, 40
+    bits = make_rows(rng, 64, vocab, std=1.0)[np.arange(rows) % 64]
+    p = params(rows, rng, temperature=0.8, top_k=0, top_p=0.9)
+    out = vi.sample_rows(to_dev(bits, 0, dev), p, want_probs=True)
+    torch.cuda.synchronize()
+    at = np.array([0, 1, 8_191, 32_767, 32_768, 32_769, 32_776])
+    g = dict(tokens=out.tokens.cpu().numpy()[at], u=out.uniforms.cpu().numpy()[at], probs=out.probs.cpu().numpy()[at],
+             stats=vi.stats_numpy(out.stats)[at])
+    tok, u, probs, stats, margins = orc.sample_rows(bits[at], 0, p[at], None, None, want_probs=True)
+    compare(g, dict(tokens=tok, u=u, probs=probs, stats=stats, margins=margins), p[at], "rows")

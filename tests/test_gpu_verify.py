@@ -276,3 +276,30 @@ def test_sampled_lists_every_dtype_pair(orc, dev, rng, tdt, ddt, vocab):
                        draft=to_dev(db, ddt, dev), params=p)
     w = orc.verify_rows(1, tb, tdt, db, ddt, lanes, drafts, drafted, p, ())
     assert_same(g, w, {l for l in range(lanes) if np.min(w[4][l]) < 1e-9})
+
+
+@pytest.mark.parametrize("lanes,drafts,vocab,bonus", [(1, 36, 12_291, False), (1, 36, 12_291, True), (3, 70, 4_097, True),
+                                                      (9, 2, 65_505, False)])
+def test_sampled_full_vocabulary_odd_rows(orc, dev, rng, lanes, drafts, vocab, bonus):
+    """Odd vocabularies (rows off a 16-byte boundary, a last range of one token),
+    more than 64 positions, tied logits at the cuts, and the row counts at which
+    fewer rows are cut into more parts."""
+    import voidinfer_amd as vi
+    tr = drafts + int(bonus)
+    x = rng.standard_normal((lanes * tr, vocab)).astype(np.float32) * 2.0
+    y = x[np.arange(lanes * tr).reshape(lanes, tr)[:, :drafts].reshape(-1)]
+    y = y + rng.standard_normal(y.shape).astype(np.float32) * 0.3
+    tb, db = W_bf16(x), W_f16(y)
+    tb[::2] &= 0xFFE0
+    db[1::2] &= 0xFF00
+    p = vi.params_array(lanes, seed=rng.integers(1, 2**62, lanes), position=rng.integers(0, 10**5, lanes),
+                        lane=np.arange(lanes), temperature=0.8, top_k=rng.choice([0, 300], lanes),
+                        top_p=rng.choice([0.8, 1.0], lanes))
+    drafted = np.zeros((lanes, drafts), dtype=np.int32)
+    for l in range(lanes):
+        for j in range(drafts):
+            prob, _ = orc.row_distribution(db[l * drafts + j], 1, p[l])
+            drafted[l, j] = rng.choice(vocab, p=prob / prob.sum())
+    g, w = run(orc, dev, 1, tb, db, drafted, p, lanes, drafts)
+    exempt = {l for l in range(lanes) if np.min(w[4][l]) < 1e-6}
+    assert len(assert_same(g, w, exempt)) <= 1

@@ -53,6 +53,37 @@ __global__ __launch_bounds__(256) void probe_copy_kernel(uint4* dst, const uint4
 
 }  // namespace
 
+SideStream* side_stream() {
+    // (one per host thread and device: concurrent callers never share events)
+    thread_local SideStream side[64];
+    thread_local bool tried[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+    SideStream& x = side[dev];
+    if (!tried[dev]) {
+        tried[dev] = true;
+        if (hipStreamCreateWithFlags(&x.stream, hipStreamNonBlocking) != hipSuccess ||
+            hipEventCreateWithFlags(&x.fork, hipEventDisableTiming) != hipSuccess ||
+            hipEventCreateWithFlags(&x.join, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            x.stream = nullptr;
+        }
+    }
+    return x.stream ? &x : nullptr;
+}
+
+int device_cus() {
+    static int cached[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    if (!cached[dev]) {
+        int n = 0;
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cached[dev] = n;
+    }
+    return cached[dev];
+}
+
 vi_status launch_presence_reset(int32_t* table, int vocabulary, hipStream_t stream) {
     hipLaunchKernelGGL(presence_fill_kernel, dim3((vocabulary + 255) / 256), dim3(256), 0, stream, table, vocabulary);
     return launch_status();

@@ -1,10 +1,13 @@
 // sample_stream.hip — full-vocabulary rows of the batched sampler, 16-bit
 // logits (temperature > 0, top_k = 0 or > 64): penalties, temperature, top-k /
 // min-p / top-p over the whole vocabulary and the Philox inverse-CDF draw.
-// Serves rows whose logits are 16-byte aligned, whose vocabulary is a multiple
-// of 8, and whose caller wants tokens (uniforms, stats, recording into penalty
-// states) but no probabilities or bounds; the slice / merge kernels
-// (sample_slices.hip) serve every other 16-bit row.
+// Every 16-bit full-vocabulary row comes here, at any row alignment: the sampler's
+// (tokens, uniforms, stats, recording into penalty states, on request the
+// filtered distribution) and verification's (the distributions' bounds).
+// (Rows with an odd vocabulary, probabilities or bounds had kernels of their own,
+// which named the support's end by ranks: verification of 8 lanes x 16 drafts over
+// 248,320 tokens, bf16 and fp16, takes 134 us this way and 232 that way;
+// 56 x 66,181 bf16 26 and 54.)
 //
 // Key fact: bf16 / fp16 logits, and penalized logits stored back in the same
 // dtype, take one of 65,536 bit patterns, and z = x' * (1/T) is a strictly
@@ -39,7 +42,12 @@
 // resolved inside its block; the part holding the drawn key's rank is read
 // again to name the token (id order among equal keys), a history token's
 // penalized key recognised from its raw key through the preimage of the drawn
-// key under the (monotone) penalty.
+// key under the (monotone) penalty.  A caller that wants the filtered distribution
+// gets the support's end as a key and the last id of that key inside, named the
+// same way (a support is then a comparison per logit, with no ranks to count).
+//
+// Probabilities (probs_kernel, then repeat_probs_kernel for the tokens seen more
+// than once): every logit's penalized key compared with the support's end.
 //
 // Roofline: HBM; V x 2 bytes of logits per row, plus the presence bitmap
 // (V / 8 bytes) and the repeat list where the row has penalties.
@@ -64,6 +72,7 @@ constexpr int kDepth = 4;                // rounds of logits in flight per threa
 constexpr int kXcds = 8;
 constexpr int kRepPF = 2;                // repeat-list entries prefetched per thread
 constexpr int kMaxParts = 16;            // parts per row
+constexpr int kMaxVocabulary = 524288;   // (every full-vocabulary route's limit)
 constexpr int kMaxPartLen = 65504;       // tokens per part (a multiple of 32 below 65,536)
 constexpr int kPub = 64;                 // words per part header: the occupancy bitmaps, by sign
 // Place of group g in an occupancy bitmap of 32 words: byte g & 127, bit g >> 7
@@ -117,7 +126,12 @@ struct StreamArgs {
     int record;
     int32_t* tokens;
     double* uniforms;
+    float* probs;
+    int64_t probs_stride;
     vi_sample_stats* stats;
+    FullBound* bounds;         // [rows] (or null): the rows' filtered distributions
+    int draw_every;            // rows whose token is drawn: every one (1), every n-th (row % n == n - 1), none (0)
+    int row0;                  // row 0's number in the call (a call of very many rows takes several launches)
     // the parts' tables: header (occupied-group bitmap, highest valid key) and
     // the occupied groups' 32 words at their place
     uint32_t* ppub;            // [rows * parts][kPub]
@@ -201,8 +215,8 @@ __device__ __forceinline__ Item part_geo(const StreamArgs& a, int row, int part)
     it.part = part;
     it.s0 = part * a.part_len;
     it.n = min(a.part_len, a.vocabulary - it.s0);
-    it.nvec = it.n >> 3;
-    it.rounds = (it.nvec + kT - 1) / kT;
+    it.nvec = it.n >> 3;   // (up to seven logits past the last vector)
+    it.rounds = max(1, (it.nvec + kT - 1) / kT);
     return it;
 }
 // Parts of XCD x (the rows x, x + 8, ... when the launch is XCD-aware, else
@@ -347,6 +361,7 @@ __global__ __launch_bounds__(kT) void stream_kernel(StreamArgs a) {
         const int q = __builtin_amdgcn_readfirstlane(sh.items[k]);
         c.it = item_at(a, x, q);
         c.vb = static_cast<const unsigned char*>(a.logits) + 2 * (size_t(c.it.row) * size_t(a.stride) + size_t(c.it.s0));
+        if (c.it.nvec == 0) c.vb = reinterpret_cast<const unsigned char*>(a.params);   // (no whole vector: read, never used)
         c.pb = presence_at(a, c.it.row, c.it.s0, c.vb);
         int z = 0;
         asm volatile("" : "+v"(z));
@@ -415,7 +430,7 @@ __global__ __launch_bounds__(kT) void stream_kernel(StreamArgs a) {
         const unsigned char* pb = in_nxt ? nxt.pb : cur.pb;
         const int nv = in_nxt ? nxt.it.nvec : cur.it.nvec;
         const int rr = in_nxt ? rel - Rp : rel;
-        const int v = min(rr * kT + opaque_tid(), nv - 1);
+        const int v = max(min(rr * kT + opaque_tid(), nv - 1), 0);
         dv = load16(vb + size_t(v) * 16);
         // the dword holding the vector's presence byte (a 32-bit load result
         // stays in its register across the loop; a byte would be re-extended)
@@ -512,6 +527,14 @@ __global__ __launch_bounds__(kT) void stream_kernel(StreamArgs a) {
             }
         }
 
+        if (it.n & 7) {   // (uniform: the last part of an odd vocabulary) the logits past the last vector
+            if (tid < (it.n & 7)) {
+                const int off = 8 * it.nvec + tid;
+                const uint32_t raw = uint32_t(row16[it.s0 + off]);
+                const bool present = pen && ((uint32_t(cur.pb[it.nvec]) >> tid) & 1u);
+                hist_inc(H, present ? pen_pattern<DT>(raw, 1u, p, inv_r, rep_fast) : raw);
+            }
+        }
         lds_barrier();
         if (pen && cur.nrep > uint32_t(kRepPF * kT)) {   // (long repeat lists: the rest of the entries)
             for (uint32_t i = uint32_t(kRepPF * kT + tid); i < cur.nrep; i += kT) {
@@ -575,9 +598,12 @@ struct MergeShared {
     uint64_t wmass[kW];
     uint32_t nslots, total_cnt, z0key, owner, orank, flags, kmin, kmax;
     uint64_t total_mass;
-    uint32_t draw_key, draw_rank;
+    // the ranks to name: [0] the last end-key logit inside the support (when the
+    // support cuts its key's logits), [1] the draw
+    uint32_t want[2], key[2], rank[2];
+    int32_t id[2];
+    uint32_t end_key;
     uint32_t n_support, ok, lo1, hi1, nflip;
-    int32_t token;
     double s_n, u;
 };
 
@@ -664,7 +690,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         if (lane == 0) { sh.kmin = km & 0xffffu; sh.kmax = km >> 16; }
     }
     for (int i = tid; i < 2048; i += kT) { bcnt[i] = 0u; bmass[i] = 0ull; }
-    if (tid == 0) { sh.flags = pv.flags; sh.token = -1; sh.ok = 1u; sh.z0key = 0u; }
+    if (tid == 0) { sh.flags = pv.flags; sh.ok = 1u; sh.z0key = 0u; }
     lds_barrier();
     if (tid < P * 32) {
         atomicOr(&occ[tid % 32], pub[0] | pub[1]);
@@ -904,6 +930,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
                 st.flags = out_flags | (fail ? VI_FLAG_ERROR : VI_FLAG_EMPTY);
                 a.stats[row] = st;
             }
+            if (a.bounds) a.bounds[row] = FullBound{0.0, 0.0, 0.0f, 0u, 0, 0u};
         }
         return;
     }
@@ -1045,15 +1072,16 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         uint64_t sm = Mtot;
         uint32_t sc = N;
         if (!all) mass_through(ek, et, &sm, &sc);
+        const bool draw = a.draw_every > 0 && (a.row0 + row) % a.draw_every == a.draw_every - 1;
         const double u = philox_uniform(p.seed, p.lane, p.position, 0u);
         const double target_d = u * double(sm);
         // the draw: the first support logit whose inclusive mass exceeds u * S_n
         const uint64_t t = uint64_t(target_d);
-        int b = block_search(2, t);
+        int b = draw ? block_search(2, t) : -1;
         const int lowest = all ? 0 : int(ek >> 5);
         if (b < lowest) b = -1;
         uint32_t dk = 0u, dr = 0u;
-        bool ok = false;
+        bool ok = !draw;
         if (b >= 0) {
             const bool in_end = !all && uint32_t(b) == (ek >> 5);
             const Fine f = fine_find(uint32_t(b), 2, t - mab[b], in_end ? ek : 0u, in_end ? et : kTakeAll);
@@ -1077,221 +1105,257 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
                 }
             }
         }
+        // does the support cut its last key's logits?
+        bool cuts = false;
+        if (a.bounds && !all && et != kTakeAll) {
+            const uint32_t c = block_key_count(ek >> 5);
+            cuts = et < readlane_u(c, 31 - int(ek & 31u));
+        }
         if (lane == 0) {
             sh.s_n = double(sm);
             sh.n_support = sc;
             sh.u = u;
-            sh.draw_key = dk;
-            sh.draw_rank = dr;
+            sh.end_key = all ? 0u : ek;
+            sh.want[0] = cuts ? 1u : 0u;
+            sh.key[0] = ek;
+            sh.rank[0] = et - 1u;
+            sh.id[0] = 0x7fffffff;
+            sh.want[1] = draw ? 1u : 0u;
+            sh.key[1] = dk;
+            sh.rank[1] = dr;
+            sh.id[1] = -1;
             sh.ok = ok ? 1u : 0u;
         }
     }
     lds_barrier();
 
-    // ---- 5. the part holding the drawn rank (parts in id order) and, for the
-    // rescan, the drawn key's preimage under the count-1 penalty: a history
-    // token counted once has the drawn key exactly when its raw key lies in
-    // [lo1, hi1) (the penalty is monotone in the logit)
+    // ---- 5. the part holding the rank to name (parts in id order) and, for the
+    // rescan, the key's preimage under the count-1 penalty: a history token
+    // counted once has the key exactly when its raw key lies in [lo1, hi1) (the
+    // penalty is monotone in the logit)
     const float inv_r = rep_inverse(p);
     const bool rep_fast = rep_fast_ok(p);
-    if (wave == 0 && sh.ok) {
-        const uint32_t dk = sh.draw_key;
-        const KeyLoc kl = key_loc(dk);
-        const GroupBit gb = group_bit(kl.group);
-        uint32_t c = 0u;
-        if (lane < P && ((pbits[lane * 32 + gb.word] >> gb.shift) & 1u)) {
-            const uint64_t* src = reinterpret_cast<const uint64_t*>(a.pwords) + ((pi0 + lane) * kGroups + kl.group) * 16;
-            const uint64_t w2 = src[kl.word >> 1];
-            const uint32_t wd = (kl.word & 1u) ? uint32_t(w2 >> 32) : uint32_t(w2);
-            c = kl.hi ? (wd >> 16) : (wd & 0xffffu);
-            if (dk == 0x8000u) c = (wd & 0xffffu) + (wd >> 16);   // +0 and -0
-        }
-        const uint32_t incl = wave_incl_scan_u32(c);
-        const uint64_t hm = ballot(lane < P && incl > sh.draw_rank);
-        if (hm) {
-            const int L = __builtin_ctzll(hm);
-            if (lane == L) { sh.owner = uint32_t(L); sh.orank = sh.draw_rank - (incl - c); }
-        } else if (lane == 0) {
-            sh.ok = 0u;
-        }
-    }
-    if (wave == 1 && pv.pen && sh.ok) {
-        constexpr int kNegMin = DT == VI_BF16 ? 0x0080 : 0x0400;
-        constexpr int kPosMax = DT == VI_BF16 ? 0xff7f : 0xfbff;
-        const uint32_t dk = sh.draw_key;
-        auto fk = [&](int k) { return key16(pen_pattern<DT>(unkey16(uint32_t(k)), 1u, p, inv_r, rep_fast)); };
-        const uint32_t lo = uint32_t(wave_search(kNegMin, kPosMax + 1, [&](int k) { return fk(k) >= dk; }));
-        const uint32_t hi = uint32_t(wave_search(kNegMin, kPosMax + 1, [&](int k) { return fk(k) > dk; }));
-        if (lane == 0) { sh.lo1 = lo; sh.hi1 = hi; }
-    }
-    for (int i = tid; i < 2048; i += kT) flip[i] = 0u;
-    if (tid == 0) sh.nflip = 0u;
-    // presence masks by byte for the rescan, in the decisions' running-sum
-    // table (free now): entry b, word q: the halves of tokens 2q and 2q + 1 all
-    // ones where that token is in the history
-    {
-        const uint32_t b = uint32_t(tid) >> 2, q = uint32_t(tid) & 3u;
-        reinterpret_cast<uint32_t*>(lds + kOffMCab)[tid] = (((b >> (2u * q)) & 1u) ? 0x0000ffffu : 0u) |
-                                                          (((b >> (2u * q + 1u)) & 1u) ? 0xffff0000u : 0u);
-    }
-    static_assert(256 * 16 <= kOffMMab - kOffMCab && kT == 1024, "presence masks");
-    lds_barrier();
-
-    // ---- 6. the owner part read again: its orank-th logit (id order) whose
-    // penalized key is the drawn key.  Repeated tokens whose count changes the
-    // answer are flipped.
-    if (sh.ok) {
-        const Item it = part_geo(a, row, int(sh.owner));
-        const uint32_t dk = sh.draw_key;
-        const bool pen = pv.pen;
-        const unsigned char* vb = static_cast<const unsigned char*>(a.logits) +
-                                  2 * (size_t(row) * size_t(a.stride) + size_t(it.s0));
-        const unsigned char* pb = pen ? pv.b1 + (it.s0 >> 3) : nullptr;
-        static_assert(kMaxPartLen / 8 <= 8 * kT, "a part is at most 8 rounds");
-        // the part's logits and presence bytes, eight rounds of 1024 vectors,
-        // all requested before the flips are worked out
-        auto load_vec = [&](int v, uint4* d, uint32_t* b) {
-            const int vc = min(v, it.nvec - 1);
-            *d = load16_cached(vb + size_t(vc) * 16);
-            *b = pb ? uint32_t(pb[vc]) : 0u;
-        };
-        uint4 vv[8];
-        uint32_t bb[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) load_vec(k * kT + tid, &vv[k], &bb[k]);
-        // the owner part's repeat entries' logits, requested behind the part
-        // (their flips are worked out after the count, which they correct)
-        auto in_owner = [&](uint2 e) { return e.y >= 2u && int(e.x) >= it.s0 && int(e.x) < it.s0 + it.n; };
-        uint32_t raw[2] = {0u, 0u};
-        if (pen) {
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if (uint32_t(j * kT + tid) >= pv.nrep) rep[j].y = 0u;
-                if (in_owner(rep[j])) raw[j] = uint32_t(row16[rep[j].x]);
-            }
-        }
-        const uint4* pmask = reinterpret_cast<const uint4*>(lds + kOffMCab);
-        // In the halves' key space (-0 just below +0): an absent token matches
-        // when its key lies in [a0, a0 + w0] (the drawn key, with -0 for +0), a
-        // history token when it lies in [a1, a1 + w1] (the preimage; none when
-        // empty).
-        const uint32_t a0 = dk == 0x8000u ? 0x7fffu : dk, w0 = dk == 0x8000u ? 1u : 0u;
-        uint32_t a1 = 0u, w1 = 0u;
-        bool empty1 = true;
-        if (pen && sh.hi1 > sh.lo1) {
-            uint32_t lo = sh.lo1, hi = sh.hi1 - 1u;
-            if (lo <= 0x8000u && hi >= 0x8000u) lo = min(lo, 0x7fffu);
-            a1 = lo; w1 = hi - lo; empty1 = false;
-        }
-        const uint32_t A0 = a0 | (a0 << 16), W0 = w0 | (w0 << 16), A1 = a1 | (a1 << 16), W1 = w1 | (w1 << 16);
-        const uint32_t force = empty1 ? 0xffffffffu : 0u;   // history halves never match
-        // Matches per round before the flips, three rounds to a word in 10-bit
-        // fields (a wave's sums stay below 1024): per half, the range of the
-        // token's kind is selected by the presence mask and tested as
-        // max(key - base - width, 0) == 0.
-        uint32_t pc[3] = {0u, 0u, 0u};
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int v = r * kT + tid;
+#pragma unroll 1
+    for (int which = 0; which < 2; ++which) {
+        if (!sh.want[which]) continue;   // (uniform)
+        lds_barrier();   // (the rank named before: its scratch is free)
+        const uint32_t dk = sh.key[which];
+        if (wave == 0 && sh.ok) {
+            const KeyLoc kl = key_loc(dk);
+            const GroupBit gb = group_bit(kl.group);
             uint32_t c = 0u;
-            if (v < it.nvec) {
-                const uint4 M = pmask[bb[r]];
-                const uint32_t w4[4] = {vv[r].x, vv[r].y, vv[r].z, vv[r].w};
-                const uint32_t m4[4] = {M.x, M.y, M.z, M.w};
-                uint32_t miss = 0u;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t base = (m4[q] & A1) | (~m4[q] & A0), width = (m4[q] & W1) | (~m4[q] & W0);
-                    const uint32_t t = pk_sub_u16(halves_key(w4[q]), base);
-                    miss += pk_nonzero_u16(pk_sub_sat_u16(t, width) | (m4[q] & force));
-                }
-                c = 8u - (miss & 0xffffu) - (miss >> 16);
+            if (lane < P && ((pbits[lane * 32 + gb.word] >> gb.shift) & 1u)) {
+                const uint64_t* src = reinterpret_cast<const uint64_t*>(a.pwords) + ((pi0 + lane) * kGroups + kl.group) * 16;
+                const uint64_t w2 = src[kl.word >> 1];
+                const uint32_t wd = (kl.word & 1u) ? uint32_t(w2 >> 32) : uint32_t(w2);
+                c = kl.hi ? (wd >> 16) : (wd & 0xffffu);
+                if (dk == 0x8000u) c = (wd & 0xffffu) + (wd >> 16);   // +0 and -0
             }
-            pc[r / 3] += c << (10 * (r % 3));
-        }
-        auto field = [](uint32_t w, int r) { return (w >> (10 * (r % 3))) & 0x3ffu; };
-        // Repeated tokens whose count changes the answer are flipped
-        if (pen) {
-            auto flip_if = [&](uint2 e, uint32_t rw) {
-                if (!in_owner(e) || !Elem<DT>::finite_bits(rw)) return;
-                const bool m1 = key16(pen_pattern<DT>(rw, 1u, p, inv_r, rep_fast)) == dk;
-                const bool mc = key16(pen_pattern<DT>(rw, e.y, p, inv_r, rep_fast)) == dk;
-                if (m1 != mc) {
-                    const uint32_t off = e.x - uint32_t(it.s0);
-                    atomicOr(&flip[off >> 5], 1u << (off & 31u));
-                    atomicAdd(&sh.nflip, 1u);
-                }
-            };
-#pragma unroll
-            for (int j = 0; j < 2; ++j) flip_if(rep[j], raw[j]);
-            for (uint32_t i = uint32_t(2 * kT + tid); i < pv.nrep; i += kT) {   // (long repeat lists)
-                const uint2 e = pv.list[i];
-                if (in_owner(e)) flip_if(e, uint32_t(row16[e.x]));
+            const uint32_t incl = wave_incl_scan_u32(c);
+            const uint32_t rank = sh.rank[which];
+            const uint64_t hm = ballot(lane < P && incl > rank);
+            if (hm) {
+                const int L = __builtin_ctzll(hm);
+                if (lane == L) { sh.owner = uint32_t(L); sh.orank = rank - (incl - c); }
+            } else if (lane == 0) {
+                sh.ok = 0u;
             }
         }
+        if (wave == 1 && pv.pen && sh.ok) {
+            constexpr int kNegMin = DT == VI_BF16 ? 0x0080 : 0x0400;
+            constexpr int kPosMax = DT == VI_BF16 ? 0xff7f : 0xfbff;
+            auto fk = [&](int k) { return key16(pen_pattern<DT>(unkey16(uint32_t(k)), 1u, p, inv_r, rep_fast)); };
+            const uint32_t lo = uint32_t(wave_search(kNegMin, kPosMax + 1, [&](int k) { return fk(k) >= dk; }));
+            const uint32_t hi = uint32_t(wave_search(kNegMin, kPosMax + 1, [&](int k) { return fk(k) > dk; }));
+            if (lane == 0) { sh.lo1 = lo; sh.hi1 = hi; }
+        }
+        for (int i = tid; i < 2048; i += kT) flip[i] = 0u;
+        if (tid == 0) sh.nflip = 0u;
+        // presence masks by byte for the rescan, in the decisions' running-sum
+        // table (free now): entry b, word q: the halves of tokens 2q and 2q + 1 all
+        // ones where that token is in the history
+        {
+            const uint32_t b = uint32_t(tid) >> 2, q = uint32_t(tid) & 3u;
+            reinterpret_cast<uint32_t*>(lds + kOffMCab)[tid] = (((b >> (2u * q)) & 1u) ? 0x0000ffffu : 0u) |
+                                                              (((b >> (2u * q + 1u)) & 1u) ? 0xffff0000u : 0u);
+        }
+        static_assert(256 * 16 <= kOffMMab - kOffMCab && kT == 1024, "presence masks");
         lds_barrier();
-        const bool flips = sh.nflip != 0u;
-        // exact match bits of one vector (the scalar form of the count, flips applied)
-        auto match_bits = [&](uint4 d, uint32_t b, int v) -> uint32_t {
-            const uint32_t w4[4] = {d.x, d.y, d.z, d.w};
-            uint32_t m = 0u;
+
+        // ---- 6. the owner part read again: its orank-th logit (id order) whose
+        // penalized key is the drawn key.  Repeated tokens whose count changes the
+        // answer are flipped.
+        if (sh.ok) {
+            const Item it = part_geo(a, row, int(sh.owner));
+            const bool pen = pv.pen;
+            const unsigned char* vb = static_cast<const unsigned char*>(a.logits) +
+                                      2 * (size_t(row) * size_t(a.stride) + size_t(it.s0));
+            const unsigned char* pb = pen ? pv.b1 + (it.s0 >> 3) : nullptr;
+            static_assert(kMaxPartLen / 8 <= 8 * kT, "a part is at most 8 rounds");
+            // the part's logits and presence bytes, eight rounds of 1024 vectors,
+            // all requested before the flips are worked out
+            auto load_vec = [&](int v, uint4* d, uint32_t* b) {
+                const int vc = max(min(v, it.nvec - 1), 0);
+                *d = load16_cached((it.nvec > 0 ? vb : reinterpret_cast<const unsigned char*>(a.params)) + size_t(vc) * 16);
+                *b = pb ? uint32_t(pb[vc]) : 0u;
+            };
+            uint4 vv[8];
+            uint32_t bb[8];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t pat = (j & 1) ? (w4[j >> 1] >> 16) : (w4[j >> 1] & 0xffffu);
-                const uint32_t k = (pat & 0x8000u) ? (~pat & 0xffffu) : (pat | 0x8000u);
-                const bool present = (b >> j) & 1u;
-                const bool hit = present ? (!empty1 && k - a1 <= w1) : (k - a0 <= w0);
-                m |= hit ? (1u << j) : 0u;
+            for (int k = 0; k < 8; ++k) load_vec(k * kT + tid, &vv[k], &bb[k]);
+            // the owner part's repeat entries' logits, requested behind the part
+            // (their flips are worked out after the count, which they correct)
+            auto in_owner = [&](uint2 e) { return e.y >= 2u && int(e.x) >= it.s0 && int(e.x) < it.s0 + it.n; };
+            uint32_t raw[2] = {0u, 0u};
+            if (pen) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (uint32_t(j * kT + tid) >= pv.nrep) rep[j].y = 0u;
+                    if (in_owner(rep[j])) raw[j] = uint32_t(row16[rep[j].x]);
+                }
             }
-            if (flips) m ^= (flip[v >> 2] >> ((v & 3) * 8)) & 0xffu;
-            return m;
-        };
-        if (flips) {   // (uniform) the flipped vectors counted again
+            const uint4* pmask = reinterpret_cast<const uint4*>(lds + kOffMCab);
+            // In the halves' key space (-0 just below +0): an absent token matches
+            // when its key lies in [a0, a0 + w0] (the drawn key, with -0 for +0), a
+            // history token when it lies in [a1, a1 + w1] (the preimage; none when
+            // empty).
+            const uint32_t a0 = dk == 0x8000u ? 0x7fffu : dk, w0 = dk == 0x8000u ? 1u : 0u;
+            uint32_t a1 = 0u, w1 = 0u;
+            bool empty1 = true;
+            if (pen && sh.hi1 > sh.lo1) {
+                uint32_t lo = sh.lo1, hi = sh.hi1 - 1u;
+                if (lo <= 0x8000u && hi >= 0x8000u) lo = min(lo, 0x7fffu);
+                a1 = lo; w1 = hi - lo; empty1 = false;
+            }
+            const uint32_t A0 = a0 | (a0 << 16), W0 = w0 | (w0 << 16), A1 = a1 | (a1 << 16), W1 = w1 | (w1 << 16);
+            const uint32_t force = empty1 ? 0xffffffffu : 0u;   // history halves never match
+            // Matches per round before the flips, three rounds to a word in 10-bit
+            // fields (a wave's sums stay below 1024): per half, the range of the
+            // token's kind is selected by the presence mask and tested as
+            // max(key - base - width, 0) == 0.
+            uint32_t pc[3] = {0u, 0u, 0u};
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 const int v = r * kT + tid;
-                if (v < it.nvec && ((flip[v >> 2] >> ((v & 3) * 8)) & 0xffu)) {
-                    const uint32_t c = uint32_t(__builtin_popcount(match_bits(vv[r], bb[r], v)));
-                    pc[r / 3] += (c - field(pc[r / 3], r)) << (10 * (r % 3));
+                uint32_t c = 0u;
+                if (v < it.nvec) {
+                    const uint4 M = pmask[bb[r]];
+                    const uint32_t w4[4] = {vv[r].x, vv[r].y, vv[r].z, vv[r].w};
+                    const uint32_t m4[4] = {M.x, M.y, M.z, M.w};
+                    uint32_t miss = 0u;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint32_t base = (m4[q] & A1) | (~m4[q] & A0), width = (m4[q] & W1) | (~m4[q] & W0);
+                        const uint32_t t = pk_sub_u16(halves_key(w4[q]), base);
+                        miss += pk_nonzero_u16(pk_sub_sat_u16(t, width) | (m4[q] & force));
+                    }
+                    c = 8u - (miss & 0xffffu) - (miss >> 16);
+                }
+                pc[r / 3] += c << (10 * (r % 3));
+            }
+            auto field = [](uint32_t w, int r) { return (w >> (10 * (r % 3))) & 0x3ffu; };
+            // Repeated tokens whose count changes the answer are flipped
+            if (pen) {
+                auto flip_if = [&](uint2 e, uint32_t rw) {
+                    if (!in_owner(e) || !Elem<DT>::finite_bits(rw)) return;
+                    const bool m1 = key16(pen_pattern<DT>(rw, 1u, p, inv_r, rep_fast)) == dk;
+                    const bool mc = key16(pen_pattern<DT>(rw, e.y, p, inv_r, rep_fast)) == dk;
+                    if (m1 != mc) {
+                        const uint32_t off = e.x - uint32_t(it.s0);
+                        atomicOr(&flip[off >> 5], 1u << (off & 31u));
+                        atomicAdd(&sh.nflip, 1u);
+                    }
+                };
+#pragma unroll
+                for (int j = 0; j < 2; ++j) flip_if(rep[j], raw[j]);
+                for (uint32_t i = uint32_t(2 * kT + tid); i < pv.nrep; i += kT) {   // (long repeat lists)
+                    const uint2 e = pv.list[i];
+                    if (in_owner(e)) flip_if(e, uint32_t(row16[e.x]));
                 }
             }
-        }
-        uint32_t pin[3];
+            lds_barrier();
+            const bool flips = sh.nflip != 0u;
+            // exact match bits of one vector (the scalar form of the count, flips applied)
+            auto match_bits = [&](uint4 d, uint32_t b, int v) -> uint32_t {
+                const uint32_t w4[4] = {d.x, d.y, d.z, d.w};
+                uint32_t m = 0u;
 #pragma unroll
-        for (int i = 0; i < 3; ++i) pin[i] = wave_incl_scan_u32(pc[i]);
-        if (lane == kWave - 1) {
+                for (int j = 0; j < 8; ++j) {
+                    const uint32_t pat = (j & 1) ? (w4[j >> 1] >> 16) : (w4[j >> 1] & 0xffffu);
+                    const uint32_t k = (pat & 0x8000u) ? (~pat & 0xffffu) : (pat | 0x8000u);
+                    const bool present = (b >> j) & 1u;
+                    const bool hit = present ? (!empty1 && k - a1 <= w1) : (k - a0 <= w0);
+                    m |= hit ? (1u << j) : 0u;
+                }
+                if (flips && v >= 0) m ^= (flip[v >> 2] >> ((v & 3) * 8)) & 0xffu;
+                return m;
+            };
+            if (flips) {   // (uniform) the flipped vectors counted again
 #pragma unroll
-            for (int r = 0; r < 8; ++r) sh.wtot[r][wave] = field(pin[r / 3], r);
-        }
-        lds_barrier();
-        // exclusive offsets of the (round, wave) blocks in id order (wave 0:
-        // lane l holds blocks 2l and 2l + 1 of the 128)
-        if (wave == 0) {
-            const uint32_t b0 = sh.wtot[(2 * lane) >> 4][(2 * lane) & 15], b1 = sh.wtot[(2 * lane + 1) >> 4][(2 * lane + 1) & 15];
-            const uint32_t incl = wave_incl_scan_u32(b0 + b1);
-            sh.wtot[(2 * lane) >> 4][(2 * lane) & 15] = incl - b0 - b1;
-            sh.wtot[(2 * lane + 1) >> 4][(2 * lane + 1) & 15] = incl - b1;
-        }
-        lds_barrier();
-        const uint32_t want = sh.orank;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const uint32_t c = field(pc[r / 3], r);
-            const uint32_t e = sh.wtot[r][wave] + field(pin[r / 3], r) - c;
-            if (c && want >= e && want < e + c) {
-                const int v = r * kT + tid;
-                uint32_t m = match_bits(vv[r], bb[r], v);
-                for (uint32_t k = want - e; k > 0u; --k) m &= m - 1u;
-                sh.token = it.s0 + 8 * v + __builtin_ctz(m);
+                for (int r = 0; r < 8; ++r) {
+                    const int v = r * kT + tid;
+                    if (v < it.nvec && ((flip[v >> 2] >> ((v & 3) * 8)) & 0xffu)) {
+                        const uint32_t c = uint32_t(__builtin_popcount(match_bits(vv[r], bb[r], v)));
+                        pc[r / 3] += (c - field(pc[r / 3], r)) << (10 * (r % 3));
+                    }
+                }
             }
+            uint32_t pin[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) pin[i] = wave_incl_scan_u32(pc[i]);
+            if (lane == kWave - 1) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) sh.wtot[r][wave] = field(pin[r / 3], r);
+            }
+            lds_barrier();
+            // exclusive offsets of the (round, wave) blocks in id order (wave 0:
+            // lane l holds blocks 2l and 2l + 1 of the 128)
+            if (wave == 0) {
+                const uint32_t b0 = sh.wtot[(2 * lane) >> 4][(2 * lane) & 15], b1 = sh.wtot[(2 * lane + 1) >> 4][(2 * lane + 1) & 15];
+                const uint32_t incl = wave_incl_scan_u32(b0 + b1);
+                sh.wtot[(2 * lane) >> 4][(2 * lane) & 15] = incl - b0 - b1;
+                sh.wtot[(2 * lane + 1) >> 4][(2 * lane + 1) & 15] = incl - b1;
+            }
+            lds_barrier();
+            const uint32_t want = sh.orank;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const uint32_t c = field(pc[r / 3], r);
+                const uint32_t e = sh.wtot[r][wave] + field(pin[r / 3], r) - c;
+                if (c && want >= e && want < e + c) {
+                    const int v = r * kT + tid;
+                    uint32_t m = match_bits(vv[r], bb[r], v);
+                    for (uint32_t k = want - e; k > 0u; --k) m &= m - 1u;
+                    sh.id[which] = it.s0 + 8 * v + __builtin_ctz(m);
+                }
+            }
+            if ((it.n & 7) && wave == kW - 1) {   // (uniform) the logits past the last vector: behind every vector
+                const uint32_t body = sh.wtot[7][kW - 1] + uint32_t(__builtin_amdgcn_readlane(int(field(pin[2], 7)), kWave - 1));
+                const bool in = lane < (it.n & 7);
+                const int off = 8 * it.nvec + min(lane, (it.n & 7) - 1);
+                const uint32_t tb = pb ? uint32_t(pb[it.nvec]) : 0u, raw = uint32_t(row16[it.s0 + off]);
+                const uint32_t one = match_bits(make_uint4(raw, 0u, 0u, 0u), (tb >> (off & 7)) & 1u, -1) & 1u;
+                const bool hit = in && (one ^ (flips ? (flip[off >> 5] >> (off & 31)) & 1u : 0u));
+                const uint64_t m = ballot(hit);
+                const uint32_t before = uint32_t(__builtin_popcountll(m & ((1ull << lane) - 1ull)));
+                if (hit && want == body + before) sh.id[which] = it.s0 + off;
+            }
+            lds_barrier();
         }
-        lds_barrier();
     }
 
     // ---- 7. outputs
     if (tid == 0) {
-        const int32_t tok = sh.token;
-        if (tok < 0) {   // the tables disagree with the logits: cannot happen for consistent inputs
+        const int32_t tok = sh.want[1] ? sh.id[1] : 0;
+        if (a.bounds)
+            a.bounds[row] = FullBound{z0, sh.s_n / kFix, inv_t, sh.end_key, sh.id[0], tok >= 0 ? 1u : 0u};
+        if (!sh.want[1]) {   // (no token of this row is wanted)
+            if (a.stats) {
+                vi_sample_stats st{};
+                st.flags = out_flags;
+                a.stats[row] = st;
+            }
+        } else if (tok < 0) {   // the tables disagree with the logits: cannot happen for consistent inputs
             a.tokens[row] = -1;
             if (a.uniforms) a.uniforms[row] = sh.u;
             if (a.stats) {
@@ -1311,7 +1375,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
                 st.uniform = sh.u;
                 a.stats[row] = st;
             }
-            if (a.record && a.pstate && tok < V) {
+            if (a.record && a.pstate && !a.probs && tok < V) {   // (with probabilities: repeat_probs_kernel)
                 const LaneState ls = lane_state(const_cast<unsigned char*>(a.pstate) + size_t(row) * a.pl.lane_bytes,
                                                 a.pl);
                 state_record_one(ls, a.pl, V, tok);
@@ -1325,6 +1389,8 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
 // stream reads from a penalty state: one workgroup per row; bitmaps of the
 // tokens seen once (B1) and more than once (B2) built with LDS atomics, then
 // each B2 token's rank (population count of B2 before it) indexes its count.
+// Rows whose bitmaps and counts exceed the LDS keep them in the workspace
+// (LDS = false: every access at agent scope).
 struct HistArgs {
     const int32_t* histories;
     const int64_t* offsets;
@@ -1333,23 +1399,35 @@ struct HistArgs {
     uint32_t* hb1;     // [rows][words]
     uint2* hlist;      // [rows][cap]
     uint32_t* hhead;   // [rows][2]
+    uint32_t* tmp;     // [rows][2 words + cap] (the workspace form)
 };
 constexpr int kHistBatch = 32;   // history tokens per thread held in registers
 
 constexpr int kHistLdsWords = 40896;   // B1 + B2 + counts (160 KB less the scalars)
 
+template <bool LDS>
 __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
-    __shared__ __attribute__((aligned(16))) uint32_t hl[kHistLdsWords];
+    __shared__ __attribute__((aligned(16))) uint32_t lds[LDS ? kHistLdsWords : 1];
     const int row = blockIdx.x, tid = threadIdx.x;
     const int W = h.words;
+    uint32_t* hl = LDS ? lds : h.tmp + size_t(row) * (2 * size_t(W) + size_t(h.cap));
     uint32_t* B1 = hl;              // then the prefix of B2 per word
     uint32_t* B2 = hl + W;
     uint32_t* cnt = hl + 2 * W;     // [cap]
+    auto get = [](const uint32_t* p) { return LDS ? *p : load_agent(p); };
+    auto put = [](uint32_t* p, uint32_t v) {
+        if (LDS) *p = v;
+        else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto sync = []() {
+        if (!LDS) __threadfence();
+        __syncthreads();
+    };
     __shared__ uint32_t flags, nrep, scan[kW + 1];
     const int64_t b = h.offsets[row], e = h.offsets[row + 1];
-    for (int i = tid; i < 2 * W; i += kT) hl[i] = 0u;
+    for (int i = tid; i < 2 * W; i += kT) put(&hl[i], 0u);
     if (tid == 0) flags = 0u;
-    __syncthreads();
+    sync();
     const int V = h.vocabulary;
     // The history in batches of kHistBatch tokens per thread (one batch for
     // up to 32,768 tokens, kept in registers for the second pass).  Each pass
@@ -1384,13 +1462,13 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
             }
         }
     }
-    __syncthreads();
+    sync();
     // B1 out; its LDS then holds the B2 rank of each word's first bit
     uint32_t* out = h.hb1 + size_t(row) * W;
-    for (int i = tid; i < W; i += kT) out[i] = B1[i];
+    for (int i = tid; i < W; i += kT) out[i] = get(&B1[i]);
     const int per = (W + kT - 1) / kT, w0 = tid * per, w1 = min(W, w0 + per);
     uint32_t own = 0u;
-    for (int i = w0; i < w1; ++i) own += uint32_t(__builtin_popcount(B2[i]));
+    for (int i = w0; i < w1; ++i) own += uint32_t(__builtin_popcount(get(&B2[i])));
     uint32_t total = 0u;
     const uint32_t ex = block_exclusive_scan_u32<kT>(own, scan, &total);   // (barriers: B1 read before)
     if (total > uint32_t(h.cap)) {   // cannot happen: the launcher sizes cap for the longest history
@@ -1399,10 +1477,10 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
     }
     {
         uint32_t r = ex;
-        for (int i = w0; i < w1; ++i) { B1[i] = r; r += uint32_t(__builtin_popcount(B2[i])); }
+        for (int i = w0; i < w1; ++i) { put(&B1[i], r); r += uint32_t(__builtin_popcount(get(&B2[i]))); }
     }
-    for (uint32_t i = tid; i < total; i += kT) cnt[i] = 0u;
-    __syncthreads();
+    for (uint32_t i = tid; i < total; i += kT) put(&cnt[i], 0u);
+    sync();
     for (int64_t base = b; base < e; base += int64_t(kHistBatch) * kT) {
         if (!one_batch) load(base);
 #pragma unroll
@@ -1412,8 +1490,8 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
             for (int j = 0; j < kHistBatch / 2; ++j) {
                 const int32_t tj = t[j0 + j];
                 const bool ok = tj >= 0 && tj < V;
-                wd[j] = ok ? B2[tj >> 5] : 0u;
-                r0[j] = ok ? B1[tj >> 5] : 0u;
+                wd[j] = ok ? get(&B2[tj >> 5]) : 0u;
+                r0[j] = ok ? get(&B1[tj >> 5]) : 0u;
             }
 #pragma unroll
             for (int j = 0; j < kHistBatch / 2; ++j) {
@@ -1422,23 +1500,127 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
             }
         }
     }
-    __syncthreads();
+    sync();
     uint2* lst = h.hlist + size_t(row) * h.cap;
     for (int i = w0; i < w1; ++i) {
-        uint32_t wd = B2[i], r = B1[i];
+        uint32_t wd = get(&B2[i]), r = get(&B1[i]);
         while (wd) {
             const int j = __builtin_ctz(wd);
             wd &= wd - 1u;
-            lst[r] = make_uint2(uint32_t(32 * i + j), cnt[r]);
+            lst[r] = make_uint2(uint32_t(32 * i + j), get(&cnt[r]));
             ++r;
         }
     }
     if (tid == 0) { h.hhead[2 * row] = total; h.hhead[2 * row + 1] = flags; }
 }
 
+// ------------------------------------------------------------ probabilities
+// The filtered distribution of each row: exp(z - z0) / S_n on the support, 0
+// elsewhere.  Bound by the memory: 2 bytes read and 4 written per logit.  Four
+// consecutive logits per lane and round (8-byte loads and 16-byte stores, whole
+// lines per wave), every round's loads requested first; a history token is
+// penalized with count 1, and the tokens seen more than once are written again
+// by repeat_probs_kernel.  (24 x 151,936 bf16: 16.4 us and 4.5 for the repeats;
+// 48.6 with eight logits per thread, each slice's penalties rebuilt in LDS and
+// end-key ranks counted.)
+constexpr int kPT = 256;                          // threads
+constexpr int kPRounds = 4;
+constexpr int kPChunk = kPT * kPRounds * 4;       // logits per workgroup
+
+// p of a logit with (penalized) pattern pat
+template <int DT>
+__device__ __forceinline__ float pattern_prob(uint32_t pat, int id, const FullBound& B, double inv_s) {
+    const uint32_t k = key16(pat);
+    const float z = Elem<DT>::decode(unkey16(k)) * B.inv_t;
+    const bool in = Elem<DT>::finite_bits(pat) && isfinite(z) && (k > B.end_key || (k == B.end_key && id <= B.end_id));
+    return in ? float(exp(double(z) - B.z0) * inv_s) : 0.0f;
+}
+
+template <int DT>
+__global__ __launch_bounds__(kPT) void probs_kernel(StreamArgs a) {
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
+    typedef float f32x4_t __attribute__((ext_vector_type(4)));
+    typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
+    const int row = blockIdx.y, V = a.vocabulary;
+    const vi_row_params p = a.params[row];
+    if (!stream_row(p)) return;
+    const FullBound B = a.bounds[row];
+    const PenView pv = pen_view(a, row, p);
+    const uint16_t* row16 = reinterpret_cast<const uint16_t*>(static_cast<const unsigned char*>(a.logits) +
+                                                              2 * size_t(row) * size_t(a.stride));
+    float* out = a.probs + size_t(row) * size_t(a.probs_stride);
+    const int i0 = int(blockIdx.x) * kPChunk + 4 * int(threadIdx.x);
+    u32x2_t v[kPRounds];
+    uint32_t b[kPRounds];
+#pragma unroll
+    for (int r = 0; r < kPRounds; ++r) {
+        const int i = i0 + r * 4 * kPT;
+        v[r] = u32x2_t{0u, 0u};
+        b[r] = 0u;
+        if (i + 4 <= V) v[r] = *reinterpret_cast<const u32x2_any_t*>(row16 + i);
+        if (pv.pen && i < V) b[r] = (uint32_t(pv.b1[i >> 3]) >> (i & 4)) & 0xfu;
+    }
+    const float inv_r = rep_inverse(p);
+    const bool rep_fast = rep_fast_ok(p);
+    const double inv_s = B.valid ? 1.0 / B.s_n : 0.0;
+    auto prob = [&](uint32_t raw, uint32_t present, int id) {
+        if (present) raw = pen_pattern<DT>(raw, 1u, p, inv_r, rep_fast);
+        return B.valid ? pattern_prob<DT>(raw, id, B, inv_s) : 0.0f;
+    };
+#pragma unroll
+    for (int r = 0; r < kPRounds; ++r) {
+        const int i = i0 + r * 4 * kPT;
+        if (i + 4 <= V) {
+            f32x4_t q;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                q[j] = prob((j & 1) ? v[r][j >> 1] >> 16 : v[r][j >> 1] & 0xffffu, (b[r] >> j) & 1u, i + j);
+            *reinterpret_cast<f32x4_any_t*>(out + i) = q;
+        } else {   // (up to three logits past the row's last four)
+            for (int j = i; j < V; ++j) out[j] = prob(uint32_t(row16[j]), (b[r] >> (j - i)) & 1u, j);
+        }
+    }
+}
+
+// The tokens seen more than once, with their counts (one workgroup per row,
+// after probs_kernel); then, with `record`, the row's token into its lane's
+// state: the distribution is the one before that occurrence.
+template <int DT>
+__global__ __launch_bounds__(kPT) void repeat_probs_kernel(StreamArgs a) {
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const vi_row_params p = a.params[row];
+    if (!stream_row(p)) return;
+    const FullBound B = a.bounds[row];
+    const PenView pv = pen_view(a, row, p);
+    const uint16_t* row16 = reinterpret_cast<const uint16_t*>(static_cast<const unsigned char*>(a.logits) +
+                                                              2 * size_t(row) * size_t(a.stride));
+    float* out = a.probs + size_t(row) * size_t(a.probs_stride);
+    if (pv.pen && B.valid) {   // (uniform)
+        const float inv_r = rep_inverse(p);
+        const bool rep_fast = rep_fast_ok(p);
+        const double inv_s = 1.0 / B.s_n;
+        for (uint32_t i = uint32_t(tid); i < pv.nrep; i += kPT) {
+            const uint2 e = pv.list[i];
+            if (e.y < 2u || e.x >= uint32_t(a.vocabulary)) continue;
+            out[e.x] = pattern_prob<DT>(pen_pattern<DT>(uint32_t(row16[e.x]), e.y, p, inv_r, rep_fast), int(e.x), B, inv_s);
+        }
+    }
+    if (a.record && a.pstate) {
+        __syncthreads();   // (the list has been read)
+        const int32_t tok = a.tokens[row];
+        if (tid == 0 && tok >= 0 && tok < a.vocabulary) {
+            const LaneState ls = lane_state(const_cast<unsigned char*>(a.pstate) + size_t(row) * a.pl.lane_bytes, a.pl);
+            state_record_one(ls, a.pl, a.vocabulary, tok);
+        }
+    }
+}
+
 }  // namespace
 
 // ------------------------------------------------------------------ host
+constexpr int kShortestPart = 12288;   // tokens of a bf16 part, unless the row has fewer (fp16: twice that)
+
 struct StreamPlan {
     int parts, part_len;
 };
@@ -1452,105 +1634,141 @@ static StreamPlan stream_plan(int rows, int vocabulary, int dtype) {
     // over a few dozen.  Stream + merge, us, with 16 / 8 / 4 parts: fp16 2 x
     // 162,880 8.8 + 43.2 / 10.5 + 34.1 / 12.8 + 30.6; bf16 8 x 248,320 9.5 + 19.8 /
     // 11.0 + 19.8 / 15.0 + 20.1; bf16 3 x 45,568 6.4 + 16.9 / 6.3 + 15.8 / 6.4 + 14.7.
-    const int shortest = dtype == VI_F16 ? 24576 : 12288;
+    const int shortest = dtype == VI_F16 ? 2 * kShortestPart : kShortestPart;
     parts = std::max(parts, std::min({kMaxParts, fill, vocabulary / shortest}));
     // a multiple of 32 tokens: every part's presence bytes start 4-byte aligned
     const int len = ((vocabulary + parts - 1) / parts + 31) / 32 * 32;
     return {(vocabulary + len - 1) / len, len};
 }
-static int hist_words(int vocabulary) { return (vocabulary + 31) / 32; }
-static int hist_cap(int64_t max_history) { return int(std::max<int64_t>(max_history / 2, 1)); }
-static bool hist_fits(int vocabulary, int64_t max_history) {
-    return max_history <= (int64_t(1) << 30) &&
-           2 * int64_t(hist_words(vocabulary)) + hist_cap(max_history) <= kHistLdsWords;
+// Most parts of a launch of up to `rows` rows (stream_plan's, whatever the count
+// of rows up to that: a workspace for more rows serves fewer).
+static size_t stream_parts_most(int rows, int vocabulary) {
+    const size_t r = size_t(rows), least = size_t(vocabulary + kMaxPartLen - 1) / kMaxPartLen;
+    const size_t split = std::min<size_t>(kMaxParts, size_t(vocabulary / kShortestPart));
+    return std::max(r * least, std::min(r * split, size_t(device_cus()) + r));
 }
 
-// The stream launch: workgroups, XCD-aware mapping, and the most parts one
-// workgroup takes (its XCD's parts shared out in turn).
+// The stream launch: workgroups and XCD-aware mapping.
 struct StreamGrid {
-    int grid, xcd, per_wg;
+    int grid, xcd;
 };
 static StreamGrid stream_grid(int rows, int parts) {
     StreamGrid g;
-    const int items = rows * parts;
-    g.grid = std::min(device_cus(), items);
+    g.grid = std::min(device_cus(), rows * parts);
     g.xcd = (rows >= kXcds && g.grid % kXcds == 0) ? 1 : 0;
-    const int xr = g.xcd ? (rows + kXcds - 1) / kXcds : rows, xw = g.xcd ? g.grid / kXcds : g.grid;
-    g.per_wg = (xr * parts + xw - 1) / xw;
     return g;
 }
 
-bool stream_supported(const SampleArgs& s) {
-    if (s.dtype != VI_BF16 && s.dtype != VI_F16) return false;
-    if (s.probs || s.full_out || s.rows <= 0) return false;
-    if (s.vocabulary <= 0 || s.vocabulary % 8 || s.vocabulary > kMaxParts * kMaxPartLen) return false;
-    if (s.stride < s.vocabulary || s.stride % 8 || reinterpret_cast<uintptr_t>(s.logits) % 16) return false;
-    if (int64_t(s.rows) * kMaxParts > (int64_t(1) << 30)) return false;
-    if (stream_grid(s.rows, stream_plan(s.rows, s.vocabulary, s.dtype).parts).per_wg > kMaxItems) return false;
-    const bool hist = !s.pstate && s.histories && s.offsets && s.max_history > 0;
-    if (hist && !hist_fits(s.vocabulary, s.max_history)) return false;
-    return true;
+static int hist_words(int vocabulary) { return (vocabulary + 31) / 32; }
+// tokens of a history that can be seen more than once
+static int hist_cap(int vocabulary, int64_t max_history) {
+    return int(std::max<int64_t>(std::min<int64_t>(max_history / 2, vocabulary), 1));
+}
+static bool hist_in_lds(int vocabulary, int64_t max_history) {
+    return 2 * hist_words(vocabulary) + hist_cap(vocabulary, max_history) <= kHistLdsWords;
+}
+
+// Rows per launch: as many as keep a workgroup's parts within kMaxItems and the
+// probabilities' grid within its limit (a multiple of 8: each XCD's rows the
+// same); more rows than that take several launches, over the same tables.
+static int stream_chunk(int rows, int parts) {
+    const int most = std::min((kMaxItems - 1) * device_cus() / parts, 32768) / kXcds * kXcds;
+    return std::min(rows, most);
+}
+
+bool stream_supported(int dtype, int vocabulary, int64_t stride) {
+    return (dtype == VI_BF16 || dtype == VI_F16) && vocabulary > 0 && vocabulary <= kMaxVocabulary && stride >= vocabulary;
 }
 
 size_t stream_workspace(int rows, int vocabulary, int64_t max_history) {
-    if (rows <= 0 || vocabulary <= 0 || vocabulary % 8 || vocabulary > kMaxParts * kMaxPartLen) return 0;
-    // (bf16 rows take the most parts)
-    const size_t np = size_t(rows) * stream_plan(rows, vocabulary, VI_BF16).parts;
-    size_t b = align_up(np * kPub * 4, 256) + align_up(np * kGroups * kGW * 4, 256);
-    if (max_history > 0 && hist_fits(vocabulary, max_history))
-        b += align_up(size_t(rows) * hist_words(vocabulary) * 4, 256) +
-             align_up(size_t(rows) * hist_cap(max_history) * 8, 256) + align_up(size_t(rows) * 8, 256);
+    if (rows <= 0 || vocabulary <= 0 || vocabulary > kMaxVocabulary) return 0;
+    const size_t np = stream_parts_most(std::min(rows, stream_chunk(rows, 1)), vocabulary), r = size_t(rows);
+    size_t b = align_up(np * kPub * 4, 256) + align_up(np * kGroups * kGW * 4, 256) + align_up(r * sizeof(FullBound), 256);
+    if (max_history > 0) {
+        const size_t words = size_t(hist_words(vocabulary)), cap = size_t(hist_cap(vocabulary, max_history));
+        b += align_up(r * words * 4, 256) + align_up(r * cap * 8, 256) + align_up(r * 8, 256);
+        if (!hist_in_lds(vocabulary, max_history)) b += align_up(r * (2 * words + cap) * 4, 256);
+    }
     return b + 256;
 }
 
+template <int DT>
+static void launch_rows(const StreamArgs& a, hipStream_t stream) {
+    const bool pen = a.pstate || a.hb1;
+    if (pen) hipLaunchKernelGGL((stream_kernel<DT, true>), dim3(a.grid), dim3(kT), 0, stream, a);
+    else hipLaunchKernelGGL((stream_kernel<DT, false>), dim3(a.grid), dim3(kT), 0, stream, a);
+    // the merge's workgroup of row r runs on the XCD whose workgroups streamed
+    // the row (workgroup r goes to XCD r % 8, as the stream's rows do)
+    hipLaunchKernelGGL(merge_kernel<DT>, dim3(a.rows), dim3(kT), 0, stream, a);
+    if (!a.probs) return;
+    hipLaunchKernelGGL(probs_kernel<DT>, dim3((a.vocabulary + kPChunk - 1) / kPChunk, a.rows), dim3(kPT), 0, stream, a);
+    if (pen) hipLaunchKernelGGL(repeat_probs_kernel<DT>, dim3(a.rows), dim3(kPT), 0, stream, a);
+}
+
 vi_status launch_stream(const SampleArgs& s, unsigned char* ws, size_t ws_bytes, hipStream_t stream) {
-    if (!stream_supported(s)) return VI_ERR_UNSUPPORTED;
+    if (!stream_supported(s.dtype, s.vocabulary, s.stride)) return VI_ERR_UNSUPPORTED;
+    if (reinterpret_cast<uintptr_t>(s.logits) % 16) return VI_ERR_UNSUPPORTED;
+    if (s.rows <= 0) return VI_OK;
     const StreamPlan pl = stream_plan(s.rows, s.vocabulary, s.dtype);
+    const int chunk = stream_chunk(s.rows, pl.parts);
     StreamArgs a{};
-    a.logits = s.logits; a.rows = s.rows; a.vocabulary = s.vocabulary; a.stride = s.stride;
+    a.vocabulary = s.vocabulary; a.stride = s.stride;
     a.parts = pl.parts; a.part_len = pl.part_len;
-    a.params = s.params;
-    a.record = s.pstate ? s.record : 0;
-    a.tokens = s.tokens; a.uniforms = s.uniforms; a.stats = s.stats;
-    const size_t np = size_t(s.rows) * pl.parts;
+    const size_t np = size_t(chunk) * pl.parts;
     Carver c(ws, ws_bytes);
     a.ppub = c.take<uint32_t>(np * kPub);
     a.pwords = c.take<uint4>(np * kGroups * (kGW / 4));
+    FullBound* bounds = c.take<FullBound>(size_t(s.rows));
+    if (s.full_out) bounds = s.full_out->bounds;
+    else if (!s.probs) bounds = nullptr;
+    a.draw_every = s.full_out ? s.full_out->draw_every : 1;
     const bool hist = !s.pstate && s.histories && s.offsets && s.max_history > 0;
     HistArgs h{};
-    if (s.pstate) {
-        a.pstate = s.pstate;
-        a.pl = s.playout;
-    } else if (hist) {
+    if (hist) {
         h.histories = s.histories; h.offsets = s.offsets; h.params = s.params; h.vocabulary = s.vocabulary;
         h.words = hist_words(s.vocabulary);
-        h.cap = hist_cap(s.max_history);
+        h.cap = hist_cap(s.vocabulary, s.max_history);
         h.hb1 = c.take<uint32_t>(size_t(s.rows) * h.words);
         h.hlist = c.take<uint2>(size_t(s.rows) * h.cap);
         h.hhead = c.take<uint32_t>(size_t(s.rows) * 2);
-        a.hb1 = h.hb1; a.hlist = h.hlist; a.hhead = h.hhead; a.hwords = h.words; a.hcap = h.cap;
+        if (!hist_in_lds(s.vocabulary, s.max_history))
+            h.tmp = c.take<uint32_t>(size_t(s.rows) * (2 * size_t(h.words) + size_t(h.cap)));
+        a.hwords = h.words; a.hcap = h.cap;
     }
     if (!c.ok) return VI_ERR_WORKSPACE;
-    const StreamGrid sg = stream_grid(s.rows, pl.parts);
-    a.grid = sg.grid;
-    a.xcd = sg.xcd;
     if (hist) {
-        hipLaunchKernelGGL(history_view_kernel, dim3(s.rows), dim3(kT), 0, stream, h);
+        if (h.tmp) hipLaunchKernelGGL(history_view_kernel<false>, dim3(s.rows), dim3(kT), 0, stream, h);
+        else hipLaunchKernelGGL(history_view_kernel<true>, dim3(s.rows), dim3(kT), 0, stream, h);
         if (launch_status() != VI_OK) return VI_ERR_LAUNCH;
     }
-    // the merge's workgroup of row r runs on the XCD whose workgroups streamed
-    // the row (workgroup r goes to XCD r % 8, as the stream's rows do)
-    const bool pb = a.pstate || a.hb1;
-    if (s.dtype == VI_BF16) {
-        if (pb) hipLaunchKernelGGL((stream_kernel<VI_BF16, true>), dim3(a.grid), dim3(kT), 0, stream, a);
-        else hipLaunchKernelGGL((stream_kernel<VI_BF16, false>), dim3(a.grid), dim3(kT), 0, stream, a);
-        hipLaunchKernelGGL(merge_kernel<VI_BF16>, dim3(s.rows), dim3(kT), 0, stream, a);
-    } else {
-        if (pb) hipLaunchKernelGGL((stream_kernel<VI_F16, true>), dim3(a.grid), dim3(kT), 0, stream, a);
-        else hipLaunchKernelGGL((stream_kernel<VI_F16, false>), dim3(a.grid), dim3(kT), 0, stream, a);
-        hipLaunchKernelGGL(merge_kernel<VI_F16>, dim3(s.rows), dim3(kT), 0, stream, a);
+    for (int r0 = 0; r0 < s.rows; r0 += chunk) {
+        const size_t at = size_t(r0);
+        a.row0 = r0;
+        a.rows = std::min(chunk, s.rows - r0);
+        a.logits = static_cast<const unsigned char*>(s.logits) + 2 * at * size_t(s.stride);
+        a.params = s.params + at;
+        a.tokens = s.tokens + at;
+        if (s.uniforms) a.uniforms = s.uniforms + at;
+        if (s.stats) a.stats = s.stats + at;
+        if (bounds) a.bounds = bounds + at;
+        if (s.probs) { a.probs = s.probs + at * size_t(s.probs_stride); a.probs_stride = s.probs_stride; }
+        if (s.pstate) {
+            a.pl = s.playout;
+            a.pstate = s.pstate + at * s.playout.lane_bytes;
+            a.record = s.record;
+        } else if (hist) {
+            a.hb1 = h.hb1 + at * size_t(h.words);
+            a.hlist = h.hlist + at * size_t(h.cap);
+            a.hhead = h.hhead + 2 * at;
+        }
+        const StreamGrid sg = stream_grid(a.rows, pl.parts);
+        a.grid = sg.grid;
+        a.xcd = sg.xcd;
+        if (s.dtype == VI_BF16) launch_rows<VI_BF16>(a, stream);
+        else launch_rows<VI_F16>(a, stream);
+        if (launch_status() != VI_OK) return VI_ERR_LAUNCH;
     }
-    return launch_status();
+    return VI_OK;
 }
 
 }  // namespace vi

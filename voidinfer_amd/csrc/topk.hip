@@ -1987,8 +1987,7 @@ size_t sample_workspace(int rows, int vocabulary, int64_t max_history) {
     size_t bytes = topk_partials_bytes(rows, vocabulary);
     bytes += align_up(size_t(rows) * 4, 256);
     if (max_history > 0) bytes += align_up(size_t(rows) * history_hash_slots(max_history) * 8, 256);
-    bytes += std::max({full_workspace(rows, vocabulary), wide_workspace(rows, vocabulary),
-                       stream_workspace(rows, vocabulary, max_history)});
+    bytes += std::max(wide_workspace(rows, vocabulary), stream_workspace(rows, vocabulary, max_history));
     return bytes + 1024;
 }
 
@@ -2008,13 +2007,12 @@ vi_status launch_sample(const SampleArgs& s, void* ws, size_t ws_bytes, hipStrea
         hash = c.take<uint2>(size_t(s.rows) * slots);
     }
     const size_t full_bytes = s.dtype == VI_F32 ? wide_workspace(s.rows, s.vocabulary)
-                                                 : std::max(full_workspace(s.rows, s.vocabulary),
-                                                            stream_workspace(s.rows, s.vocabulary, s.max_history));
+                                                 : stream_workspace(s.rows, s.vocabulary, s.max_history);
     unsigned char* full_ws = c.take<unsigned char>(full_bytes);
     if (!c.ok) return VI_ERR_WORKSPACE;
     const bool run_topk = (s.route_mask & VI_ROUTE_TOPK) != 0;
     const bool full_ok = s.dtype == VI_F32 ? wide_supported(s.vocabulary, s.stride)
-                                           : full_supported(s.dtype, s.vocabulary, s.stride);
+                                           : stream_supported(s.dtype, s.vocabulary, s.stride);
     vi_status st = VI_OK;
     // Histories counted straight into each slice's LDS when the slice's counts
     // fit and no fp32 full-route row needs the hash: no hash launch
@@ -2066,9 +2064,8 @@ vi_status launch_sample(const SampleArgs& s, void* ws, size_t ws_bytes, hipStrea
     }
     if (full_run) {
         if (st == VI_OK)
-            st = s.dtype == VI_F32     ? launch_wide(s, full_ws, full_bytes, hash, shift, slots, row_flags, stream)
-                 : stream_supported(s) ? launch_stream(s, full_ws, full_bytes, stream)
-                                       : launch_full(s, full_ws, full_bytes, stream);
+            st = s.dtype == VI_F32 ? launch_wide(s, full_ws, full_bytes, hash, shift, slots, row_flags, stream)
+                                   : launch_stream(s, full_ws, full_bytes, stream);
     } else if ((s.route_mask & VI_ROUTE_FULL) && !run_topk) {
         return VI_ERR_UNSUPPORTED;
     }

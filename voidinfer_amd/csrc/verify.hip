@@ -9,7 +9,7 @@
 // Sampled mode: the target and draft rows are filtered with the lane's
 // temperature / top-k / top-p / min-p, giving p and q: from top-k lists
 // (topk.hip) for lanes with 1 <= top_k <= 64, from the full-vocabulary
-// sampler's row distributions (sample_slices.hip / sample_wide.hip) for the
+// sampler's row distributions (sample_stream.hip / sample_wide.hip) for the
 // others.  Per position, in order, the rule of
 // Exl3IndependentAcceptanceReference::evaluate
 // (src/exl3/sampled_acceptance_reference.h:48-88): accept iff
@@ -19,12 +19,12 @@
 // (seed, lane, position + j, purpose 1 / 2).  Every (lane, position) decision
 // is taken at once, one wave each over the <= 64-entry lists (fp64): entry-wise
 // work on the lanes, the order-dependent sums on lane 0; the last position of
-// a lane to finish then walks its accept chain in order (after the
-// full-vocabulary kernels, a separate per-lane pass does).  Full-vocabulary lanes: the accept test
-// evaluates the target softmax p and the draft q at the drafted token from the
-// rows' supports, and the correction walks the target softmax, the draft q and
-// their residual over the whole vocabulary in id order (ranges of 16,384
-// tokens summed in parallel, then the crossing range scanned again).
+// a lane to finish then walks its accept chain in order.  Full-vocabulary lanes:
+// the accept test evaluates the target softmax p and the draft q at the drafted
+// token from the rows' supports, and the correction walks the target softmax,
+// the draft q and their residual over the whole vocabulary in id order (ranges
+// of 4,096 tokens summed in parallel, then the crossing range scanned again) and
+// the lane's accept chain.
 #include <algorithm>
 #include <math.h>
 
@@ -61,44 +61,27 @@ __global__ void verify_greedy_kernel(const vi_greedy_row* rows, int lanes, int d
     if (lane_flags) lane_flags[l] = flags;
 }
 
-// The accept chains after the full-vocabulary kernels (one thread per lane).
-__global__ void verify_chain_kernel(const PosDecision* dec, int lanes, int drafts, int target_rows,
-                                    const int32_t* drafted, const vi_row_params* params, const int64_t* terminal,
-                                    int n_terminal, int full_ok, int32_t* accepted, int32_t* committed,
-                                    int32_t* committed_count, uint32_t* lane_flags) {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= lanes) return;
-    const PosDecision* D = dec + size_t(l) * (drafts + 1);
-    lane_chain(l, [&](int j) { return D[j]; }, drafts, target_rows, drafted, params, terminal, n_terminal, full_ok,
-               accepted, committed, committed_count, lane_flags);
-}
-
 // ------------------------------------------------------- full-vocabulary lanes
 // Lanes with temperature > 0 and top_k outside [1, 64].  The full-route sampler
 // leaves every target and draft row's filtered distribution (FullBound: the
-// support's end and mass; bases: end-key logits before each slice) and every
-// target row's own draw (the bonus token); p and q are read off them.
+// support's end and mass) and the bonus rows' draws; p and q are read off them.
 
-constexpr int kFT = 1024;                // accept kernel threads
-constexpr int kRT = 1024;                // residual kernels' threads
-constexpr int kRange = 16384;            // residual range (divides both routes' slices)
+constexpr int kRT = 256;                 // residual kernels' threads
+constexpr int kRange = 4096;             // residual range
 constexpr int kREPT = kRange / kRT;      // tokens per thread and range
 constexpr int kW = kRT / kWave;
-static_assert(kFullSlice16 % kRange == 0 && kFullSlice32 % kRange == 0, "residual ranges");
 
 struct FullRows {
     const void* row0;
     int dtype;
     int64_t stride;
     const FullBound* bound;          // [rows]
-    const uint32_t* bases;           // [rows][kFullBaseSlots]
     const vi_sample_stats* stats;    // [rows]
-    int slice;                       // logits per slice (bases granularity)
 };
 
 struct FullVerifyArgs {
     FullRows t, d;                   // target rows [lanes][target_rows], draft rows [lanes][drafts]
-    const int32_t* ttok;             // the target rows' draws
+    const int32_t* ttok;             // the target rows' tokens (the bonus rows' drawn)
     int lanes, drafts, target_rows, vocabulary;
     const int32_t* drafted;
     const vi_row_params* params;
@@ -108,6 +91,10 @@ struct FullVerifyArgs {
     double* rsum;                    // [lanes][ranges][2]: residual mass, p mass of each range
     int* rlast;                      // [lanes][ranges][2]: last id with residual / with p (-1: none)
     int ranges;
+    int32_t* accepted;
+    int32_t* committed;
+    int32_t* committed_count;
+    uint32_t* lane_flags;
 };
 
 __device__ __forceinline__ const void* row_at(const FullRows& R, size_t r) {
@@ -138,64 +125,32 @@ __device__ __forceinline__ float dist_z(uint32_t k, float inv_t) {
     else return Elem<DT>::decode(unkey16(k)) * inv_t;
 }
 
-// Support membership of a logit of key k; rank: its place among the row's
-// end-key logits in id order (used only when k is the end key).
-__device__ __forceinline__ bool in_support(uint32_t k, const FullBound& B, uint32_t rank) {
-    if (!k || !B.valid) return false;
-    if (k != B.end_key) return k > B.end_key;
-    return B.end_take == 0xffffffffu || rank < B.end_take;
-}
-__device__ __forceinline__ bool counts_rank(uint32_t k, const FullBound& B) {
-    return k && B.valid && k == B.end_key && B.end_take != 0xffffffffu;
+// Support membership of logit `id` of key k.
+__device__ __forceinline__ bool in_support(uint32_t k, int id, const FullBound& B) {
+    return k && B.valid && (k > B.end_key || (k == B.end_key && id <= B.end_id));
 }
 
-// End-key logits of ids [lo, hi) of a row; all threads (NT of them).
-template <int DT, int NT>
-__device__ uint32_t end_key_count(const void* row, int64_t lo, int64_t hi, const FullBound& B, uint32_t* tmp) {
-    uint32_t c = 0u;
-    constexpr int U = 8;   // loads in flight per thread
-    for (int64_t i0 = lo + threadIdx.x; i0 < hi; i0 += int64_t(U) * NT) {
-        uint32_t b[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t i = i0 + int64_t(u) * NT;
-            b[u] = i < hi ? load_bits<DT>(row, i) : 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            c += (i0 + int64_t(u) * NT < hi && counts_rank(dist_key<DT>(b[u], B.inv_t), B)) ? 1u : 0u;
-    }
-    uint32_t tot = 0u;
-    (void)block_exclusive_scan_u32<NT>(c, tmp, &tot);
-    return tot;
-}
-
-// p (or q) of token x in row r; all threads.
-template <int DT, int NT>
-__device__ double prob_at(const FullRows& R, size_t r, int x, uint32_t* tmp) {
+// p (or q) of token x in row r.
+template <int DT>
+__device__ __forceinline__ double prob_at(const FullRows& R, size_t r, int x) {
     const FullBound B = R.bound[r];
-    const void* row = row_at(R, r);
-    const uint32_t k = dist_key<DT>(load_bits<DT>(row, x), B.inv_t);
-    uint32_t rank = 0u;
-    if (counts_rank(k, B)) {   // (uniform)
-        const int s = x / R.slice;
-        rank = R.bases[r * kFullBaseSlots + s] + end_key_count<DT, NT>(row, int64_t(s) * R.slice, x, B, tmp);
-    }
-    return in_support(k, B, rank) ? exp(double(dist_z<DT>(k, B.inv_t)) - B.z0) / B.s_n : 0.0;
+    const uint32_t k = dist_key<DT>(load_bits<DT>(row_at(R, r), x), B.inv_t);
+    return in_support(k, x, B) ? exp(double(dist_z<DT>(k, B.inv_t)) - B.z0) / B.s_n : 0.0;
 }
 
 // The accept test of every (lane, position) of the full-vocabulary lanes:
 // u_a < min(1, p(d) / q(d)) with the target softmax p and the draft q at the
-// drafted token; position `drafts` takes the bonus row's draw.
+// drafted token; position `drafts` takes the bonus row's draw.  A thread per
+// position.
 template <int TDT, int DDT>
-__global__ __launch_bounds__(kFT) void verify_full_accept_kernel(FullVerifyArgs a) {
-    __shared__ uint32_t tmp[kFT / kWave + 1];
-    const int j = blockIdx.x, l = blockIdx.y;
+__global__ __launch_bounds__(kWave) void verify_full_accept_kernel(FullVerifyArgs a) {
+    const int l = blockIdx.y, j = int(blockIdx.x) * kWave + int(threadIdx.x);
+    if (j > a.drafts) return;
     const vi_row_params p = a.params[l];
     if (!verify_list_refused(p)) return;
     PosDecision* out = a.dec + size_t(l) * (a.drafts + 1) + j;
     if (j == a.drafts) {
-        if (a.target_rows != a.drafts + 1 || threadIdx.x != 0) return;
+        if (a.target_rows != a.drafts + 1) return;
         const size_t tr = size_t(l) * a.target_rows + j;
         const uint32_t f = a.t.stats[tr].flags;
         const int32_t tok = a.ttok[tr];
@@ -209,17 +164,15 @@ __global__ __launch_bounds__(kFT) void verify_full_accept_kernel(FullVerifyArgs 
                      uint32_t(VI_FLAG_NONFINITE | VI_FLAG_EMPTY | VI_FLAG_ERROR);
     double q = 0.0, pv = 0.0;
     if (x >= 0 && x < a.vocabulary) {
-        q = prob_at<DDT, kFT>(a.d, dr, x, tmp);
-        pv = prob_at<TDT, kFT>(a.t, tr, x, tmp);
+        q = prob_at<DDT>(a.d, dr, x);
+        pv = prob_at<TDT>(a.t, tr, x);
     }
-    if (threadIdx.x == 0) {
-        const double ua = philox_uniform(p.seed, p.lane, p.position + j, 1u);
-        double acc = 0.0;
-        if (q == 0.0) flags |= VI_FLAG_ZERO_Q;
-        else acc = fmin(1.0, pv / q);
-        const int accept = (!(flags & VI_FLAG_ERROR) && q != 0.0 && ua < acc) ? 1 : 0;
-        *out = PosDecision{-1, flags, accept, 0};
-    }
+    const double ua = philox_uniform(p.seed, p.lane, p.position + j, 1u);
+    double acc = 0.0;
+    if (q == 0.0) flags |= VI_FLAG_ZERO_Q;
+    else acc = fmin(1.0, pv / q);
+    const int accept = (!(flags & VI_FLAG_ERROR) && q != 0.0 && ua < acc) ? 1 : 0;
+    *out = PosDecision{-1, flags, accept, 0};
 }
 
 // The lane's first rejected position before any accepted terminal token, or -1:
@@ -248,37 +201,26 @@ __device__ __forceinline__ float weight_f(float z, float z0) {
     return __builtin_amdgcn_exp2f((z - z0) * 1.44269504088896340736f);
 }
 
-// End-key logits of the row before id r0 (a range start).
-template <int DT>
-__device__ uint32_t range_base(const FullRows& R, size_t r, const FullBound& B, int r0, uint32_t* tmp) {
-    if (!B.valid || B.end_take == 0xffffffffu) return 0u;   // (uniform)
-    const int s = r0 / R.slice, in = r0 - s * R.slice;
-    return R.bases[r * kFullBaseSlots + s] +
-           (in ? end_key_count<DT, kRT>(row_at(R, r), int64_t(s) * R.slice, r0, B, tmp) : 0u);
-}
-
 // Tokens [r0, r1) of the target and draft rows of one position: fn(e, id, p, q)
 // for this thread's tokens r0 + kREPT t + e, in id order; all threads.
 template <int TDT, int DDT, class F>
-__device__ __forceinline__ void range_pass(const FullVerifyArgs& a, size_t tr, size_t dr, int r0, int r1,
-                                           uint32_t* tmp, F&& fn) {
+__device__ __forceinline__ void range_pass(const FullVerifyArgs& a, size_t tr, size_t dr, int r0, int r1, F&& fn) {
     const FullBound TB = a.t.bound[tr], DB = a.d.bound[dr];
     const void* trow = row_at(a.t, tr);
     const void* drow = row_at(a.d, dr);
     // weights exp(z - z0) in single precision (z0 is a float z); 1 / S_n in double
     const float tz0 = float(TB.z0), dz0 = float(DB.z0);
     const double tinv = TB.valid ? 1.0 / TB.s_n : 0.0, dinv = DB.valid ? 1.0 / DB.s_n : 0.0;
-    const uint32_t bt = range_base<TDT>(a.t, tr, TB, r0, tmp), bd = range_base<DDT>(a.d, dr, DB, r0, tmp);
     const int e0 = r0 + kREPT * int(threadIdx.x);
-    // this thread's kREPT consecutive logits of each row: whole 16-byte vectors
-    // when the row is aligned and they are all inside the range (the pass is
-    // latency bound: a few wide loads instead of one 2- or 4-byte load each)
+    // this thread's kREPT consecutive logits of each row: 16-byte vectors when
+    // they are all inside the range (the pass is latency bound: a few wide loads
+    // instead of one 2- or 4-byte load each)
     uint32_t bt_[kREPT], bd_[kREPT];
     auto fetch = [&](const void* rowp, auto dt, uint32_t (&b)[kREPT]) {
         constexpr int DT = decltype(dt)::value;
         constexpr int PV = Elem<DT>::kPerVec;
         const unsigned char* p = static_cast<const unsigned char*>(rowp) + size_t(e0) * (DT == VI_F32 ? 4 : 2);
-        if (e0 + kREPT <= r1 && (reinterpret_cast<uintptr_t>(p) & 15u) == 0) {
+        if (e0 + kREPT <= r1) {
 #pragma unroll
             for (int q = 0; q < kREPT / PV; ++q) {
                 const uint4 v = load16_cached(p + 16 * q);
@@ -292,26 +234,14 @@ __device__ __forceinline__ void range_pass(const FullVerifyArgs& a, size_t tr, s
     };
     fetch(trow, std::integral_constant<int, TDT>{}, bt_);
     fetch(drow, std::integral_constant<int, DDT>{}, bd_);
-    uint32_t kt[kREPT], kd[kREPT], ct = 0u, cd = 0u;
 #pragma unroll
     for (int e = 0; e < kREPT; ++e) {
         const int i = e0 + e;
-        kt[e] = i < r1 ? dist_key<TDT>(bt_[e], TB.inv_t) : 0u;
-        kd[e] = i < r1 ? dist_key<DDT>(bd_[e], DB.inv_t) : 0u;
-        ct += counts_rank(kt[e], TB) ? 1u : 0u;
-        cd += counts_rank(kd[e], DB) ? 1u : 0u;
-    }
-    uint32_t tot = 0u;
-    uint32_t rt = bt + block_exclusive_scan_u32<kRT>(ct, tmp, &tot);
-    uint32_t rd = bd + block_exclusive_scan_u32<kRT>(cd, tmp, &tot);
-#pragma unroll
-    for (int e = 0; e < kREPT; ++e) {
-        const bool it = in_support(kt[e], TB, rt), id = in_support(kd[e], DB, rd);
-        rt += counts_rank(kt[e], TB) ? 1u : 0u;
-        rd += counts_rank(kd[e], DB) ? 1u : 0u;
-        const double pv = it ? double(weight_f(dist_z<TDT>(kt[e], TB.inv_t), tz0)) * tinv : 0.0;
-        const double qv = id ? double(weight_f(dist_z<DDT>(kd[e], DB.inv_t), dz0)) * dinv : 0.0;
-        fn(e, e0 + e, pv, qv);
+        const uint32_t kt = i < r1 ? dist_key<TDT>(bt_[e], TB.inv_t) : 0u;
+        const uint32_t kd = i < r1 ? dist_key<DDT>(bd_[e], DB.inv_t) : 0u;
+        const double pv = in_support(kt, i, TB) ? double(weight_f(dist_z<TDT>(kt, TB.inv_t), tz0)) * tinv : 0.0;
+        const double qv = in_support(kd, i, DB) ? double(weight_f(dist_z<DDT>(kd, DB.inv_t), dz0)) * dinv : 0.0;
+        fn(e, i, pv, qv);
     }
 }
 
@@ -340,7 +270,6 @@ __device__ int block_max_i(int v, int* tmp) {
 // Residual and p mass of each range of each lane's rejected position.
 template <int TDT, int DDT>
 __global__ __launch_bounds__(kRT) void verify_full_ranges_kernel(FullVerifyArgs a) {
-    __shared__ uint32_t tmp[kW + 1];
     __shared__ double dtmp[kW];
     __shared__ int itmp[kW];
     const int rg = blockIdx.x, l = blockIdx.y;
@@ -351,7 +280,7 @@ __global__ __launch_bounds__(kRT) void verify_full_ranges_kernel(FullVerifyArgs 
     const int r0 = rg * kRange, r1 = min(a.vocabulary, r0 + kRange);
     double R = 0.0, P = 0.0;
     int lr = -1, lp = -1;
-    range_pass<TDT, DDT>(a, tr, dr, r0, r1, tmp, [&](int, int i, double pv, double qv) {
+    range_pass<TDT, DDT>(a, tr, dr, r0, r1, [&](int, int i, double pv, double qv) {
         const double rv = fmax(0.0, pv - qv);
         R += rv;
         P += pv;
@@ -372,10 +301,9 @@ __global__ __launch_bounds__(kRT) void verify_full_ranges_kernel(FullVerifyArgs 
 // The correction of each lane's rejected position: the first token (id order)
 // whose cumulative residual exceeds u_c times the residual mass, or, with no
 // residual mass (<= 1e-9), the first whose cumulative p exceeds u_c; past the
-// end by round-off, the last token with mass.
+// end by round-off, the last token with mass.  Then the lane's accept chain.
 template <int TDT, int DDT>
 __global__ __launch_bounds__(kRT) void verify_full_correction_kernel(FullVerifyArgs a) {
-    __shared__ uint32_t tmp[kW + 1];
     __shared__ double dtmp[kW + 1];
     __shared__ int s_range, s_tok;
     __shared__ double s_before, s_target;
@@ -384,41 +312,49 @@ __global__ __launch_bounds__(kRT) void verify_full_correction_kernel(FullVerifyA
     const vi_row_params p = a.params[l];
     if (!verify_list_refused(p)) return;
     const int js = first_rejection(a, l);
-    if (js < 0) return;
-    if (wave == 0) {   // the ranges in order (each lane loads a range's sums; the sums read lane by lane)
+    if (tid == 0) { s_range = -1; s_tok = -1; s_nores = 0u; }
+    __syncthreads();
+    if (js >= 0 && wave == 0) {   // the ranges' sums, 64 at a time in id order
         double R = 0.0, P = 0.0;
         int lr = -1, lp = -1;
         for (int r0 = 0; r0 < a.ranges; r0 += kWave) {
-            const int r = min(r0 + lane, a.ranges - 1);
-            const size_t at = (size_t(l) * a.ranges + r) * 2;
-            const double rs = a.rsum[at], ps = a.rsum[at + 1];
-            const int rl = a.rlast[at], pl = a.rlast[at + 1];
-            for (int q = 0; q < min(kWave, a.ranges - r0); ++q) {
-                R += readlane_d(rs, q);
-                P += readlane_d(ps, q);
-                lr = max(lr, __builtin_amdgcn_readlane(rl, q));
-                lp = max(lp, __builtin_amdgcn_readlane(pl, q));
-            }
+            const bool in = r0 + lane < a.ranges;
+            const size_t at = (size_t(l) * a.ranges + min(r0 + lane, a.ranges - 1)) * 2;
+            R += readlane_d(wave_incl_scan_f64(in ? a.rsum[at] : 0.0), kWave - 1);
+            P += readlane_d(wave_incl_scan_f64(in ? a.rsum[at + 1] : 0.0), kWave - 1);
+            lr = max(lr, a.rlast[at]);
+            lp = max(lp, a.rlast[at + 1]);
+        }
+#pragma unroll
+        for (int o = 32; o; o >>= 1) {
+            lr = max(lr, __shfl_xor(lr, o, kWave));
+            lp = max(lp, __shfl_xor(lp, o, kWave));
         }
         const double uc = philox_uniform(p.seed, p.lane, p.position + js, 2u);
         const bool nores = !(R > 1e-9) || !isfinite(R);
         const double target = nores ? uc : uc * R;
         int range = -1;
-        double cum = 0.0;
+        double cum = 0.0, before = 0.0;
         for (int r0 = 0; r0 < a.ranges && range < 0; r0 += kWave) {
-            const double mv = a.rsum[(size_t(l) * a.ranges + min(r0 + lane, a.ranges - 1)) * 2 + (nores ? 1 : 0)];
-            for (int q = 0; q < min(kWave, a.ranges - r0) && range < 0; ++q) {
-                const double m = readlane_d(mv, q);
-                if (cum + m > target) range = r0 + q;
-                else cum += m;
+            const bool in = r0 + lane < a.ranges;
+            const double m = in ? a.rsum[(size_t(l) * a.ranges + r0 + lane) * 2 + (nores ? 1 : 0)] : 0.0;
+            const double incl = wave_incl_scan_f64(m);
+            const uint64_t hit = ballot(in && cum + incl > target);
+            if (hit) {
+                const int f = __builtin_ctzll(hit);
+                range = r0 + f;
+                before = cum + (f ? readlane_d(incl, f - 1) : 0.0);
             }
+            cum += readlane_d(incl, kWave - 1);
         }
         if (lane == 0) {
             s_range = range;
-            s_before = cum;
+            s_before = before;
             s_target = target;
             s_nores = nores ? 1u : 0u;
-            s_tok = max(0, nores ? lp : lr);   // (round-off past the end)
+            // (round-off past the end)
+            const int last = range < 0 ? -1 : a.rlast[(size_t(l) * a.ranges + range) * 2 + (nores ? 1 : 0)];
+            s_tok = max(0, last >= 0 ? last : nores ? lp : lr);
         }
     }
     __syncthreads();
@@ -429,7 +365,7 @@ __global__ __launch_bounds__(kRT) void verify_full_correction_kernel(FullVerifyA
         const bool nores = s_nores != 0u;
         double v[kREPT], own = 0.0;
         int last = -1;
-        range_pass<TDT, DDT>(a, tr, dr, r0, r1, tmp, [&](int e, int i, double pv, double qv) {
+        range_pass<TDT, DDT>(a, tr, dr, r0, r1, [&](int e, int i, double pv, double qv) {
             v[e] = nores ? pv : fmax(0.0, pv - qv);
             own += v[e];
             if (v[e] > 0.0) last = i;
@@ -460,10 +396,19 @@ __global__ __launch_bounds__(kRT) void verify_full_correction_kernel(FullVerifyA
         }
         __syncthreads();
     }
-    if (tid == 0) {
-        PosDecision* out = a.dec + size_t(l) * (a.drafts + 1) + js;
-        out->token = s_tok;
-        if (s_nores) out->flags |= VI_FLAG_NO_RESIDUAL;
+    if (wave == 0) {
+        const PosDecision* D = a.dec + size_t(l) * (a.drafts + 1);
+        const int tok = s_tok;
+        const uint32_t nores = s_nores;
+        lane_chain_wave(l, [&](int j) {
+            PosDecision e = D[j];
+            if (j == js) {
+                e.token = tok;
+                if (nores) e.flags |= VI_FLAG_NO_RESIDUAL;
+            }
+            return e;
+        }, a.drafts, a.target_rows, a.drafted, a.params, a.terminal, a.n_terminal, 1, a.accepted, a.committed,
+           a.committed_count, a.lane_flags);
     }
 }
 
@@ -507,14 +452,13 @@ VerifyLayout verify_layout(int lanes, int drafts, int vocabulary) {
 namespace {
 inline int full_ranges(int vocabulary) { return (vocabulary + kRange - 1) / kRange; }
 inline size_t full_sampler_bytes(int rows, int vocabulary) {
-    return std::max(full_workspace(rows, vocabulary), wide_workspace(rows, vocabulary));
+    return std::max(stream_workspace(rows, vocabulary, 0), wide_workspace(rows, vocabulary));
 }
 // The full-vocabulary path's part of the workspace (after the list path's).
 size_t full_verify_bytes(int lanes, int drafts, int vocabulary) {
     const size_t rows = size_t(lanes) * size_t(2 * drafts + 1);   // target (with bonus) and draft rows
     size_t b = align_up(rows * sizeof(vi_row_params), 256) + align_up(rows * sizeof(FullBound), 256);
-    b += align_up(rows * kFullBaseSlots * 4, 256) + align_up(rows * sizeof(vi_sample_stats), 256);
-    b += align_up(rows * 4, 256);
+    b += align_up(rows * sizeof(vi_sample_stats), 256) + align_up(rows * 4, 256);
     b += align_up(size_t(lanes) * full_ranges(vocabulary) * 2 * 8, 256) +
          align_up(size_t(lanes) * full_ranges(vocabulary) * 2 * 4, 256);
     // (one sampler workspace per row set: the two sets are sampled side by side)
@@ -523,12 +467,12 @@ size_t full_verify_bytes(int lanes, int drafts, int vocabulary) {
 }
 bool full_path_ok(const void* logits, int dtype, int vocabulary, int64_t stride) {
     if (dtype == VI_F32) return wide_supported(vocabulary, stride) && reinterpret_cast<uintptr_t>(logits) % 4 == 0;
-    return full_supported(dtype, vocabulary, stride) && reinterpret_cast<uintptr_t>(logits) % 16 == 0;
+    return stream_supported(dtype, vocabulary, stride) && reinterpret_cast<uintptr_t>(logits) % 16 == 0;
 }
 
 template <int TDT, int DDT>
 void launch_full_verify(const FullVerifyArgs& f, hipStream_t stream) {
-    hipLaunchKernelGGL((verify_full_accept_kernel<TDT, DDT>), dim3(f.drafts + 1, f.lanes), dim3(kFT), 0, stream, f);
+    hipLaunchKernelGGL((verify_full_accept_kernel<TDT, DDT>), dim3(f.drafts / kWave + 1, f.lanes), dim3(kWave), 0, stream, f);
     hipLaunchKernelGGL((verify_full_ranges_kernel<TDT, DDT>), dim3(f.ranges, f.lanes), dim3(kRT), 0, stream, f);
     hipLaunchKernelGGL((verify_full_correction_kernel<TDT, DDT>), dim3(f.lanes), dim3(kRT), 0, stream, f);
 }
@@ -625,8 +569,6 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
     vi_row_params* dpar = c.take<vi_row_params>(dn);
     FullBound* tb = c.take<FullBound>(tn);
     FullBound* db = c.take<FullBound>(dn);
-    uint32_t* tbase = c.take<uint32_t>(tn * kFullBaseSlots);
-    uint32_t* dbase = c.take<uint32_t>(dn * kFullBaseSlots);
     vi_sample_stats* tst = c.take<vi_sample_stats>(tn);
     vi_sample_stats* dst = c.take<vi_sample_stats>(dn);
     int32_t* ttok = c.take<int32_t>(tn);
@@ -641,7 +583,7 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
     if (!c.ok) return VI_ERR_WORKSPACE;
     hipLaunchKernelGGL(verify_row_params_kernel, dim3((trows + drows + 255) / 256), dim3(256), 0, stream,
                        a.params, a.lanes, a.target_rows, tpar, a.drafts, dpar);
-    // the rows' filtered distributions (and the target rows' draws) from the
+    // the rows' filtered distributions (and the bonus rows' draws) from the
     // full-vocabulary sampler, each row set in its own workspace: the draft
     // rows on the side stream beside the target rows on the caller's, joined
     // back before the accept launch
@@ -651,9 +593,9 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
         SampleArgs s{};
         s.logits = logits; s.dtype = dtype; s.rows = rows; s.vocabulary = a.vocabulary; s.stride = stride;
         s.params = par; s.tokens = tok; s.stats = stats; s.route_mask = VI_ROUTE_FULL; s.full_out = out;
-        return dtype == VI_F32 ? launch_wide(s, w, wb, nullptr, 0, 0, nullptr, on) : launch_full(s, w, wb, on);
+        return dtype == VI_F32 ? launch_wide(s, w, wb, nullptr, 0, 0, nullptr, on) : launch_stream(s, w, wb, on);
     };
-    const FullOut tout{tb, tbase}, dout{db, dbase};
+    const FullOut tout{tb, a.target_rows == a.drafts + 1 ? a.target_rows : 0}, dout{db, 0};
     SideStream* side = drows > 0 ? side_stream() : nullptr;
     if (side && (hipEventRecord(side->fork, stream) != hipSuccess ||
                  hipStreamWaitEvent(side->stream, side->fork, 0) != hipSuccess)) {
@@ -670,10 +612,10 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
         return VI_ERR_LAUNCH;
     if (st != VI_OK) return st;
     FullVerifyArgs f{};
-    f.t = FullRows{a.target, a.target_dtype, a.target_stride, tb, tbase, tst,
-                   a.target_dtype == VI_F32 ? kFullSlice32 : kFullSlice16};
-    f.d = FullRows{a.draft, a.draft_dtype, a.draft_stride, db, dbase, dst,
-                   a.draft_dtype == VI_F32 ? kFullSlice32 : kFullSlice16};
+    f.t = FullRows{a.target, a.target_dtype, a.target_stride, tb, tst};
+    f.d = FullRows{a.draft, a.draft_dtype, a.draft_stride, db, dst};
+    f.accepted = a.accepted; f.committed = a.committed; f.committed_count = a.committed_count;
+    f.lane_flags = a.lane_flags;
     f.ttok = ttok; f.lanes = a.lanes; f.drafts = a.drafts; f.target_rows = a.target_rows;
     f.vocabulary = a.vocabulary; f.drafted = a.drafted; f.params = a.params; f.terminal = a.terminal;
     f.n_terminal = a.n_terminal; f.dec = dec; f.rsum = rsum; f.rlast = rlast; f.ranges = ranges;
@@ -682,11 +624,6 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
         case VI_F16: launch_full_verify_d<VI_F16>(f, stream); break;
         default: launch_full_verify_d<VI_F32>(f, stream); break;
     }
-    st = launch_status();
-    if (st != VI_OK) return st;
-    hipLaunchKernelGGL(verify_chain_kernel, dim3(blocks), dim3(threads), 0, stream, dec, a.lanes, a.drafts,
-                       a.target_rows, a.drafted, a.params, a.terminal, a.n_terminal, full_ok, a.accepted, a.committed,
-                       a.committed_count, a.lane_flags);
     return launch_status();
 }
 

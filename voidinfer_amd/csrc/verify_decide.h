@@ -235,49 +235,7 @@ __device__ inline void position_decision(const vi_row_params& p, int j, int l, i
 // accepted drafts are committed until the first rejection (its correction is
 // committed and ends the chain) or a terminal token; a lane that accepted
 // every draft commits the bonus draw.  Flags of the positions visited (and the
-// bonus row).
-template <class Load>
-__device__ __forceinline__ void lane_chain(int l, Load load, int drafts, int target_rows, const int32_t* drafted,
-                                           const vi_row_params* params, const int64_t* terminal, int n_terminal,
-                                           int full_ok, int32_t* accepted, int32_t* committed,
-                                           int32_t* committed_count, uint32_t* lane_flags) {
-    int32_t* out = committed + size_t(l) * (drafts + 1);
-    for (int j = 0; j <= drafts; ++j) out[j] = -1;
-    if (verify_list_refused(params[l]) && !full_ok) {   // refused lane: nothing accepted, nothing committed
-        accepted[l] = 0;
-        committed_count[l] = 0;
-        if (lane_flags) lane_flags[l] = VI_FLAG_ERROR;
-        return;
-    }
-    uint32_t flags = 0;
-    int c = 0, acc = 0;
-    bool stopped = false, rejected = false;
-    for (int j = 0; j < drafts; ++j) {
-        const PosDecision e = load(j);
-        flags |= e.flags;
-        if (e.accept) {
-            const int32_t d = drafted[size_t(l) * drafts + j];
-            out[c++] = d;
-            ++acc;
-            stopped = is_terminal(terminal, n_terminal, d);
-            if (stopped) break;
-            continue;
-        }
-        out[c++] = e.token;
-        rejected = true;
-        break;
-    }
-    if (!rejected && !stopped && acc == drafts && target_rows == drafts + 1) {
-        const PosDecision b = load(drafts);
-        flags |= b.flags;
-        if (b.token >= 0) out[c++] = b.token;
-    }
-    accepted[l] = acc;
-    committed_count[l] = c;
-    if (lane_flags) lane_flags[l] = flags;
-}
-
-// The same chain walked by one wave: 64 positions' decisions and drafted tokens
+// bonus row).  Walked by one wave: 64 positions' decisions and drafted tokens
 // read at once (load(j) with a different j on every lane), the first position
 // that stops the chain (a rejection, or an accepted terminal token) found by a
 // ballot, the visited positions' flags OR-reduced; the committed entries are

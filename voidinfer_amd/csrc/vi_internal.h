@@ -81,12 +81,8 @@ vi_status launch_sampled_scores(const void* scores, int dtype, int rows, int voc
                                 const int64_t* next, int64_t* chosen, float* gap, void* ws, size_t ws_bytes,
                                 hipStream_t stream);
 
-// Sorted, filtered top-k lists (z values, ids) of verification rows.  With
-// `decide` (every lane listed) the rows' last workgroups also take decisions:
-// decide_mode 2 over the target rows draws the bonus rows' tokens; decide_mode
-// 1 over the draft rows (the target rows' lists complete before the launch)
-// takes each position's accept decision, and each lane's last position walks
-// the lane's chain.
+// What the verification rows' sorted, filtered top-k lists (z values, ids) are
+// decided with.
 struct PosDecision;
 struct VerifyDecideArgs {
     int drafts, target_rows;
@@ -168,24 +164,23 @@ vi_status launch_penalty_update(void* states, int lanes, int vocabulary, const P
 
 // Filtered distribution of one full-route row, as the merges leave it for the
 // probabilities and for verification: the support is every valid logit whose
-// order key lies above end_key, plus the first end_take logits of end_key in id
-// order (end_take ~0u: all of them; end_key 0: every valid logit); there
-// p = exp(z - z0) / s_n.  valid = 0: no distribution (empty or failed row).
+// order key lies above end_key, plus those of end_key with ids up to end_id
+// (end_key 0: every valid logit); there p = exp(z - z0) / s_n.  valid = 0: no distribution (empty or failed row).
 // Order keys: key16 of the (penalized) 16-bit pattern, or the 32-bit order key
 // of z for fp32 rows.
 struct FullBound {
     double z0, s_n;
     float inv_t;
-    uint32_t end_key, end_take, valid;
+    uint32_t end_key;
+    int32_t end_id;
+    uint32_t valid;
 };
-constexpr int kFullBaseSlots = 32;   // bases per row: end-key logits in the slices before each slice
 // Optional outputs of a full-route launch (verification reads them back).
 struct FullOut {
     FullBound* bounds;   // [rows]
-    uint32_t* bases;     // [rows][kFullBaseSlots]
+    int draw_every;      // rows whose token is drawn: every n-th (row % n == n - 1), or none (0); the others'
+                         // tokens, uniforms and support sizes are not written
 };
-// Logits per slice of the full routes (granularity of FullOut::bases).
-constexpr int kFullSlice16 = 32768, kFullSlice32 = 16384;
 
 struct SampleArgs {
     const void* logits;
@@ -209,7 +204,7 @@ struct SampleArgs {
 size_t sample_workspace(int rows, int vocabulary, int64_t max_history);
 vi_status launch_sample(const SampleArgs& a, void* ws, size_t ws_bytes, hipStream_t stream);
 
-// ---- full-vocabulary pair kernel --------------------------------------------
+// ---- launch helpers ------------------------------------------------------------
 int device_cus();
 // A second stream of the calling host thread on the current device, with a
 // fork and a join event (created on first use; nullptr when unavailable): a
@@ -220,14 +215,10 @@ struct SideStream {
     hipEvent_t fork, join;
 };
 SideStream* side_stream();
-// ---- full-vocabulary rows, stream and merge launches (sample_stream.hip): 16-bit logits,
-// aligned rows, vocabulary a multiple of 8, no probabilities or bounds wanted.
-bool stream_supported(const SampleArgs& s);
+// ---- full-vocabulary rows of 16-bit logits (sample_stream.hip)
+bool stream_supported(int dtype, int vocabulary, int64_t stride);
 size_t stream_workspace(int rows, int vocabulary, int64_t max_history);
 vi_status launch_stream(const SampleArgs& s, unsigned char* ws, size_t ws_bytes, hipStream_t stream);
-size_t full_workspace(int rows, int vocabulary);
-vi_status launch_full(const SampleArgs& a, unsigned char* ws, size_t ws_bytes, hipStream_t stream);
-bool full_supported(int dtype, int vocabulary, int64_t stride);
 // fp32 rows of the full route (sample_wide.hip); the history route's hash and
 // flags are the top-k route's buffers (rows of the two routes are disjoint).
 size_t wide_workspace(int rows, int vocabulary);
