@@ -106,9 +106,11 @@ constexpr int kOffMBmass = kOffMBcnt + 8192;          // u64[2048]: block masses
 constexpr int kOffMCab = kOffMBmass + 16384;          // u32[2048]: logits in the blocks above
 constexpr int kOffMMab = kOffMCab + 8192;             // u64[2048]: mass of the blocks above
 constexpr int kOffMFlip = kOffMMab + 16384;           // u32[2048]: rescan flips (65,536 bits)
-constexpr int kOffMKeys = kOffMFlip + 8192;           // uint4[slot][16]: (lo, hi) counts of word pairs
+constexpr int kOffMKeys = kOffMFlip + 8192;           // uint4[slot][16]: (lo, hi) counts of word pairs; then (the
+                                                      // rescan) uint2[2048]: the owner part's repeat entries
 constexpr int kMLds = 155648;
 constexpr uint32_t kSlotCap = (kMLds - kOffMKeys) / (16 * 16);
+constexpr uint32_t kNoSlot = 0xffffu;    // slot of a group no part holds
 static_assert(kOffMKeys % 16 == 0 && kSlotCap >= 256, "merge map");
 
 struct StreamArgs {
@@ -596,6 +598,8 @@ struct MergeShared {
     uint32_t scan[kW + 1];
     uint32_t wtot[8][kW];
     uint64_t wmass[kW];
+    uint32_t wci[kW];   // the running sums through each wave's 128 blocks
+    uint64_t wmi[kW];
     uint32_t nslots, total_cnt, z0key, owner, orank, flags, kmin, kmax;
     uint64_t total_mass;
     // the ranks to name: [0] the last end-key logit inside the support (when the
@@ -603,7 +607,7 @@ struct MergeShared {
     uint32_t want[2], key[2], rank[2];
     int32_t id[2];
     uint32_t end_key;
-    uint32_t n_support, ok, lo1, hi1, nflip;
+    uint32_t n_support, ok, lo1, hi1, nflip, nown;
     double s_n, u;
 };
 
@@ -690,6 +694,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         if (lane == 0) { sh.kmin = km & 0xffffu; sh.kmax = km >> 16; }
     }
     for (int i = tid; i < 2048; i += kT) { bcnt[i] = 0u; bmass[i] = 0ull; }
+    if (tid == 2 * kWave) sh.u = philox_uniform(p.seed, p.lane, p.position, 0u);
     if (tid == 0) { sh.flags = pv.flags; sh.ok = 1u; sh.z0key = 0u; }
     lds_barrier();
     if (tid < P * 32) {
@@ -704,7 +709,8 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         const uint32_t o = (occ[gb.word] >> gb.shift) & 1u;
         uint32_t n = 0u;
         const uint32_t e = block_scan_lds(o, sh.scan, &n);
-        if (o) { slot_of[tid] = uint16_t(e); group_of[e] = uint16_t(tid); }
+        slot_of[tid] = uint16_t(o ? e : kNoSlot);
+        if (o) group_of[e] = uint16_t(tid);
         if (tid == 0) sh.nslots = n;
     }
     lds_barrier();
@@ -911,6 +917,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             cb = readlane_u(wave_incl_scan_u32(e ? sh.scan[lane] : 0u), kWave - 1);
             mb = readlane_u64(wave_incl_scan_u64(e ? sh.wmass[lane] : 0ull), kWave - 1);
         }
+        if (lane == kWave - 1) { sh.wci[wave] = cb + ci; sh.wmi[wave] = mb + mi; }
         if (tid == kT - 1) { sh.total_cnt = cb + ci; sh.total_mass = mb + mi; }
         const uint32_t ce = cb + ci - (c0 + c1);
         const uint64_t me = mb + mi - (m0 + m1);
@@ -941,29 +948,36 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         const uint32_t k = 32u * b + 31u - uint32_t(lane & 31);
         if (lane >= 32 || !key_valid<DT>(k, kmin, kmax)) return 0u;
         const KeyLoc kl = key_loc(k);
-        const GroupBit gb = group_bit(kl.group);
-        if (!((occ[gb.word] >> gb.shift) & 1u)) return 0u;
-        const uint4 c = store_keys ? keys[uint32_t(slot_of[kl.group]) * 16u + (kl.word >> 1)]
-                                   : sum_pair(kl.group, kl.word >> 1);
+        const uint32_t slot = slot_of[kl.group];
+        if (slot == kNoSlot) return 0u;
+        const uint4 c = store_keys ? keys[slot * 16u + (kl.word >> 1)] : sum_pair(kl.group, kl.word >> 1);
         const uint32_t lo = (kl.word & 1u) ? c.z : c.x, hi = (kl.word & 1u) ? c.w : c.y;
         return kl.hi ? hi : lo;
     };
     // Wave 0: the first block (descending) at which the cumulative count
     // (mode 0: >= target) or fixed-point mass (mode 1: >= target, mode 2: >
-    // target) is reached, searched over the blocks' running sums; -1 if none.
+    // target) is reached; -1 if none.  First the wave of the running sums that
+    // holds it, then its 128 blocks, two to a lane.  (A search over the 2048
+    // sums themselves probes every 32nd first, all in one LDS bank: 1,700 cycles.)
     auto block_search = [&](int mode, uint64_t target) -> int {
         if (mode == 1 && target == 0u) return -1;
-        const int i = wave_search(0, 2048, [&](int i) {
-            const int b = 2047 - i;
-            if (mode == 0) return uint64_t(cab[b]) + bcnt[b] >= target;
-            const uint64_t inc = mab[b] + bmass[b];
-            return mode == 1 ? inc >= target : inc > target;
-        });
-        return i < 2048 ? 2047 - i : -1;
+        auto reached = [&](uint64_t x) { return mode == 2 ? x > target : x >= target; };
+        const int wl = lane & (kW - 1);
+        const uint64_t wm = ballot(lane < kW && reached(mode == 0 ? uint64_t(sh.wci[wl]) : sh.wmi[wl]));
+        if (!wm) return -1;
+        const int b0 = 2047 - 128 * __builtin_ctzll(wm) - 2 * lane, b1 = b0 - 1;
+        const uint64_t s0 = mode == 0 ? uint64_t(cab[b1]) : mab[b1];   // (through b0)
+        const uint64_t s1 = s0 + (mode == 0 ? uint64_t(bcnt[b1]) : bmass[b1]);
+        const uint64_t m0 = ballot(reached(s0)), m1 = ballot(reached(s1));
+        if (!m1) return -1;
+        const int L = __builtin_ctzll(m1);
+        return 2047 - 128 * __builtin_ctzll(wm) - 2 * L - (((m0 >> L) & 1ull) ? 0 : 1);
     };
     struct Fine {
         bool found;
         uint32_t key, take;   // position: the first `take` logits of `key` in id order
+        uint32_t of, cnt;     // logits of the key, and up to the position
+        uint64_t mass;        // mass up to the position
     };
     // Wave 0, inside block b: the first key at which the cumulative count
     // (mode 0: >= target) or mass (1: >= target, 2: > target) is reached, with
@@ -971,10 +985,14 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     // to the block's start.
     auto fine_find = [&](uint32_t b, int mode, uint64_t target, uint32_t lim_key, uint32_t lim_take) -> Fine {
         const uint32_t k = 32u * b + 31u - uint32_t(lane & 31);
-        uint32_t c = block_key_count(b);
+        const uint32_t of = block_key_count(b);
+        const uint64_t ma = mab[b];
+        const uint32_t ca = cab[b];
+        uint32_t c = of;
         if (k < lim_key) c = 0u;
         else if (k == lim_key) c = min(c, lim_take);
-        const uint64_t m = c ? fixed_mass(c, key_weight<DT>(k, inv_t, z0)) : 0ull;
+        const double w = c ? key_weight<DT>(k, inv_t, z0) : 0.0;
+        const uint64_t m = c ? fixed_mass(c, w) : 0ull;
         const uint64_t mi = wave_incl_scan_u64(m);
         const uint32_t ci = wave_incl_scan_u32(c);
         const uint64_t me = mi - m;
@@ -986,13 +1004,11 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
                 hit = uint64_t(ci) >= target;
                 if (hit) take = uint32_t(target - cexcl);
             } else {
-                const double unit = double(m) / double(c);   // one logit's mass
-                if (mode == 1) {
-                    hit = mi >= target;
-                    if (hit) take = uint32_t(ceil(double(target - me) / unit));
-                } else {
-                    hit = mi > target;
-                    if (hit) take = uint32_t(floor(double(target - me) / unit)) + 1u;
+                // (m / c: one logit's mass)
+                hit = mode == 1 ? mi >= target : mi > target;
+                if (hit) {
+                    const double x = double(target - me) * double(c) / double(m);
+                    take = mode == 1 ? uint32_t(ceil(x)) : uint32_t(floor(x)) + 1u;
                 }
             }
             take = min(max(take, 1u), c);
@@ -1004,14 +1020,19 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             f.found = true;
             f.key = 32u * b + 31u - uint32_t(L);
             f.take = readlane_u(take, L);
+            f.of = readlane_u(of, L);
+            f.cnt = ca + readlane_u(cexcl + take, L);
+            f.mass = ma + readlane_u64(me + (take ? fixed_mass(take, w) : 0ull), L);
         }
         return f;
     };
     // Wave 0: mass and count of the support through position (key, take).
-    auto mass_through = [&](uint32_t key, uint32_t take, uint64_t* mass, uint32_t* cnt) {
+    // (of: logits of the key)
+    auto mass_through = [&](uint32_t key, uint32_t take, uint64_t* mass, uint32_t* cnt, uint32_t* of) {
         const uint32_t b = key >> 5;
         const uint32_t k = 32u * b + 31u - uint32_t(lane & 31);
         uint32_t c = block_key_count(b);
+        *of = readlane_u(c, 31 - int(key & 31u));
         if (k < key) c = 0u;
         else if (k == key) c = min(c, take);
         const uint64_t m = c ? fixed_mass(c, key_weight<DT>(k, inv_t, z0)) : 0ull;
@@ -1024,16 +1045,14 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     if (wave == 0) {
         const bool has_cap = p.top_k > 0 && uint32_t(p.top_k) < N;
         uint32_t cap_key = 0u, cap_take = kTakeAll;
+        Fine cap{}, topp{};
         double s_cap = double(Mtot);
         if (has_cap) {
             const int b = block_search(0, uint64_t(p.top_k));
-            const Fine f = fine_find(uint32_t(b), 0, uint64_t(p.top_k) - cab[b], 0u, kTakeAll);
-            uint64_t m;
-            uint32_t c;
-            mass_through(f.key, f.take, &m, &c);
-            cap_key = f.key;
-            cap_take = f.take;
-            s_cap = double(m);
+            cap = fine_find(uint32_t(b), 0, uint64_t(p.top_k) - cab[b], 0u, kTakeAll);
+            cap_key = cap.key;
+            cap_take = cap.take;
+            s_cap = double(cap.mass);
         }
         // min-p: the lowest key whose weight reaches min_p
         uint32_t minp_key = 0u;
@@ -1044,36 +1063,36 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             }));
         }
         // top-p: the first position whose cumulative mass reaches top_p of the cap's
-        bool has_topp = false;
-        uint32_t topp_key = 0u, topp_take = kTakeAll;
         if (p.top_p < 1.0f) {
             const uint64_t target = uint64_t(llrint(double(p.top_p) * s_cap));
             const int b = block_search(1, target);
             const int lowest = has_cap ? int(cap_key >> 5) : 0;
             if (b >= lowest) {
                 const bool in_cap = has_cap && uint32_t(b) == (cap_key >> 5);
-                const Fine f = fine_find(uint32_t(b), 1, target - mab[b], in_cap ? cap_key : 0u,
-                                         in_cap ? cap_take : kTakeAll);
-                has_topp = f.found;
-                topp_key = f.key;
-                topp_take = f.take;
+                topp = fine_find(uint32_t(b), 1, target - mab[b], in_cap ? cap_key : 0u, in_cap ? cap_take : kTakeAll);
             }
         }
         // the support's end, its mass, the uniform and the draw's target
-        bool all = true;
+        bool all = true, known = false, cuts = false;   // (known: its mass and count; cuts: it cuts its last key's logits)
         uint32_t ek = 0u, et = kTakeAll;
-        auto consider = [&](uint32_t k, uint32_t t) {
-            if (all || k > ek || (k == ek && t < et)) { ek = k; et = t; all = false; }
-        };
-        if (has_cap) consider(cap_key, cap_take);
-        if (p.min_p > 0.0f) consider(minp_key, kTakeAll);
-        if (has_topp) consider(topp_key, topp_take);
-        if (!all && ek > z0key) { ek = z0key; et = 1u; }   // no logit passes min-p: the best one
         uint64_t sm = Mtot;
         uint32_t sc = N;
-        if (!all) mass_through(ek, et, &sm, &sc);
+        auto consider = [&](uint32_t k, uint32_t t, const Fine& f) {
+            if (!(all || k > ek || (k == ek && t < et))) return;
+            ek = k; et = t; all = false;
+            known = f.found; cuts = f.found && t < f.of; sm = f.mass; sc = f.cnt;
+        };
+        if (has_cap) consider(cap_key, cap_take, cap);
+        if (p.min_p > 0.0f) consider(minp_key, kTakeAll, Fine{});
+        if (topp.found) consider(topp.key, topp.take, topp);
+        if (!all && ek > z0key) { ek = z0key; et = 1u; known = false; }   // no logit passes min-p: the best one
+        if (!all && !known) {
+            uint32_t of;
+            mass_through(ek, et, &sm, &sc, &of);
+            cuts = et < of;
+        }
         const bool draw = a.draw_every > 0 && (a.row0 + row) % a.draw_every == a.draw_every - 1;
-        const double u = philox_uniform(p.seed, p.lane, p.position, 0u);
+        const double u = sh.u;
         const double target_d = u * double(sm);
         // the draw: the first support logit whose inclusive mass exceeds u * S_n
         const uint64_t t = uint64_t(target_d);
@@ -1105,18 +1124,11 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
                 }
             }
         }
-        // does the support cut its last key's logits?
-        bool cuts = false;
-        if (a.bounds && !all && et != kTakeAll) {
-            const uint32_t c = block_key_count(ek >> 5);
-            cuts = et < readlane_u(c, 31 - int(ek & 31u));
-        }
         if (lane == 0) {
             sh.s_n = double(sm);
             sh.n_support = sc;
-            sh.u = u;
             sh.end_key = all ? 0u : ek;
-            sh.want[0] = cuts ? 1u : 0u;
+            sh.want[0] = a.bounds && cuts ? 1u : 0u;
             sh.key[0] = ek;
             sh.rank[0] = et - 1u;
             sh.id[0] = 0x7fffffff;
@@ -1170,7 +1182,7 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             if (lane == 0) { sh.lo1 = lo; sh.hi1 = hi; }
         }
         for (int i = tid; i < 2048; i += kT) flip[i] = 0u;
-        if (tid == 0) sh.nflip = 0u;
+        if (tid == 0) { sh.nflip = 0u; sh.nown = 0u; }
         // presence masks by byte for the rescan, in the decisions' running-sum
         // table (free now): entry b, word q: the halves of tokens 2q and 2q + 1 all
         // ones where that token is in the history
@@ -1203,15 +1215,31 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             uint32_t bb[8];
 #pragma unroll
             for (int k = 0; k < 8; ++k) load_vec(k * kT + tid, &vv[k], &bb[k]);
-            // the owner part's repeat entries' logits, requested behind the part
-            // (their flips are worked out after the count, which they correct)
+            // The owner part's repeat entries gathered into a list (the other parts'
+            // would leave most lanes idle below), their logits requested behind the
+            // part (their flips are worked out after the count, which they correct)
             auto in_owner = [&](uint2 e) { return e.y >= 2u && int(e.x) >= it.s0 && int(e.x) < it.s0 + it.n; };
-            uint32_t raw[2] = {0u, 0u};
-            if (pen) {
+            uint2* own = reinterpret_cast<uint2*>(lds + kOffMKeys);
+            static_assert(16 * 16 * kSlotCap >= 2 * kT * sizeof(uint2), "repeat entries");
+            uint2 oe[2] = {make_uint2(0u, 0u), make_uint2(0u, 0u)};
+            uint32_t raw[2] = {0u, 0u}, nown = 0u;
+            if (pen && pv.nrep) {   // (uniform)
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    if (uint32_t(j * kT + tid) >= pv.nrep) rep[j].y = 0u;
-                    if (in_owner(rep[j])) raw[j] = uint32_t(row16[rep[j].x]);
+                    const bool mine = uint32_t(j * kT + tid) < pv.nrep && in_owner(rep[j]);
+                    const uint64_t m = ballot(mine);
+                    uint32_t at = 0u;
+                    if (lane == 0 && m) at = atomicAdd(&sh.nown, uint32_t(__builtin_popcountll(m)));
+                    at = readlane_u(at, 0) + uint32_t(__builtin_popcountll(m & ((1ull << lane) - 1ull)));
+                    if (mine) own[at] = rep[j];
+                }
+                lds_barrier();
+                nown = readlane_u(sh.nown, 0);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    if (uint32_t(j * kT + tid) >= nown) continue;
+                    oe[j] = own[j * kT + tid];
+                    raw[j] = uint32_t(row16[oe[j].x]);
                 }
             }
             const uint4* pmask = reinterpret_cast<const uint4*>(lds + kOffMCab);
@@ -1254,20 +1282,24 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
                 pc[r / 3] += c << (10 * (r % 3));
             }
             auto field = [](uint32_t w, int r) { return (w >> (10 * (r % 3))) & 0x3ffu; };
+            // exact match of a 16-bit pattern (the scalar form of the count)
+            auto match_one = [&](uint32_t pat, uint32_t present) -> uint32_t {
+                const uint32_t k = (pat & 0x8000u) ? (~pat & 0xffffu) : (pat | 0x8000u);
+                return (present ? !empty1 && k - a1 <= w1 : k - a0 <= w0) ? 1u : 0u;
+            };
             // Repeated tokens whose count changes the answer are flipped
             if (pen) {
                 auto flip_if = [&](uint2 e, uint32_t rw) {
                     if (!in_owner(e) || !Elem<DT>::finite_bits(rw)) return;
-                    const bool m1 = key16(pen_pattern<DT>(rw, 1u, p, inv_r, rep_fast)) == dk;
-                    const bool mc = key16(pen_pattern<DT>(rw, e.y, p, inv_r, rep_fast)) == dk;
-                    if (m1 != mc) {
+                    const uint32_t mc = key16(pen_pattern<DT>(rw, e.y, p, inv_r, rep_fast)) == dk ? 1u : 0u;
+                    if (match_one(rw, 1u) != mc) {
                         const uint32_t off = e.x - uint32_t(it.s0);
                         atomicOr(&flip[off >> 5], 1u << (off & 31u));
                         atomicAdd(&sh.nflip, 1u);
                     }
                 };
-#pragma unroll
-                for (int j = 0; j < 2; ++j) flip_if(rep[j], raw[j]);
+#pragma unroll 1
+                for (uint32_t j = 0; j < 2u && j * kT < nown; ++j) flip_if(j ? oe[1] : oe[0], j ? raw[1] : raw[0]);   // (uniform)
                 for (uint32_t i = uint32_t(2 * kT + tid); i < pv.nrep; i += kT) {   // (long repeat lists)
                     const uint2 e = pv.list[i];
                     if (in_owner(e)) flip_if(e, uint32_t(row16[e.x]));
@@ -1275,19 +1307,13 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             }
             lds_barrier();
             const bool flips = sh.nflip != 0u;
-            // exact match bits of one vector (the scalar form of the count, flips applied)
-            auto match_bits = [&](uint4 d, uint32_t b, int v) -> uint32_t {
+            auto match_bits = [&](uint4 d, uint32_t b, int v) -> uint32_t {   // (of a vector, flips applied)
                 const uint32_t w4[4] = {d.x, d.y, d.z, d.w};
                 uint32_t m = 0u;
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint32_t pat = (j & 1) ? (w4[j >> 1] >> 16) : (w4[j >> 1] & 0xffffu);
-                    const uint32_t k = (pat & 0x8000u) ? (~pat & 0xffffu) : (pat | 0x8000u);
-                    const bool present = (b >> j) & 1u;
-                    const bool hit = present ? (!empty1 && k - a1 <= w1) : (k - a0 <= w0);
-                    m |= hit ? (1u << j) : 0u;
-                }
-                if (flips && v >= 0) m ^= (flip[v >> 2] >> ((v & 3) * 8)) & 0xffu;
+                for (int j = 0; j < 8; ++j)
+                    m |= match_one((j & 1) ? w4[j >> 1] >> 16 : w4[j >> 1] & 0xffffu, (b >> j) & 1u) << j;
+                if (flips) m ^= (flip[v >> 2] >> ((v & 3) * 8)) & 0xffu;
                 return m;
             };
             if (flips) {   // (uniform) the flipped vectors counted again
@@ -1318,23 +1344,27 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             }
             lds_barrier();
             const uint32_t want = sh.orank;
+            // the vector holding the rank, then its logit
+            uint4 hv = make_uint4(0u, 0u, 0u, 0u);
+            uint32_t hb = 0u, he = 0u;
+            int at = -1;
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 const uint32_t c = field(pc[r / 3], r);
                 const uint32_t e = sh.wtot[r][wave] + field(pin[r / 3], r) - c;
-                if (c && want >= e && want < e + c) {
-                    const int v = r * kT + tid;
-                    uint32_t m = match_bits(vv[r], bb[r], v);
-                    for (uint32_t k = want - e; k > 0u; --k) m &= m - 1u;
-                    sh.id[which] = it.s0 + 8 * v + __builtin_ctz(m);
-                }
+                if (c && want >= e && want < e + c) { at = r * kT + tid; hv = vv[r]; hb = bb[r]; he = e; }
+            }
+            if (at >= 0) {
+                uint32_t m = match_bits(hv, hb, at);
+                for (uint32_t k = want - he; k > 0u; --k) m &= m - 1u;
+                sh.id[which] = it.s0 + 8 * at + __builtin_ctz(m);
             }
             if ((it.n & 7) && wave == kW - 1) {   // (uniform) the logits past the last vector: behind every vector
                 const uint32_t body = sh.wtot[7][kW - 1] + uint32_t(__builtin_amdgcn_readlane(int(field(pin[2], 7)), kWave - 1));
                 const bool in = lane < (it.n & 7);
                 const int off = 8 * it.nvec + min(lane, (it.n & 7) - 1);
                 const uint32_t tb = pb ? uint32_t(pb[it.nvec]) : 0u, raw = uint32_t(row16[it.s0 + off]);
-                const uint32_t one = match_bits(make_uint4(raw, 0u, 0u, 0u), (tb >> (off & 7)) & 1u, -1) & 1u;
+                const uint32_t one = match_one(raw, (tb >> (off & 7)) & 1u);
                 const bool hit = in && (one ^ (flips ? (flip[off >> 5] >> (off & 31)) & 1u : 0u));
                 const uint64_t m = ballot(hit);
                 const uint32_t before = uint32_t(__builtin_popcountll(m & ((1ull << lane) - 1ull)));
@@ -1401,11 +1431,14 @@ struct HistArgs {
     uint32_t* hhead;   // [rows][2]
     uint32_t* tmp;     // [rows][2 words + cap] (the workspace form)
 };
-constexpr int kHistBatch = 32;   // history tokens per thread held in registers
+// History tokens per thread held in registers: 4 where that covers the longest
+// history, else 32.  (A batch's steps are issued whatever part of it holds
+// tokens: 24 rows of 2,048-token histories over 151,936 tokens take 7.4 us with 4, 12.9 with 32.)
+constexpr int kHistShort = 4, kHistLong = 32;
 
 constexpr int kHistLdsWords = 40896;   // B1 + B2 + counts (160 KB less the scalars)
 
-template <bool LDS>
+template <bool LDS, int kHistBatch>
 __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
     __shared__ __attribute__((aligned(16))) uint32_t lds[LDS ? kHistLdsWords : 1];
     const int row = blockIdx.x, tid = threadIdx.x;
@@ -1425,14 +1458,11 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
     };
     __shared__ uint32_t flags, nrep, scan[kW + 1];
     const int64_t b = h.offsets[row], e = h.offsets[row + 1];
-    for (int i = tid; i < 2 * W; i += kT) put(&hl[i], 0u);
-    if (tid == 0) flags = 0u;
-    sync();
     const int V = h.vocabulary;
-    // The history in batches of kHistBatch tokens per thread (one batch for
-    // up to 32,768 tokens, kept in registers for the second pass).  Each pass
-    // issues a batch's LDS operations back to back and uses their results
-    // after, so their latencies overlap.
+    // The history in batches of kHistBatch tokens per thread (one batch: kept in
+    // registers for the second pass; the first is requested before the LDS is
+    // cleared).  Each pass issues a batch's LDS operations back to back and uses
+    // their results after, so their latencies overlap.
     const bool one_batch = e - b <= int64_t(kHistBatch) * kT;
     int32_t t[kHistBatch];
     auto load = [&](int64_t base) {
@@ -1442,8 +1472,12 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
             t[j] = i < e ? h.histories[i] : -2;   // (-2: past the end)
         }
     };
+    load(b);
+    for (int i = tid; i < 2 * W; i += kT) put(&hl[i], 0u);
+    if (tid == 0) flags = 0u;
+    sync();
     for (int64_t base = b; base < e; base += int64_t(kHistBatch) * kT) {
-        load(base);
+        if (base != b) load(base);
 #pragma unroll
         for (int j0 = 0; j0 < kHistBatch; j0 += kHistBatch / 2) {
             uint32_t old[kHistBatch / 2];
@@ -1737,8 +1771,10 @@ vi_status launch_stream(const SampleArgs& s, unsigned char* ws, size_t ws_bytes,
     }
     if (!c.ok) return VI_ERR_WORKSPACE;
     if (hist) {
-        if (h.tmp) hipLaunchKernelGGL(history_view_kernel<false>, dim3(s.rows), dim3(kT), 0, stream, h);
-        else hipLaunchKernelGGL(history_view_kernel<true>, dim3(s.rows), dim3(kT), 0, stream, h);
+        const dim3 rows(s.rows), block(kT);
+        if (h.tmp) hipLaunchKernelGGL((history_view_kernel<false, kHistLong>), rows, block, 0, stream, h);
+        else if (s.max_history <= kHistShort * kT) hipLaunchKernelGGL((history_view_kernel<true, kHistShort>), rows, block, 0, stream, h);
+        else hipLaunchKernelGGL((history_view_kernel<true, kHistLong>), rows, block, 0, stream, h);
         if (launch_status() != VI_OK) return VI_ERR_LAUNCH;
     }
     for (int r0 = 0; r0 < s.rows; r0 += chunk) {
