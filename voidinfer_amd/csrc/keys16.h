@@ -16,7 +16,9 @@ __device__ __forceinline__ float key_z(uint32_t key, float inv_t) {
 }
 
 // Smallest i in [lo, hi) with pred(i) (pred monotone false -> true), or hi.
-// Wave-uniform call; 64 probes per round.
+// Wave-uniform call; 64 probes per round, an odd number of places apart (probes of
+// a table in LDS then spread over its banks; every 64th of 4,096 doubles lies in
+// one bank).
 template <class P>
 __device__ __forceinline__ int wave_search(int lo, int hi, P pred) {
     const int lane = lane_id();
@@ -26,7 +28,7 @@ __device__ __forceinline__ int wave_search(int lo, int hi, P pred) {
             const uint64_t m = ballot(lane < n && pred(lo + lane));
             return m ? lo + __builtin_ctzll(m) : hi;
         }
-        const int step = (n + kWave - 1) / kWave;
+        const int step = ((n + kWave - 1) / kWave) | 1;
         const int p = lo + lane * step;
         const uint64_t valid = ballot(p < hi);
         const uint64_t m = ballot(p < hi && pred(p));

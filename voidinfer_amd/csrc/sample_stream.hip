@@ -1552,13 +1552,15 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
 // The filtered distribution of each row: exp(z - z0) / S_n on the support, 0
 // elsewhere.  Bound by the memory: 2 bytes read and 4 written per logit.  Four
 // consecutive logits per lane and round (8-byte loads and 16-byte stores, whole
-// lines per wave), every round's loads requested first; a history token is
-// penalized with count 1, and the tokens seen more than once are written again
-// by repeat_probs_kernel.  (24 x 151,936 bf16: 16.4 us and 4.5 for the repeats;
-// 48.6 with eight logits per thread, each slice's penalties rebuilt in LDS and
-// end-key ranks counted.)
+// lines per wave), every round's loads requested first.  A wave's history tokens
+// are listed over all its rounds and penalized one per lane with count 1 (where
+// they lie, nearly every wave would run the penalty for nearly every logit of a
+// lane); the tokens seen more than once are written again by repeat_probs_kernel.
+// (24 / 128 x 151,936 bf16, 2,048-token histories: 11.7 / 38.3 us with two rounds,
+// 11.0 / 40.5 with one, 14.0 / 40.4 with four, and 3.9 / 4.8 for the repeats; 24 rows took 48.6 us with eight logits per thread, each slice's
+// penalties rebuilt in LDS and end-key ranks counted.)
 constexpr int kPT = 256;                          // threads
-constexpr int kPRounds = 4;
+constexpr int kPRounds = 2;
 constexpr int kPChunk = kPT * kPRounds * 4;       // logits per workgroup
 
 // p of a logit with (penalized) pattern pat
@@ -1567,7 +1569,7 @@ __device__ __forceinline__ float pattern_prob(uint32_t pat, int id, const FullBo
     const uint32_t k = key16(pat);
     const float z = Elem<DT>::decode(unkey16(k)) * B.inv_t;
     const bool in = Elem<DT>::finite_bits(pat) && isfinite(z) && (k > B.end_key || (k == B.end_key && id <= B.end_id));
-    return in ? float(exp(double(z) - B.z0) * inv_s) : 0.0f;
+    return in ? float(exp_neg(double(z) - B.z0) * inv_s) : 0.0f;
 }
 
 template <int DT>
@@ -1576,7 +1578,9 @@ __global__ __launch_bounds__(kPT) void probs_kernel(StreamArgs a) {
     typedef u32x2_t u32x2_any_t __attribute__((aligned(2)));
     typedef float f32x4_t __attribute__((ext_vector_type(4)));
     typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
-    const int row = blockIdx.y, V = a.vocabulary;
+    __shared__ __attribute__((aligned(16))) u32x2_t stage_all[kPT / kWave][kPRounds * kWave];
+    __shared__ uint16_t list_all[kPT / kWave][kPRounds * kWave * 4];
+    const int row = blockIdx.y, V = a.vocabulary, lane = lane_id(), wave = int(threadIdx.x) / kWave;
     const vi_row_params p = a.params[row];
     if (!stream_row(p)) return;
     const FullBound B = a.bounds[row];
@@ -1598,21 +1602,49 @@ __global__ __launch_bounds__(kPT) void probs_kernel(StreamArgs a) {
     const float inv_r = rep_inverse(p);
     const bool rep_fast = rep_fast_ok(p);
     const double inv_s = B.valid ? 1.0 / B.s_n : 0.0;
-    auto prob = [&](uint32_t raw, uint32_t present, int id) {
-        if (present) raw = pen_pattern<DT>(raw, 1u, p, inv_r, rep_fast);
-        return B.valid ? pattern_prob<DT>(raw, id, B, inv_s) : 0.0f;
-    };
+    if (pv.pen && B.valid) {   // (uniform)
+        u32x2_t* stage = stage_all[wave];
+        uint16_t* stage16 = reinterpret_cast<uint16_t*>(stage);
+        uint16_t* list = list_all[wave];
+        uint32_t m = 0u;   // bit 4 r + j: logit j of round r
+#pragma unroll
+        for (int r = 0; r < kPRounds; ++r) {
+            if (i0 + r * 4 * kPT + 4 <= V) m |= b[r] << (4 * r);
+            stage[r * kWave + lane] = v[r];
+        }
+        const uint32_t n = uint32_t(__builtin_popcount(m)), incl = wave_incl_scan_u32(n), N = readlane_u(incl, kWave - 1);
+        uint32_t pos = incl - n;
+        while (m) {
+            const uint32_t t = uint32_t(__builtin_ctz(m));
+            list[pos++] = uint16_t((t >> 2) * (4 * kWave) + 4u * uint32_t(lane) + (t & 3u));
+            m &= m - 1u;
+        }
+        wave_lds_fence();
+        for (uint32_t q = uint32_t(lane); q < N; q += kWave) {
+            const uint32_t off = list[q];
+            stage16[off] = uint16_t(pen_pattern<DT>(stage16[off], 1u, p, inv_r, rep_fast));
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int r = 0; r < kPRounds; ++r) v[r] = stage[r * kWave + lane];
+    }
 #pragma unroll
     for (int r = 0; r < kPRounds; ++r) {
         const int i = i0 + r * 4 * kPT;
         if (i + 4 <= V) {
-            f32x4_t q;
+            f32x4_t q = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (B.valid) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                q[j] = prob((j & 1) ? v[r][j >> 1] >> 16 : v[r][j >> 1] & 0xffffu, (b[r] >> j) & 1u, i + j);
+                for (int j = 0; j < 4; ++j)
+                    q[j] = pattern_prob<DT>((j & 1) ? v[r][j >> 1] >> 16 : v[r][j >> 1] & 0xffffu, i + j, B, inv_s);
+            }
             *reinterpret_cast<f32x4_any_t*>(out + i) = q;
         } else {   // (up to three logits past the row's last four)
-            for (int j = i; j < V; ++j) out[j] = prob(uint32_t(row16[j]), (b[r] >> (j - i)) & 1u, j);
+            for (int j = i; j < V; ++j) {
+                uint32_t raw = uint32_t(row16[j]);
+                if ((b[r] >> (j - i)) & 1u) raw = pen_pattern<DT>(raw, 1u, p, inv_r, rep_fast);
+                out[j] = B.valid ? pattern_prob<DT>(raw, j, B, inv_s) : 0.0f;
+            }
         }
     }
 }

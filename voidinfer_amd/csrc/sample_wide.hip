@@ -229,37 +229,60 @@ __device__ __forceinline__ float logit_z(const WPen& w, const vi_row_params& p, 
 }
 
 // The history route's presence bitmap and count hash of each full-route row
-// with penalties (the top-k route builds its own rows' hashes).
-__global__ __launch_bounds__(256) void wide_history_kernel(WideArgs a) {
-    const int r = blockIdx.x;
+// with penalties (the top-k route builds its own rows' hashes), both in LDS and
+// copied out; a table past kHistLdsSlots is built in place.  Bound by the chain of
+// compare-and-swap round trips: 23 rows of 739 tokens over 151,936 take 12.6 us with
+// 256 threads and every atomic in global memory.
+constexpr int kHistLdsSlots = 8192;
+constexpr int kHistWords = kMaxSlices * kSL / 32;
+__global__ __launch_bounds__(kT) void wide_history_kernel(WideArgs a) {
+    __shared__ uint2 s_table[kHistLdsSlots];
+    __shared__ uint32_t s_bits[kHistWords];
+    __shared__ uint32_t s_flags;
+    const int r = blockIdx.x, tid = threadIdx.x;
     const vi_row_params p = a.params[r];
     if (!full_row(p) || !penalties_active(p)) return;
     const int64_t b = a.offsets[r], n = a.offsets[r + 1] - b;
     if (n <= 0) return;
-    __shared__ uint32_t s_flags;
-    if (threadIdx.x == 0) s_flags = 0u;
     uint32_t* bits = a.hbits + size_t(r) * size_t(a.words);
-    uint2* table = a.hash + size_t(r) * size_t(a.hash_slots);
-    for (int i = threadIdx.x; i < a.words; i += blockDim.x) bits[i] = 0u;
-    for (int i = threadIdx.x; i < a.hash_slots; i += blockDim.x) table[i] = make_uint2(0u, 0u);
-    __syncthreads();
-    if (n > a.max_history) {
-        if (threadIdx.x == 0) s_flags = VI_FLAG_ERROR;
-    } else {
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-            const int32_t t = a.histories[b + i];
-            if (t < 0 || t >= a.vocabulary) { atomicOr(&s_flags, uint32_t(VI_FLAG_BAD_HISTORY)); continue; }
-            uint32_t s = (uint32_t(t) * 0x9E3779B1u) >> a.hash_shift;
-            for (int probe = 0; probe < a.hash_slots; ++probe) {
-                const uint32_t old = atomicCAS(&table[s].x, 0u, uint32_t(t) + 1u);
-                if (old == 0u || old == uint32_t(t) + 1u) { atomicAdd(&table[s].y, 1u); break; }
-                s = (s + 1u) & uint32_t(a.hash_slots - 1);
-            }
-            atomicOr(&bits[t >> 5], 1u << (t & 31));
+    uint2* out = a.hash + size_t(r) * size_t(a.hash_slots);
+    const bool in_lds = a.hash_slots <= kHistLdsSlots;
+    auto build = [&](uint2* table) {
+        for (int i = tid; i < a.hash_slots; i += kT) table[i] = make_uint2(0u, 0u);
+        __syncthreads();
+        if (n > a.max_history) {
+            if (tid == 0) s_flags = VI_FLAG_ERROR;
+            return;
         }
-    }
+        constexpr int kU = 4;   // (the history loads of a round issued together)
+        for (int64_t i0 = 0; i0 < n; i0 += int64_t(kU) * kT) {
+            int32_t tk[kU];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) tk[u] = a.histories[b + min(i0 + int64_t(u) * kT + tid, n - 1)];
+#pragma unroll
+            for (int u = 0; u < kU; ++u) {
+                if (i0 + int64_t(u) * kT + tid >= n) continue;
+                const int32_t t = tk[u];
+                if (t < 0 || t >= a.vocabulary) { atomicOr(&s_flags, uint32_t(VI_FLAG_BAD_HISTORY)); continue; }
+                atomicOr(&s_bits[t >> 5], 1u << (t & 31));
+                uint32_t s = (uint32_t(t) * 0x9E3779B1u) >> a.hash_shift;
+                for (int probe = 0; probe < a.hash_slots; ++probe) {
+                    const uint32_t old = atomicCAS(&table[s].x, 0u, uint32_t(t) + 1u);
+                    if (old == 0u || old == uint32_t(t) + 1u) { atomicAdd(&table[s].y, 1u); break; }
+                    s = (s + 1u) & uint32_t(a.hash_slots - 1);
+                }
+            }
+        }
+    };
+    if (tid == 0) s_flags = 0u;
+    for (int i = tid; i < a.words; i += kT) s_bits[i] = 0u;
+    if (in_lds) build(s_table);
+    else build(out);
     __syncthreads();
-    if (threadIdx.x == 0) a.row_flags[r] = s_flags;
+    for (int i = tid; i < a.words; i += kT) bits[i] = s_bits[i];
+    if (in_lds)
+        for (int i = tid; i < a.hash_slots; i += kT) out[i] = s_table[i];
+    if (tid == 0) a.row_flags[r] = s_flags;
 }
 
 struct WGeo {
@@ -1369,56 +1392,43 @@ __global__ __launch_bounds__(kT) void wide_finish_kernel(WideArgs a) {
 }
 
 // Filtered distribution of the full-route rows: exp(z - z0) / S_n on the support,
-// 0 elsewhere.  Bound by the memory (4 bytes read and 4 written per logit): four
-// consecutive logits per lane and round, every round's loads requested first
-// (23 x 151,936, 739-token histories: 17.6 us; 33 with sixteen consecutive
-// logits per thread and end-key ranks counted).
-constexpr int kPT = 256;                          // threads
-constexpr int kPRounds = 4;
-constexpr int kPChunk = kPT * kPRounds * 4;       // logits per workgroup
+// 0 elsewhere.  Bound by the memory (4 bytes read and 4 written per logit) and, for
+// few rows, by one pass' latency: four consecutive logits per lane and one round
+// per thread (23 x 151,936, 739-token histories: 11.4 us, 18.7 with four rounds; 128
+// rows: 45.4 and 51.0).
+constexpr int kPT = 256;              // threads
+constexpr int kPChunk = 4 * kPT;      // logits per workgroup
 __global__ __launch_bounds__(kPT) void wide_probs_kernel(WideArgs a) {
     typedef float f32x4_t __attribute__((ext_vector_type(4)));
     typedef f32x4_t f32x4_any_t __attribute__((aligned(4)));
-    const int row = blockIdx.y, V = a.vocabulary;
+    const int row = blockIdx.y, V = a.vocabulary, i = int(blockIdx.x) * kPChunk + 4 * int(threadIdx.x);
     const vi_row_params p = a.params[row];
-    if (!full_row(p)) return;
+    if (!full_row(p) || i >= V) return;
     const WideBound bd = a.bounds[row];
     const WPen w = wpen(a, row, p);
     const int unrec = a.record && a.pstate ? a.tokens[row] : -1;
     const uint32_t* base = static_cast<const uint32_t*>(a.logits) + int64_t(row) * a.stride;
     float* out = a.probs + size_t(row) * size_t(a.probs_stride);
-    const int i0 = int(blockIdx.x) * kPChunk + 4 * int(threadIdx.x);
-    uint4 v[kPRounds];
-    uint32_t word[kPRounds];   // the presence word of the round's four logits
-#pragma unroll
-    for (int r = 0; r < kPRounds; ++r) {
-        const int i = i0 + r * 4 * kPT;
-        v[r] = make_uint4(0u, 0u, 0u, 0u);
-        word[r] = 0u;
-        if (i + 4 <= V) v[r] = load16(base + i);
-        if (w.on && i < V) word[r] = w.bits[i >> 5];
-    }
+    const bool whole = i + 4 <= V;
+    const uint4 v = whole ? load16(base + i) : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t word = w.on ? w.bits[i >> 5] : 0u;   // (four logits share a presence word)
     const double inv_s = bd.valid ? 1.0 / bd.s_n : 0.0;
-    auto prob = [&](uint32_t bits, uint32_t wd, int id) {
+    auto prob = [&](uint32_t bits, int id) {
         bool bad = false;
-        const float z = logit_z(w, p, bd.inv_t, id, bits, wd, &bad, unrec);
+        const float z = logit_z(w, p, bd.inv_t, id, bits, word, &bad, unrec);
         const uint32_t k = isnan(z) ? 0u : key32(z);
         const bool in = bd.valid && k && (k > bd.end_key || (k == bd.end_key && id <= bd.end_id));
-        return in ? float(exp(double(z) - bd.z0) * inv_s) : 0.0f;
+        return in ? float(exp_neg(double(z) - bd.z0) * inv_s) : 0.0f;
     };
-#pragma unroll
-    for (int r = 0; r < kPRounds; ++r) {
-        const int i = i0 + r * 4 * kPT;
-        if (i + 4 <= V) {
-            f32x4_t q;
-            q[0] = prob(v[r].x, word[r], i);
-            q[1] = prob(v[r].y, word[r], i + 1);
-            q[2] = prob(v[r].z, word[r], i + 2);
-            q[3] = prob(v[r].w, word[r], i + 3);
-            *reinterpret_cast<f32x4_any_t*>(out + i) = q;
-        } else {   // (up to three logits past the row's last four)
-            for (int j = i; j < V; ++j) out[j] = prob(base[j], word[r], j);
-        }
+    if (whole) {
+        f32x4_t q;
+        q[0] = prob(v.x, i);
+        q[1] = prob(v.y, i + 1);
+        q[2] = prob(v.z, i + 2);
+        q[3] = prob(v.w, i + 3);
+        *reinterpret_cast<f32x4_any_t*>(out + i) = q;
+    } else {   // (up to three logits past the row's last four)
+        for (int j = i; j < V; ++j) out[j] = prob(base[j], j);
     }
 }
 
@@ -1472,7 +1482,7 @@ vi_status launch_wide(const SampleArgs& s, unsigned char* ws, size_t ws_bytes, u
     if (s.full_out) a.bounds = s.full_out->bounds;
     a.draw_every = s.full_out ? s.full_out->draw_every : 1;
     a.want_bounds = (s.probs || s.full_out) ? 1 : 0;
-    if (a.hash) hipLaunchKernelGGL(wide_history_kernel, dim3(s.rows), dim3(256), 0, stream, a);
+    if (a.hash) hipLaunchKernelGGL(wide_history_kernel, dim3(s.rows), dim3(kT), 0, stream, a);
     const bool pen = a.pstate || a.hash;
     const dim3 slices(a.slices, s.rows);
     if (pen) hipLaunchKernelGGL(wide_hist_kernel<true>, slices, dim3(kT), 0, stream, a);
