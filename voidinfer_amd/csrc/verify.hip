@@ -138,26 +138,11 @@ __device__ __forceinline__ double prob_at(const FullRows& R, size_t r, int x) {
     return in_support(k, x, B) ? exp(double(dist_z<DT>(k, B.inv_t)) - B.z0) / B.s_n : 0.0;
 }
 
-// The accept test of every (lane, position) of the full-vocabulary lanes:
+// The accept test of position j < drafts of a full-vocabulary lane:
 // u_a < min(1, p(d) / q(d)) with the target softmax p and the draft q at the
-// drafted token; position `drafts` takes the bonus row's draw.  A thread per
-// position.
+// drafted token.
 template <int TDT, int DDT>
-__global__ __launch_bounds__(kWave) void verify_full_accept_kernel(FullVerifyArgs a) {
-    const int l = blockIdx.y, j = int(blockIdx.x) * kWave + int(threadIdx.x);
-    if (j > a.drafts) return;
-    const vi_row_params p = a.params[l];
-    if (!verify_list_refused(p)) return;
-    PosDecision* out = a.dec + size_t(l) * (a.drafts + 1) + j;
-    if (j == a.drafts) {
-        if (a.target_rows != a.drafts + 1) return;
-        const size_t tr = size_t(l) * a.target_rows + j;
-        const uint32_t f = a.t.stats[tr].flags;
-        const int32_t tok = a.ttok[tr];
-        const bool bad = (f & VI_FLAG_ERROR) || tok < 0 || tok >= a.vocabulary;
-        *out = PosDecision{bad ? -1 : tok, (f & VI_FLAG_ERROR) ? uint32_t(VI_FLAG_ERROR) : 0u, 0, 0};
-        return;
-    }
+__device__ __forceinline__ PosDecision accept_test(const FullVerifyArgs& a, const vi_row_params& p, int l, int j) {
     const size_t tr = size_t(l) * a.target_rows + j, dr = size_t(l) * a.drafts + j;
     const int32_t x = a.drafted[dr];
     uint32_t flags = (a.t.stats[tr].flags | a.d.stats[dr].flags) &
@@ -172,18 +157,29 @@ __global__ __launch_bounds__(kWave) void verify_full_accept_kernel(FullVerifyArg
     if (q == 0.0) flags |= VI_FLAG_ZERO_Q;
     else acc = fmin(1.0, pv / q);
     const int accept = (!(flags & VI_FLAG_ERROR) && q != 0.0 && ua < acc) ? 1 : 0;
-    *out = PosDecision{-1, flags, accept, 0};
+    return PosDecision{-1, flags, accept, 0};
+}
+// The bonus row's decision: its draw.
+__device__ __forceinline__ PosDecision bonus_decision(const FullVerifyArgs& a, int l) {
+    const size_t tr = size_t(l) * a.target_rows + a.drafts;
+    const uint32_t f = a.t.stats[tr].flags;
+    const int32_t tok = a.ttok[tr];
+    const bool bad = (f & VI_FLAG_ERROR) || tok < 0 || tok >= a.vocabulary;
+    return PosDecision{bad ? -1 : tok, (f & VI_FLAG_ERROR) ? uint32_t(VI_FLAG_ERROR) : 0u, 0, 0};
 }
 
 // The lane's first rejected position before any accepted terminal token, or -1:
-// 64 positions per round, one per lane of the wave (every wave alike).
-__device__ int first_rejection(const FullVerifyArgs& a, int l) {
+// 64 positions per round, one per lane of the wave (every wave alike); load(j)
+// gives a position's decision.  Rounds past the one that holds the end are not
+// loaded (nor read by the chain, which ends there too).
+template <class Load>
+__device__ __forceinline__ int first_rejection(const FullVerifyArgs& a, int l, Load load) {
     const int lane = lane_id();
     for (int j0 = 0; j0 < a.drafts; j0 += kWave) {
         const int j = j0 + lane;
         bool ends = false, usable = false;
         if (j < a.drafts) {
-            const PosDecision e = a.dec[size_t(l) * (a.drafts + 1) + j];
+            const PosDecision e = load(j);
             ends = e.accept ? is_terminal(a.terminal, a.n_terminal, a.drafted[size_t(l) * a.drafts + j]) : true;
             usable = !e.accept && !(e.flags & VI_FLAG_ERROR);
         }
@@ -267,14 +263,27 @@ __device__ int block_max_i(int v, int* tmp) {
     return m;
 }
 
-// Residual and p mass of each range of each lane's rejected position.
+// The lane's accept tests, and the residual and p mass of each range of its
+// rejected position.  Every workgroup takes the tests itself, a position per
+// lane of its waves (two gathers and a few hundred instructions), and the first
+// range's writes them for the correction: a launch of their own before this one
+// cost more than their repetition (8 x 16 drafts, 248,320 tokens: 127.1 us per
+// call, 130.4 with it).
 template <int TDT, int DDT>
 __global__ __launch_bounds__(kRT) void verify_full_ranges_kernel(FullVerifyArgs a) {
     __shared__ double dtmp[kW];
     __shared__ int itmp[kW];
     const int rg = blockIdx.x, l = blockIdx.y;
-    if (!verify_list_refused(a.params[l])) return;
-    const int js = first_rejection(a, l);
+    const vi_row_params p = a.params[l];
+    if (!verify_list_refused(p)) return;
+    PosDecision* dec = a.dec + size_t(l) * (a.drafts + 1);
+    const bool writes = rg == 0 && threadIdx.x < kWave;
+    if (writes && threadIdx.x == 0 && a.target_rows == a.drafts + 1) dec[a.drafts] = bonus_decision(a, l);
+    const int js = first_rejection(a, l, [&](int j) {
+        const PosDecision e = accept_test<TDT, DDT>(a, p, l, j);
+        if (writes) dec[j] = e;
+        return e;
+    });
     if (js < 0) return;
     const size_t tr = size_t(l) * a.target_rows + js, dr = size_t(l) * a.drafts + js;
     const int r0 = rg * kRange, r1 = min(a.vocabulary, r0 + kRange);
@@ -311,7 +320,7 @@ __global__ __launch_bounds__(kRT) void verify_full_correction_kernel(FullVerifyA
     const int l = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
     const vi_row_params p = a.params[l];
     if (!verify_list_refused(p)) return;
-    const int js = first_rejection(a, l);
+    const int js = first_rejection(a, l, [&](int j) { return a.dec[size_t(l) * (a.drafts + 1) + j]; });
     if (tid == 0) { s_range = -1; s_tok = -1; s_nores = 0u; }
     __syncthreads();
     if (js >= 0 && wave == 0) {   // the ranges' sums, 64 at a time in id order
@@ -472,7 +481,6 @@ bool full_path_ok(const void* logits, int dtype, int vocabulary, int64_t stride)
 
 template <int TDT, int DDT>
 void launch_full_verify(const FullVerifyArgs& f, hipStream_t stream) {
-    hipLaunchKernelGGL((verify_full_accept_kernel<TDT, DDT>), dim3(f.drafts / kWave + 1, f.lanes), dim3(kWave), 0, stream, f);
     hipLaunchKernelGGL((verify_full_ranges_kernel<TDT, DDT>), dim3(f.ranges, f.lanes), dim3(kRT), 0, stream, f);
     hipLaunchKernelGGL((verify_full_correction_kernel<TDT, DDT>), dim3(f.lanes), dim3(kRT), 0, stream, f);
 }
@@ -586,7 +594,7 @@ vi_status launch_verify(const VerifyArgs& a, void* ws, size_t ws_bytes, hipStrea
     // the rows' filtered distributions (and the bonus rows' draws) from the
     // full-vocabulary sampler, each row set in its own workspace: the draft
     // rows on the side stream beside the target rows on the caller's, joined
-    // back before the accept launch
+    // back before the ranges launch
     auto sample = [&](const void* logits, int dtype, int rows, int64_t stride, const vi_row_params* par,
                       int32_t* tok, vi_sample_stats* stats, const FullOut* out, unsigned char* w, size_t wb,
                       hipStream_t on) {
