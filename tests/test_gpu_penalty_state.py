@@ -131,6 +131,33 @@ def test_state_error_flags(dev, rng):
     assert tok[1] == -1 and tok[2] == -1 and s["flags"][1] & FLAG_ERROR and s["flags"][2] & FLAG_ERROR
 
 
+@pytest.mark.parametrize("vocab", [5000, 5001])
+@pytest.mark.parametrize("want_probs", [False, True])
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_rows_without_penalties_ignore_the_lanes_failures(orc, dev, rng, dtype, want_probs, vocab):
+    """A row that takes no penalties is sampled as from a clean lane, whatever its
+    lane's state or history holds: an ERROR lane (table full), a BAD_HISTORY lane, a
+    history with tokens outside the vocabulary."""
+    import voidinfer_amd as vi
+    from test_gpu_sample import compare, make_rows, params, run_both
+    rows = 6
+    st = vi.PenaltyState(rows, vocab, 64, device=dev)
+    full, bad = list(range(100)), [1, -4, vocab + 3]
+    update(st, dev, [full, bad, full, bad, full, bad])
+    flags = st.header()[:, 0]
+    assert (flags[::2] & FLAG_ERROR).all() and (flags[1::2] == FLAG_BAD_HISTORY).all()
+    bits = make_rows(rng, rows, vocab, std=1.0, dtype=dtype)
+    p = params(rows, rng, temperature=0.9, top_k=np.array([0, 0, 100, 100, 20, 20]), top_p=0.9)
+    hist, offs = csr([bad] * rows)
+    g, w = run_both(orc, dev, bits, dtype, p, hist, offs, want_probs=want_probs)
+    assert (w["stats"]["flags"] == 0).all()
+    compare(g, w, p, "history")
+    out = vi.sample_rows_state(to_dev(bits, dtype, dev), p, st, want_probs=want_probs)
+    torch.cuda.synchronize()
+    compare(dict(tokens=out.tokens.cpu().numpy(), u=out.uniforms.cpu().numpy(), stats=vi.stats_numpy(out.stats),
+                 probs=out.probs.cpu().numpy() if want_probs else None), w, p, "state")
+
+
 def same_outputs(a, b, label):
     import voidinfer_amd as vi
     assert torch.equal(a.tokens, b.tokens), label

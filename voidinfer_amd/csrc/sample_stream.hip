@@ -231,6 +231,8 @@ __device__ __forceinline__ Item item_at(const StreamArgs& a, int x, int q) {
 }
 __device__ __forceinline__ bool stream_row(const vi_row_params& p) { return !topk_route(p); }
 
+// A row's penalty inputs.  flags: the failures of the lane's state or history,
+// which concern only the rows that take penalties from it (none without `pen`).
 struct PenView {
     const unsigned char* b1;
     const uint2* list;
@@ -245,14 +247,14 @@ __device__ __forceinline__ PenView pen_view(const StreamArgs& a, int row, const 
         v.b1 = st + a.pl.off_b1;
         v.list = reinterpret_cast<const uint2*>(st + a.pl.off_list);
         v.nrep = min(h->nrep, uint32_t(a.pl.slots));
-        v.flags = h->flags & (VI_FLAG_BAD_HISTORY | VI_FLAG_ERROR);
         v.pen = penalties_active(p);
+        v.flags = v.pen ? h->flags & (VI_FLAG_BAD_HISTORY | VI_FLAG_ERROR) : 0u;
     } else if (a.hb1) {
         v.b1 = reinterpret_cast<const unsigned char*>(a.hb1 + size_t(row) * a.hwords);
         v.list = a.hlist + size_t(row) * a.hcap;
         v.nrep = a.hhead[2 * row];
-        v.flags = a.hhead[2 * row + 1];
         v.pen = penalties_active(p);
+        v.flags = v.pen ? a.hhead[2 * row + 1] : 0u;
     }
     return v;
 }
