@@ -138,6 +138,24 @@ def test_stream_bad_history_tokens_flagged(orc, dev, rng):
     assert (g["stats"]["flags"][0] & 16) and (g["stats"]["flags"][2] & 16)
 
 
+@pytest.mark.parametrize("want_probs", [False, True])
+@pytest.mark.parametrize("vocab,length", [(5_000, 100), (5_001, 100), (5_001, 5_000), (500_001, 24_000)])
+def test_stream_every_bad_history_token_is_flagged(orc, dev, rng, vocab, length, want_probs):
+    """One token outside the vocabulary per row, among valid ones: -1, -2, INT_MIN,
+    the first id past the end, INT_MAX; a clean row; over both batch sizes of the
+    history view and the one built in the workspace."""
+    bad = [-1, -2, -(2 ** 31), vocab, 2 ** 31 - 1, 0]
+    rows = len(bad)
+    bits = make_rows(rng, rows, vocab)
+    p = params(rows, rng, temperature=1.0, top_k=0, presence_penalty=0.5)
+    hist = rng.integers(0, vocab, (rows, length)).astype(np.int32)
+    hist[np.arange(rows), rng.integers(0, length, rows)] = np.array(bad, np.int64).astype(np.int32)
+    offs = np.arange(rows + 1, dtype=np.int64) * length
+    g, w = run_both(orc, dev, bits, 0, p, hist.reshape(-1), offs, want_probs=want_probs)
+    compare(g, w, p, "badhist")
+    assert (g["stats"]["flags"] & 16).astype(bool).tolist() == [True] * 5 + [False]
+
+
 def test_stream_repeat_calls_same_workspace(orc, dev, rng):
     """The part and arrival counters reset themselves: three calls in a row
     on one workspace give the same outputs."""

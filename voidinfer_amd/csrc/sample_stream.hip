@@ -1471,7 +1471,7 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
 #pragma unroll
         for (int j = 0; j < kHistBatch; ++j) {
             const int64_t i = base + int64_t(j) * kT + tid;
-            t[j] = i < e ? h.histories[i] : -2;   // (-2: past the end)
+            t[j] = i < e ? h.histories[i] : -1;
         }
     };
     load(b);
@@ -1488,7 +1488,7 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
                 const int32_t tj = t[j0 + j];
                 old[j] = 0u;
                 if (tj >= 0 && tj < V) old[j] = atomicOr(&B1[tj >> 5], 1u << (tj & 31));
-                else if (tj != -2) flags = VI_FLAG_BAD_HISTORY;
+                else if (base + int64_t(j0 + j) * kT + tid < e) flags = VI_FLAG_BAD_HISTORY;   // (not past the end)
             }
 #pragma unroll
             for (int j = 0; j < kHistBatch / 2; ++j) {
