@@ -487,3 +487,29 @@ def test_full_route_fp32_slice_edges_and_long_chains(orc, dev, rng, vocab):
     assert np.array_equal(out.tokens.cpu().numpy(), g["tokens"])
     assert np.array_equal(vi.stats_numpy(out.stats), g["stats"])
     assert np.array_equal(out.probs.cpu().numpy(), g["probs"])
+
+
+@pytest.mark.parametrize("vocab", [5_000, 20_482])
+@pytest.mark.parametrize("top_k", [0, 20])
+def test_fp32_history_token_whose_unpenalized_z_overflows(orc, dev, rng, vocab, top_k):
+    """A token of a partial slice's last whole vector whose z overflows without its
+    penalty and is finite with it: nothing of the row is invalid (the lanes past the
+    vector hold its logits too, without their counts).  Row 0: the row's largest
+    logit; row 1: its smallest; row 2: invalid with its penalty as well."""
+    import voidinfer_amd as vi
+    rows, last = 3, vocab // 4 * 4 - 2
+    x = make_rows(rng, rows, vocab, std=1.0, dtype=2)
+    x[:, last] = [2.5e38, -2.5e38, 3.3e38]
+    p = params(rows, rng, temperature=0.5, top_k=top_k, top_p=0.9,
+               repetition_penalty=np.array([2.0, 0.5, 1.1], np.float32))
+    hist = np.tile(np.array([last, 5], np.int32), rows)
+    offs = np.arange(rows + 1, dtype=np.int64) * 2
+    g, w = run_both(orc, dev, x, 2, p, hist, offs)
+    assert w["stats"]["flags"].tolist() == [0, 0, vi.FLAG_NONFINITE] and w["tokens"][0] == last
+    compare(g, w, p, "history")
+    state = vi.PenaltyState(rows, vocab, slots=64, device=dev)
+    state.update(torch.from_numpy(hist).to(dev), torch.from_numpy(offs).to(dev))
+    out = vi.sample_rows_state(to_dev(x, 2, dev), p, state, want_probs=True)
+    torch.cuda.synchronize()
+    compare(dict(tokens=out.tokens.cpu().numpy(), u=out.uniforms.cpu().numpy(), stats=vi.stats_numpy(out.stats),
+                 probs=out.probs.cpu().numpy()), w, p, "state")

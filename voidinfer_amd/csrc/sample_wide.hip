@@ -355,7 +355,8 @@ __device__ __forceinline__ SliceZ slice_z(const WideArgs& a, const WGeo& g, int 
             }
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                const int t0 = g.s0 + 4 * ((i0 + h) * kT + tid);
+                const int x = (i0 + h) * kT + tid, t0 = g.s0 + 4 * x;
+                bool bad = false;   // (not of a lane past the last vector: its logits lack their counts)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const uint32_t b = vec_bits<VI_F32>(v[i0 + h], e);
@@ -365,8 +366,9 @@ __device__ __forceinline__ SliceZ slice_z(const WideArgs& a, const WGeo& g, int 
                             : first[h][e].x == 0u                  ? 0u
                                                   : hash_count(w.table, w.shift, w.slots, t0 + e);
                     }
-                    r.z[i0 + h][e] = counted_z(p, inv_t, b, c, &r.bad);
+                    r.z[i0 + h][e] = counted_z(p, inv_t, b, c, &bad);
                 }
+                r.bad |= bad && x < g.nvec;
             }
         }
     } else {
