@@ -513,3 +513,62 @@ def test_fp32_history_token_whose_unpenalized_z_overflows(orc, dev, rng, vocab, 
     torch.cuda.synchronize()
     compare(dict(tokens=out.tokens.cpu().numpy(), u=out.uniforms.cpu().numpy(), stats=vi.stats_numpy(out.stats),
                  probs=out.probs.cpu().numpy()), w, p, "state")
+
+
+def cut_on_a_bin_end(count):
+    """A row and a top_p whose target is the running mass at the end of the bin z in
+    [-J/64, -(J-1)/64) as a double holds it, while that bin's own mass, added to what
+    lies before it without rounding, stays below: 100,000 logits of 0, `count` of
+    -J/64, and a tail whose mass is 2^-24 of the row's."""
+    from fractions import Fraction
+    top_p, n0 = np.float32(1.0 - 2.0 ** -24), 100_000
+    for J in range(40, 200):
+        own = float(count) * np.exp(-J / 64.0)
+        end = n0 + own                                     # (rounded to 2^-36)
+        up = float((Fraction(end) - n0 - Fraction(own)) * 2 ** 36)
+        if 0.2 < up < 0.45:
+            break
+    # the tail: exp(-8) as often as it fits, then five single weights found by a search
+    # over pair sums, so that top_p times the rounded total is `end` itself
+    total = end / float(top_p)
+    while float(top_p) * total < end:
+        total = np.nextafter(total, np.inf)
+    while float(top_p) * total > end:
+        total = np.nextafter(total, 0.0)
+    assert float(top_p) * total == end
+    w = np.exp(-np.arange(512, 768) / 64.0)
+    n = int((total - end) / w[0]) - 1
+    pair = np.add.outer(w, w).ravel()
+    order = np.argsort(pair)
+    for first, single in enumerate(w):
+        want = total - end - n * w[0] - single - pair
+        at = np.clip(np.searchsorted(pair[order], want), 0, len(pair) - 1)
+        err = np.abs(pair[order][at] - want)
+        i = int(err.argmin())
+        if err[i] < 2.0 ** -39:
+            break
+    j = int(order[at[i]])
+    tail = np.array([0] * n + [first, i // 256, i % 256, j // 256, j % 256]) + 512
+    z = np.concatenate([np.zeros(n0), np.full(count, -J / 64.0), -tail / 64.0]).astype(np.float32)
+    assert end + float(np.sum(np.exp(z[n0 + count:].astype(np.float64)))) == total
+    return z, top_p, n0 + count
+
+
+@pytest.mark.parametrize("count", [63, 64, 65, 1000])
+def test_full_route_fp32_cut_on_a_bin_end(orc, dev, rng, count):
+    """A top-p target that the running sums reach at a bin's end and the bin's own
+    mass misses by its rounding: the cut is the bin's last logit, or the next one."""
+    import voidinfer_amd as vi
+    z, top_p, end = cut_on_a_bin_end(count)
+    rows = 4
+    x = np.tile(z, (rows, 1))
+    p = params(rows, rng, temperature=1.0, top_p=top_p)
+    out = vi.sample_rows(to_dev(x, 2, dev), p, want_probs=True)
+    torch.cuda.synchronize()
+    s, tok = vi.stats_numpy(out.stats), out.tokens.cpu().numpy()
+    w_tok, w_u, _, w_stats, margins = orc.sample_rows(x, 2, p, None, None, want_probs=False)
+    assert (np.abs(margins[:, 1:3]).min(axis=1) < 1e-9).all() and (np.abs(w_stats["support"].astype(int) - end) <= 1).all()
+    assert (s["flags"] == 0).all() and (np.abs(s["support"].astype(int) - end) <= 1).all(), s
+    np.testing.assert_allclose(s["support_mass"], w_stats["support_mass"], rtol=1e-9)
+    assert ((out.probs > 0).sum(dim=1).cpu().numpy() == s["support"]).all()
+    assert (tok == w_tok)[margins[:, 0] > 1e-6].all()

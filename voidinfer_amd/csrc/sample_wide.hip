@@ -959,8 +959,10 @@ __device__ __forceinline__ BinSel select_bin(const RowCtx& c, FinishLds& L, int 
 
 // Narrows the selected bin J (b) to the logit at which the cumulative count
 // (mode 0: >= target) or mass (mode 1: >= target, mode 2: > target) over the
-// bin's logits in order is reached; target counts from the bin's start.  All
-// threads; the result in every thread.
+// bin's logits in order is reached; target counts from the bin's start.  The
+// running sums said that it is reached in this bin: where rounding of the
+// differences says otherwise, the bin's last logit.  All threads; the result in
+// every thread.
 __device__ __forceinline__ RHit narrow(const RowCtx& c, FinishLds& L, int J, const BinSel& b0, int mode, double target) {
     const int tid = threadIdx.x, lane = lane_id(), wave = tid / kWave;
     const bool massy = J < kNB;   // (the deep bin's logits carry no mass)
@@ -995,7 +997,7 @@ __device__ __forceinline__ RHit narrow(const RowCtx& c, FinishLds& L, int J, con
                 }
                 const double incl = double(fa + (unsigned long long)eq * wk) * unit;
                 const bool hit = k && (mode == 0 ? double(above + eq) >= tgt : mode == 1 ? incl >= tgt : incl > tgt);
-                const uint32_t best = wave_max_u32(hit ? k : 0u);
+                const uint32_t best = ballot(hit) ? wave_max_u32(hit ? k : 0u) : ~wave_max_u32(k ? ~k : 0u);
                 if (k == best && lane == __builtin_ctzll(ballot(k == best))) {
                     L.u0 = best;
                     L.u1 = above;
@@ -1007,7 +1009,7 @@ __device__ __forceinline__ RHit narrow(const RowCtx& c, FinishLds& L, int J, con
             const uint32_t best = L.u0, ca = L.u1, ce = L.u2;
             const unsigned long long f = L.f0;
             __syncthreads();
-            if (!best) { h.found = false; return h; }
+            if (!best) return h;   // (no pair in the range)
             h.cnt_before += ca;
             h.fix_before += f;
             h.cnt_key = ce;
@@ -1043,9 +1045,9 @@ __device__ __forceinline__ RHit narrow(const RowCtx& c, FinishLds& L, int J, con
             }
             uint32_t cc = wave_incl_scan_u32(tc) - tc;
             double cf = wave_incl_scan_f64(tf) - tf;
-            int fq = -1;
-            uint32_t fc = 0u;
-            double ff = 0.0;
+            int fq = -1, lq = -1;   // the lane's first bucket that reaches the target, its last with logits
+            uint32_t fc = 0u, lc = 0u;
+            double ff = 0.0, lf = 0.0;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const uint32_t nc = cc + bc[q];
@@ -1055,12 +1057,14 @@ __device__ __forceinline__ RHit narrow(const RowCtx& c, FinishLds& L, int J, con
                 else if (mode == 1) hit = nf * unit >= tgt;
                 else hit = nf * unit > tgt;
                 if (fq < 0 && bc[q] && hit) { fq = q; fc = cc; ff = cf; }
+                if (bc[q]) { lq = q; lc = cc; lf = cf; }
                 cc = nc;
                 cf = nf;
             }
-            const uint64_t m = ballot(fq >= 0);
-            if (lane == 0) L.u0 = m ? 1u : 0u;
-            if (m && lane == __builtin_ctzll(m)) {
+            const uint64_t m = ballot(fq >= 0), o = ballot(lq >= 0);
+            if (lane == 0) L.u0 = o ? 1u : 0u;
+            if (!m) { fq = lq; fc = lc; ff = lf; }
+            if (o && lane == (m ? __builtin_ctzll(m) : 63 - __builtin_clzll(o))) {
                 const uint32_t b = uint32_t(kDig - 1 - 4 * lane - fq);
                 L.u1 = b;
                 L.u2 = fc;
@@ -1069,7 +1073,7 @@ __device__ __forceinline__ RHit narrow(const RowCtx& c, FinishLds& L, int J, con
             }
         }
         __syncthreads();
-        if (!L.u0) { h.found = false; __syncthreads(); return h; }
+        if (!L.u0) { __syncthreads(); return h; }   // (no pair in the range)
         const uint32_t b = L.u1;
         h.cnt_before += L.u2;
         h.fix_before += (unsigned long long)(L.d0);
