@@ -156,6 +156,35 @@ def test_stream_every_bad_history_token_is_flagged(orc, dev, rng, vocab, length,
     assert (g["stats"]["flags"] & 16).astype(bool).tolist() == [True] * 5 + [False]
 
 
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("vocab", [64, 4_099])
+def test_stream_top_p_of_nothing_keeps_the_first_logit(orc, dev, rng, dtype, vocab):
+    """top_p so small that its share of the mass is below the sums' unit, 0, or
+    negative: the support is the row's first logit (first id among equal ones), alone
+    and beside the other filters, with probabilities and without; the same row's
+    verification accepts and corrects from that support."""
+    import voidinfer_amd as vi
+    rows = 8
+    bits = make_rows(rng, rows, vocab, std=1.0, dtype=dtype)
+    bits[1::2] = 0                                       # all equal: id 0
+    p = params(rows, rng, temperature=0.8, top_k=np.array([0, 0, 100, 100, 0, 0, 0, 0]),
+               top_p=np.array([0, 0, 0, 0, 1e-14, 1e-14, -0.5, -0.5], np.float32),
+               min_p=np.array([0, 0, 0, 0, 0.1, 0.1, 0, 0], np.float32))
+    for want_probs in (False, True):
+        g, w = run_both(orc, dev, bits, dtype, p, want_probs=want_probs)
+        assert (w["stats"]["support"] == 1).all() and (w["tokens"][1::2] == 0).all()
+        assert np.array_equal(g["tokens"], w["tokens"]) and np.array_equal(g["stats"]["support"], w["stats"]["support"])
+        np.testing.assert_allclose(g["stats"]["support_mass"], 1.0, rtol=1e-6)
+        if want_probs:
+            assert np.array_equal(g["probs"] > 0, w["probs"] > 0)
+    drafted = np.where(np.arange(rows) % 3 == 0, w["tokens"], 1).astype(np.int32)
+    t = to_dev(bits, dtype, dev)
+    got = vi.verify_rows(vi.VERIFY_SAMPLED, t, torch.from_numpy(drafted).to(dev), rows, 1, draft=t, params=p)
+    want = orc.verify_rows(1, bits, dtype, bits, dtype, rows, 1, drafted, p, ())
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)
+
+
 def test_stream_repeat_calls_same_workspace(orc, dev, rng):
     """The part and arrival counters reset themselves: three calls in a row
     on one workspace give the same outputs."""

@@ -962,7 +962,6 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
     // holds it, then its 128 blocks, two to a lane.  (A search over the 2048
     // sums themselves probes every 32nd first, all in one LDS bank: 1,700 cycles.)
     auto block_search = [&](int mode, uint64_t target) -> int {
-        if (mode == 1 && target == 0u) return -1;
         auto reached = [&](uint64_t x) { return mode == 2 ? x > target : x >= target; };
         const int wl = lane & (kW - 1);
         const uint64_t wm = ballot(lane < kW && reached(mode == 0 ? uint64_t(sh.wci[wl]) : sh.wmi[wl]));
@@ -1066,7 +1065,8 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
         }
         // top-p: the first position whose cumulative mass reaches top_p of the cap's
         if (p.top_p < 1.0f) {
-            const uint64_t target = uint64_t(llrint(double(p.top_p) * s_cap));
+            // (a target of less than one unit, of any top_p <= 0 too: the first logit)
+            const uint64_t target = uint64_t(std::max(llrint(double(p.top_p) * s_cap), 1ll));
             const int b = block_search(1, target);
             const int lowest = has_cap ? int(cap_key >> 5) : 0;
             if (b >= lowest) {
