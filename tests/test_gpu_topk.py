@@ -129,3 +129,18 @@ def test_rows_off_a_16_byte_boundary(orc, dev, rng, dtype, offset, vocab):
     w_g, w_gap = orc.row_scores(inner, dtype, nxt)
     assert np.array_equal(g.cpu().numpy(), w_g)
     np.testing.assert_array_equal(gap.cpu().numpy(), w_gap)
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("rows,vocab", [(3, 5_003), (64, 60_001), (64, 120_000)])
+def test_logprobs_of_rows_masked_with_the_lowest_value(orc, dev, rng, dtype, rows, vocab):
+    """Grammar masks set with the type's lowest finite value: a lane may see
+    nothing else for many vectors (x log2(e) of it overflows)."""
+    x = rng.standard_normal((rows, vocab)).astype(np.float32)
+    low = np.float32([-3.3895314e38, -65504.0, -3.4028235e38][dtype])
+    keep = rng.random((rows, vocab)) < np.array([0.5, 0.02, 0.001])[np.arange(rows) % 3][:, None]
+    keep[:, rng.integers(0, vocab, 8)] = True
+    x = np.where(keep, x, low)
+    bits = x if dtype == 2 else (x.astype(np.float16).view(np.uint16) if dtype == 1 else
+                                 (x.view(np.uint32) >> 16).astype(np.uint16))
+    run(orc, dev, bits, dtype, 8)

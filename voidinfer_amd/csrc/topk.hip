@@ -639,11 +639,13 @@ __device__ __forceinline__ void topk_body(const TopkArgs& a, const int slice, co
     // terms 2^(x log2(e) - m2) are taken against (x log2(e) as x * kL2E + x *
     // kL2ELo, the second the rounding residual of the first), so the row's
     // log-sum-exp is ln 2 * (m2 + log2(sum)) with no rounding of m2 left over.
+    // m2 is kept finite: logits down to the type's lowest value (a mask) may be
+    // all that a lane sees first, and terms against -inf would be infinite.
     constexpr float kL2E = 1.4426950408889634f;
     constexpr float kL2ELo = 1.925963e-8f;
     auto lse_term = [&](float x) { return __builtin_amdgcn_exp2f(fmaf(x, kL2ELo, fmaf(x, kL2E, -lse_m))); };
     auto lse_rebase = [&](float xmax) {   // (per lane)
-        const float m2 = xmax * kL2E;
+        const float m2 = fmaxf(xmax * kL2E, -3.402823466e38f);
         if (m2 > lse_m) {
             lse_s = lse_s * __builtin_amdgcn_exp2f(lse_m - m2);
             lse_m = m2;
