@@ -157,6 +157,27 @@ def test_stream_every_bad_history_token_is_flagged(orc, dev, rng, vocab, length,
 
 
 @pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("want_probs", [False, True])
+@pytest.mark.parametrize("vocab", [4_096, 4_099])
+def test_stream_min_p_between_weights_closer_than_fp32(orc, dev, rng, dtype, want_probs, vocab):
+    """Logits so small, or temperatures so high, that their weights round to one
+    another in single precision: min_p 1 keeps the largest ones only, and min_p at
+    the weight of a value between two neighbours keeps what lies above."""
+    rows = 4
+    x = rng.integers(1, 40, (rows, vocab)).astype(np.float32) * np.float32(2.0 ** -10)
+    bits = {0: lambda: (x.view(np.uint32) >> 16).astype(np.uint16), 1: lambda: x.astype(np.float16).view(np.uint16),
+            2: lambda: x}[dtype]()
+    p = params(rows, rng, temperature=np.array([60_000, 60_000, 30_000, 65_536], np.float32), top_p=1.0,
+               min_p=np.array([1.0, 1.0 - 2.0 ** -24, 1.0, 1.0 - 2.0 ** -23], np.float32))
+    g, w = run_both(orc, dev, bits, dtype, p, want_probs=want_probs)
+    assert (w["stats"]["support"][[0, 2]] < vocab // 20).all()
+    assert np.array_equal(g["stats"]["support"], w["stats"]["support"]), (g["stats"], w["stats"])
+    assert np.array_equal(g["tokens"], w["tokens"])
+    if want_probs:
+        assert np.array_equal(g["probs"] > 0, w["probs"] > 0)
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
 @pytest.mark.parametrize("vocab", [64, 4_099])
 def test_stream_top_p_of_nothing_keeps_the_first_logit(orc, dev, rng, dtype, vocab):
     """top_p so small that its share of the mass is below the sums' unit, 0, or

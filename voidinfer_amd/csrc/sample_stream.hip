@@ -1055,12 +1055,13 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
             cap_take = cap.take;
             s_cap = double(cap.mass);
         }
-        // min-p: the lowest key whose weight reaches min_p
+        // min-p: the lowest key whose weight reaches min_p (in double precision: the
+        // masses' weights are good to an fp32 ulp, which a key near the cut may miss)
         uint32_t minp_key = 0u;
         if (p.min_p > 0.0f) {
             const double mp = double(p.min_p);
             minp_key = uint32_t(wave_search(int(kmin), int(z0key) + 1, [&](int k) {
-                return key_weight<DT>(uint32_t(k), inv_t, z0) >= mp;
+                return exp(double(key_z<DT>(uint32_t(k), inv_t)) - z0) >= mp;
             }));
         }
         // top-p: the first position whose cumulative mass reaches top_p of the cap's
