@@ -215,3 +215,33 @@ def test_selector_chain_chunk_edges(orc, dev, lanes, positions):
         check_chain_fp64(got[diff], anchors[diff], cands[diff], unary[diff], hidden[diff], pred, succ)
     if positions > 16:
         assert (got[1, 16:] == -1).all() and (got[1, :16] >= 0).all()
+
+
+@pytest.mark.parametrize("lanes,positions", [(5, 5), (256, 9), (257, 17), (513, 5), (1030, 3)])
+def test_selector_chain_many_lanes_with_sampled_ones(orc, dev, lanes, positions):
+    """Lane counts on both sides of the lines where the chunk gets shorter, sampled
+    lanes (four to a workgroup) between greedy ones, the last ones sampled, invalid
+    anchors and candidates on both kinds."""
+    import voidinfer_amd as vi
+    rng = np.random.default_rng(lanes)
+    vocab = 600
+    anchors, cands, unary, hidden, pred, succ = _chain_case(rng, lanes, positions, vocab)
+    sampled = rng.random(lanes) < 0.5
+    sampled[-3:], sampled[:2] = True, (False, True)
+    anchors[0], anchors[1] = vocab, -1
+    cands[2, positions - 1, 7] = vocab
+    cands[lanes - 1, 1, 0] = -1
+    smp = np.zeros(lanes, dtype=vi.DRAFT_SAMPLING)
+    smp["inv_temperature"] = np.where(sampled, 1.25, 0.0)
+    smp["top_k"], smp["top_p"], smp["presence_penalty"] = 10, 0.9, 0.5
+    smp["seed"] = rng.integers(1, 2**62, lanes)
+    got = _run_chain(dev, anchors, cands, unary, hidden, pred, succ, smp)
+    want = orc.selector_chain(anchors, cands, unary, hidden.view(np.uint16), pred.view(np.uint16),
+                              succ.view(np.uint16), smp)
+    assert (got[:2] == -1).all() and (got[lanes - 1, 1:] == -1).all() and got[lanes - 1, 0] >= 0
+    assert np.array_equal(got == -1, want == -1)
+    greedy = np.flatnonzero(~sampled)
+    check_chain_fp64(got[greedy], anchors[greedy], cands[greedy], unary[greedy], hidden[greedy], pred, succ)
+    for l in np.flatnonzero(sampled & (got != want).any(axis=1)):
+        p = int(np.argmax(got[l] != want[l]))
+        assert near_boundary(orc, unary[l, p], cands[l, p], smp[l], int(smp["key_base"][l]) + p), (l, p)

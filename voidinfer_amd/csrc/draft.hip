@@ -14,6 +14,8 @@
 // lane; the per-thread candidate arrays live in LDS.
 #include <math.h>
 
+#include <algorithm>
+
 #include "vi_device.h"
 #include "vi_internal.h"
 
@@ -160,9 +162,12 @@ __device__ __forceinline__ int first_max16_lanes(float score, int c) {
     return __builtin_ctzll(ballot(key == m));
 }
 
-template <int CH>   // positions per chunk
+// CH: positions per chunk.  GROUPS: the first groups of the grid take the sampled
+// lanes, one per wave, and a workgroup per lane the others; else every lane has a
+// workgroup.
+template <int CH, bool GROUPS>
 __global__ __launch_bounds__(kChainThreads) void selector_chain_kernel(
-    int positions, int vocabulary, const int64_t* anchors, const int64_t* candidates, const float* unary,
+    int lanes, int positions, int vocabulary, const int64_t* anchors, const int64_t* candidates, const float* unary,
     const uint16_t* hidden, const uint16_t* pred_cb, const uint16_t* succ_cb, const vi_draft_sampling* sampling,
     int64_t* proposals) {
     __shared__ __attribute__((aligned(16))) uint16_t s_pred[CH][kDraftK][kRank];
@@ -170,9 +175,17 @@ __global__ __launch_bounds__(kChainThreads) void selector_chain_kernel(
     __shared__ float s_unary[CH][kDraftK];
     __shared__ __attribute__((aligned(16))) float s_score[2][kDraftK];
     __shared__ int s_valid[kChainWaves];
-    __shared__ float s_val[kDraftK], s_prob[kDraftK];
-    __shared__ int s_ord[kDraftK];
-    const int t = threadIdx.x, w = t / kWave, k = lane_id(), l = blockIdx.x;
+    constexpr int kSerial = GROUPS ? kChainWaves : 1;   // sampled lanes of a workgroup
+    __shared__ float s_val[kSerial][kDraftK + 1], s_prob[kSerial][kDraftK + 1];
+    __shared__ int s_ord[kSerial][kDraftK + 1];
+    const int t = threadIdx.x, w = t / kWave, k = lane_id();
+    int l = blockIdx.x;
+    if constexpr (GROUPS) {
+        const int groups = (lanes + kChainWaves - 1) / kChainWaves;
+        const bool group = l < groups;
+        l = group ? l * kChainWaves + w : l - groups;
+        if (l >= lanes || (sampling[l].inv_temperature > 0.0f) != group) return;   // (whole waves; a group has no barrier)
+    }
     const int64_t seed_token = anchors[l];
     int64_t* out = proposals + size_t(l) * positions;
     const int64_t* lane_cand = candidates + size_t(l) * positions * kDraftK;
@@ -180,7 +193,8 @@ __global__ __launch_bounds__(kChainThreads) void selector_chain_kernel(
     bool bad = seed_token < 0 || seed_token >= vocabulary;   // ends the chain (workgroup-uniform)
     if (sampling && sampling[l].inv_temperature > 0.0f) {
         // the coupled choice over the unary scores: serial, one wave
-        if (w != 0) return;
+        if (!GROUPS && w != 0) return;
+        const int own = GROUPS ? w : 0;
         const vi_draft_sampling smp = sampling[l];
         for (int pos = 0; pos < positions; ++pos) {
             const int64_t* cd = lane_cand + size_t(pos) * kDraftK;
@@ -189,7 +203,7 @@ __global__ __launch_bounds__(kChainThreads) void selector_chain_kernel(
             if (k != 0) continue;
             if (bad) { out[pos] = -1; continue; }
             const int best = sampled_pick(smp, pos, vocabulary, lane_unary + size_t(pos) * kDraftK, cd, seed_token, out,
-                                          s_val, s_prob, s_ord);
+                                          s_val[own], s_prob[own], s_ord[own]);
             out[pos] = cd[best];
         }
         return;
@@ -277,13 +291,25 @@ vi_status launch_selector_chain(int lanes, int positions, int vocabulary, const 
                                 const int64_t* candidates, const float* unary, const void* hidden,
                                 const void* pred_codebook, const void* succ_codebook,
                                 const vi_draft_sampling* sampling, int64_t* proposals, hipStream_t stream) {
-    // the smallest chunk that holds the chain: its rows are all requested at once
-    auto* kernel = positions <= 4 ? &selector_chain_kernel<4>
-                   : positions <= 8 ? &selector_chain_kernel<8>
-                                    : &selector_chain_kernel<kChainMax>;
-    hipLaunchKernelGGL(kernel, dim3(lanes), dim3(kChainThreads), 0, stream, positions, vocabulary, anchors, candidates,
-                       unary, static_cast<const uint16_t*>(hidden), static_cast<const uint16_t*>(pred_codebook),
-                       static_cast<const uint16_t*>(succ_codebook), sampling, proposals);
+    // The smallest chunk that holds the chain (its rows are all requested at once),
+    // unless its LDS leaves lanes waiting for a CU: one workgroup fits a CU with 16
+    // positions, two with 8, four with 4.  (16 positions, us, chunks of 16 / by this
+    // rule: 512 lanes 39 / 28, 1,024 lanes 74 / 42, 4,096 lanes 277 / 153.)
+    // A sampled lane works with one thread: past what the CUs hold at once, four of
+    // them share a workgroup.  (All sampled, a workgroup each with chunks of 16 / by
+    // this rule: 512 lanes 314 / 172, 1,024 lanes 624 / 181, 4,096 lanes 2,458 / 213.)
+    const int cus = device_cus(), most = lanes <= cus ? kChainMax : lanes <= 2 * cus ? 8 : 4;
+    const int chunk = std::min(positions <= 4 ? 4 : positions <= 8 ? 8 : kChainMax, most);
+    const bool groups = sampling && lanes > 4 * cus;
+    auto* kernel = groups       ? &selector_chain_kernel<4, true>
+                   : chunk == 4 ? &selector_chain_kernel<4, false>
+                   : chunk == 8 ? &selector_chain_kernel<8, false>
+                                : &selector_chain_kernel<kChainMax, false>;
+    const int extra = groups ? (lanes + kChainWaves - 1) / kChainWaves : 0;
+    hipLaunchKernelGGL(kernel, dim3(extra + lanes), dim3(kChainThreads), 0, stream, lanes, positions, vocabulary,
+                       anchors, candidates, unary, static_cast<const uint16_t*>(hidden),
+                       static_cast<const uint16_t*>(pred_codebook), static_cast<const uint16_t*>(succ_codebook),
+                       sampling, proposals);
     return launch_status();
 }
 
