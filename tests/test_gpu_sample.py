@@ -572,3 +572,22 @@ def test_full_route_fp32_cut_on_a_bin_end(orc, dev, rng, count):
     np.testing.assert_allclose(s["support_mass"], w_stats["support_mass"], rtol=1e-9)
     assert ((out.probs > 0).sum(dim=1).cpu().numpy() == s["support"]).all()
     assert (tok == w_tok)[margins[:, 0] > 1e-6].all()
+
+
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+@pytest.mark.parametrize("vocab", [50_000, 50_001])
+def test_full_route_probabilities_are_rounded_fp64_values(dev, rng, dtype, vocab):
+    """exp(z - z0) / S_n in double precision, rounded once to fp32, with the row's
+    own S_n: another value only where the fp64 one lies within a few of its ulps of
+    a rounding boundary (one in 10^8)."""
+    import voidinfer_amd as vi
+    rows = 6
+    bits = make_rows(rng, rows, vocab, std=1.0, dtype=dtype)
+    p = params(rows, rng, temperature=1.0, top_p=np.array([1.0, 0.95] * 3, np.float32))
+    out = vi.sample_rows(to_dev(bits, dtype, dev), p, want_probs=True)
+    torch.cuda.synchronize()
+    got, mass = out.probs.cpu().numpy(), vi.stats_numpy(out.stats)["support_mass"]
+    z = decode_rows(bits, dtype).astype(np.float64)
+    want = (np.exp(z - z.max(axis=1, keepdims=True)) / mass[:, None]).astype(np.float32)
+    assert (got > 0).sum() > 100 * rows
+    assert (got != want)[got > 0].sum() <= 3

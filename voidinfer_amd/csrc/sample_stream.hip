@@ -1572,7 +1572,7 @@ __device__ __forceinline__ float pattern_prob(uint32_t pat, int id, const FullBo
     const uint32_t k = key16(pat);
     const float z = Elem<DT>::decode(unkey16(k)) * B.inv_t;
     const bool in = Elem<DT>::finite_bits(pat) && isfinite(z) && (k > B.end_key || (k == B.end_key && id <= B.end_id));
-    return in ? float(exp_neg(double(z) - B.z0) * inv_s) : 0.0f;
+    return in ? float(exp(double(z) - B.z0) * inv_s) : 0.0f;
 }
 
 template <int DT>

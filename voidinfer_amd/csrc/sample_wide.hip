@@ -1424,7 +1424,7 @@ __global__ __launch_bounds__(kPT) void wide_probs_kernel(WideArgs a) {
         const float z = logit_z(w, p, bd.inv_t, id, bits, word, &bad, unrec);
         const uint32_t k = isnan(z) ? 0u : key32(z);
         const bool in = bd.valid && k && (k > bd.end_key || (k == bd.end_key && id <= bd.end_id));
-        return in ? float(exp_neg(double(z) - bd.z0) * inv_s) : 0.0f;
+        return in ? float(exp(double(z) - bd.z0) * inv_s) : 0.0f;
     };
     if (whole) {
         f32x4_t q;

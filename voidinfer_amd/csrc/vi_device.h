@@ -143,24 +143,6 @@ __device__ __forceinline__ uint4 load16_cached(const void* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
-// exp(d) for d <= 0, relative error below 3e-9 (a twentieth of the rounding of
-// the fp32 result it is meant for): d = k ln 2 + r with |r| <= ln 2 / 2, the terms of
-// exp(r)'s series up to r^2 in fp64 and the rest, at most 0.008, in fp32.  About a
-// third of the fp64 instructions of the library's exp.
-__device__ __forceinline__ double exp_neg(double d) {
-    const float k = rintf(fmaxf(float(d), -800.0f) * 1.44269504088896340736f);
-    const double r = fma(double(k), -0.69314718055994530942, d);
-    const float f = float(r);
-    // r^3 / 3! .. r^8 / 8!
-    float q = fmaf(f, 2.48015873e-5f, 1.98412698e-4f);
-    q = fmaf(f, q, 1.38888889e-3f);
-    q = fmaf(f, q, 8.33333333e-3f);
-    q = fmaf(f, q, 4.16666667e-2f);
-    q = fmaf(f, q, 1.66666667e-1f) * (f * f) * f;
-    const double e = fma(r * r, 0.5, r) + double(q) + 1.0;
-    return d < -800.0 ? 0.0 : ldexp(e, int(k));
-}
-
 // 16-bit order-preserving key of a sign-magnitude bf16 / fp16 pattern; -0 and
 // +0 share the key of +0.
 __device__ __forceinline__ uint32_t key16(uint32_t b) {
