@@ -206,6 +206,23 @@ def test_stream_top_p_of_nothing_keeps_the_first_logit(orc, dev, rng, dtype, voc
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("vocab,length", [(5_001, 4_096), (5_001, 4_097), (5_001, 8_193), (5_001, 16_384),
+                                          (5_001, 16_385), (5_001, 40_000), (300_001, 3_200), (300_001, 3_202),
+                                          (524_288, 16_256), (524_288, 16_260), (524_287, 70_000)])
+def test_stream_history_view_sizes(orc, dev, rng, vocab, length):
+    """Histories at the edges of the view's batches and of where its counts lie (half
+    a CU's LDS, a CU's, the workspace): tokens seen once and many times, one of them
+    up to the whole history, a short and an empty history beside the longest."""
+    rows = 5
+    bits = make_rows(rng, rows, vocab, std=0.5)
+    p = params(rows, rng, temperature=rng.uniform(0.5, 1.2, rows), top_k=0, top_p=0.95,
+               repetition_penalty=rng.uniform(1.0, 1.3, rows), presence_penalty=0.2, frequency_penalty=0.001)
+    hist = [rng.integers(0, vocab, length), np.tile(rng.choice(vocab, length // 2, replace=length // 2 > vocab), 2),
+            np.full(length, vocab - 1), rng.integers(vocab - 40, vocab, 100), np.zeros(0, int)]
+    offs = np.concatenate([[0], np.cumsum([len(h) for h in hist])]).astype(np.int64)
+    stream(orc, dev, bits, 0, p, np.concatenate(hist).astype(np.int32), offs, f"view-{vocab}-{length}")
+
+
 def test_stream_repeat_calls_same_workspace(orc, dev, rng):
     """The part and arrival counters reset themselves: three calls in a row
     on one workspace give the same outputs."""

@@ -1422,40 +1422,41 @@ __global__ __launch_bounds__(kT) void merge_kernel(StreamArgs a) {
 // stream reads from a penalty state: one workgroup per row; bitmaps of the
 // tokens seen once (B1) and more than once (B2) built with LDS atomics, then
 // each B2 token's rank (population count of B2 before it) indexes its count.
-// Rows whose bitmaps and counts exceed the LDS keep them in the workspace
-// (LDS = false: every access at agent scope).
+// The bitmaps of the largest vocabulary fit the LDS; counts that no longer do
+// beside them are kept in the workspace (every access to them at agent scope):
+// 2 rows x 500,001 tokens with histories of 30,000, 60 us per call, 190 with the
+// bitmaps there too.
 struct HistArgs {
     const int32_t* histories;
     const int64_t* offsets;
-    const vi_row_params* params;
     int vocabulary, words, cap;
     uint32_t* hb1;     // [rows][words]
     uint2* hlist;      // [rows][cap]
     uint32_t* hhead;   // [rows][2]
-    uint32_t* tmp;     // [rows][2 words + cap] (the workspace form)
+    uint32_t* tmp;     // [rows][cap]: the counts, where they are not in LDS
 };
-// History tokens per thread held in registers: 4 where that covers the longest
-// history, else 32.  (A batch's steps are issued whatever part of it holds
-// tokens: 24 rows of 2,048-token histories over 151,936 tokens take 7.4 us with 4, 12.9 with 32.)
-constexpr int kHistShort = 4, kHistLong = 32;
+// History tokens per thread held in registers: the first of 4, 8, 16 and 32 that
+// covers the longest history, else 32.  (A batch's steps are issued whatever part of
+// it holds tokens.  16 rows x 131,071, us per call with histories of 4,096 / 6,000 /
+// 12,000 / 16,384 / 20,000 tokens: 36 / 37 / 40 / 41 / 46; with 4 and 32 alone
+// 36 / 44 / 44 / 45 / 46.)
+constexpr int kHistLong = 32;
 
-constexpr int kHistLdsWords = 40896;   // B1 + B2 + counts (160 KB less the scalars)
+constexpr int kHistLdsWords = 40896;       // B1 + B2 + counts (160 KB less the scalars): one workgroup per CU
+constexpr int kHistLdsHalf = 20352;        // the same where two fit a CU (4,096 rows x 1,001: 398 us per call, 414)
+constexpr int kHistLdsBits = 2 * kMaxVocabulary / 32;   // B1 + B2
 
-template <bool LDS, int kHistBatch>
+// WORDS: the LDS (kHistLdsBits: the counts are in the workspace).
+template <int WORDS, int kHistBatch>
 __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
-    __shared__ __attribute__((aligned(16))) uint32_t lds[LDS ? kHistLdsWords : 1];
+    constexpr bool LDS = WORDS != kHistLdsBits;
+    __shared__ __attribute__((aligned(16))) uint32_t hl[WORDS];
     const int row = blockIdx.x, tid = threadIdx.x;
     const int W = h.words;
-    uint32_t* hl = LDS ? lds : h.tmp + size_t(row) * (2 * size_t(W) + size_t(h.cap));
     uint32_t* B1 = hl;              // then the prefix of B2 per word
     uint32_t* B2 = hl + W;
-    uint32_t* cnt = hl + 2 * W;     // [cap]
-    auto get = [](const uint32_t* p) { return LDS ? *p : load_agent(p); };
-    auto put = [](uint32_t* p, uint32_t v) {
-        if (LDS) *p = v;
-        else __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-    auto sync = []() {
+    uint32_t* cnt = LDS ? hl + 2 * W : h.tmp + size_t(row) * size_t(h.cap);     // [cap]
+    auto sync = []() {              // (the counts' stores and atomics with it)
         if (!LDS) __threadfence();
         __syncthreads();
     };
@@ -1476,9 +1477,9 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
         }
     };
     load(b);
-    for (int i = tid; i < 2 * W; i += kT) put(&hl[i], 0u);
+    for (int i = tid; i < (2 * W + 3) / 4; i += kT) reinterpret_cast<uint4*>(hl)[i] = make_uint4(0u, 0u, 0u, 0u);
     if (tid == 0) flags = 0u;
-    sync();
+    __syncthreads();
     for (int64_t base = b; base < e; base += int64_t(kHistBatch) * kT) {
         if (base != b) load(base);
 #pragma unroll
@@ -1499,13 +1500,14 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
             }
         }
     }
-    sync();
+    __syncthreads();
     // B1 out; its LDS then holds the B2 rank of each word's first bit
     uint32_t* out = h.hb1 + size_t(row) * W;
-    for (int i = tid; i < W; i += kT) out[i] = get(&B1[i]);
-    const int per = (W + kT - 1) / kT, w0 = tid * per, w1 = min(W, w0 + per);
+    for (int i = tid; i < W; i += kT) out[i] = B1[i];
+    // (ranks in the order of the threads' words tid, tid + kT, ...: the list's order is
+    // free, and the words a thread would hold in a run lie in few LDS banks)
     uint32_t own = 0u;
-    for (int i = w0; i < w1; ++i) own += uint32_t(__builtin_popcount(get(&B2[i])));
+    for (int i = tid; i < W; i += kT) own += uint32_t(__builtin_popcount(B2[i]));
     uint32_t total = 0u;
     const uint32_t ex = block_exclusive_scan_u32<kT>(own, scan, &total);   // (barriers: B1 read before)
     if (total > uint32_t(h.cap)) {   // cannot happen: the launcher sizes cap for the longest history
@@ -1514,9 +1516,12 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
     }
     {
         uint32_t r = ex;
-        for (int i = w0; i < w1; ++i) { put(&B1[i], r); r += uint32_t(__builtin_popcount(get(&B2[i]))); }
+        for (int i = tid; i < W; i += kT) { B1[i] = r; r += uint32_t(__builtin_popcount(B2[i])); }
     }
-    for (uint32_t i = tid; i < total; i += kT) put(&cnt[i], 0u);
+    for (uint32_t i = tid; i < total; i += kT) {
+        if (LDS) cnt[i] = 0u;
+        else __hip_atomic_store(&cnt[i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     sync();
     for (int64_t base = b; base < e; base += int64_t(kHistBatch) * kT) {
         if (!one_batch) load(base);
@@ -1527,8 +1532,8 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
             for (int j = 0; j < kHistBatch / 2; ++j) {
                 const int32_t tj = t[j0 + j];
                 const bool ok = tj >= 0 && tj < V;
-                wd[j] = ok ? get(&B2[tj >> 5]) : 0u;
-                r0[j] = ok ? get(&B1[tj >> 5]) : 0u;
+                wd[j] = ok ? B2[tj >> 5] : 0u;
+                r0[j] = ok ? B1[tj >> 5] : 0u;
             }
 #pragma unroll
             for (int j = 0; j < kHistBatch / 2; ++j) {
@@ -1539,12 +1544,12 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
     }
     sync();
     uint2* lst = h.hlist + size_t(row) * h.cap;
-    for (int i = w0; i < w1; ++i) {
-        uint32_t wd = get(&B2[i]), r = get(&B1[i]);
+    for (int i = tid; i < W; i += kT) {
+        uint32_t wd = B2[i], r = B1[i];
         while (wd) {
             const int j = __builtin_ctz(wd);
             wd &= wd - 1u;
-            lst[r] = make_uint2(uint32_t(32 * i + j), get(&cnt[r]));
+            lst[r] = make_uint2(uint32_t(32 * i + j), LDS ? cnt[r] : load_agent(&cnt[r]));
             ++r;
         }
     }
@@ -1733,8 +1738,17 @@ static int hist_words(int vocabulary) { return (vocabulary + 31) / 32; }
 static int hist_cap(int vocabulary, int64_t max_history) {
     return int(std::max<int64_t>(std::min<int64_t>(max_history / 2, vocabulary), 1));
 }
-static bool hist_in_lds(int vocabulary, int64_t max_history) {
-    return 2 * hist_words(vocabulary) + hist_cap(vocabulary, max_history) <= kHistLdsWords;
+// words of LDS that the bitmaps and counts take
+static int hist_lds(int vocabulary, int64_t max_history) {
+    return 2 * hist_words(vocabulary) + hist_cap(vocabulary, max_history);
+}
+template <int WORDS>
+static void launch_history_view(const HistArgs& h, int rows, int64_t max_history, hipStream_t stream) {
+    auto* kernel = max_history <= 4 * kT    ? &history_view_kernel<WORDS, 4>
+                   : max_history <= 8 * kT  ? &history_view_kernel<WORDS, 8>
+                   : max_history <= 16 * kT ? &history_view_kernel<WORDS, 16>
+                                            : &history_view_kernel<WORDS, kHistLong>;
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kT), 0, stream, h);
 }
 
 // Rows per launch: as many as keep a workgroup's parts within kMaxItems and the
@@ -1756,7 +1770,7 @@ size_t stream_workspace(int rows, int vocabulary, int64_t max_history) {
     if (max_history > 0) {
         const size_t words = size_t(hist_words(vocabulary)), cap = size_t(hist_cap(vocabulary, max_history));
         b += align_up(r * words * 4, 256) + align_up(r * cap * 8, 256) + align_up(r * 8, 256);
-        if (!hist_in_lds(vocabulary, max_history)) b += align_up(r * (2 * words + cap) * 4, 256);
+        if (hist_lds(vocabulary, max_history) > kHistLdsWords) b += align_up(r * cap * 4, 256);
     }
     return b + 256;
 }
@@ -1794,22 +1808,21 @@ vi_status launch_stream(const SampleArgs& s, unsigned char* ws, size_t ws_bytes,
     const bool hist = !s.pstate && s.histories && s.offsets && s.max_history > 0;
     HistArgs h{};
     if (hist) {
-        h.histories = s.histories; h.offsets = s.offsets; h.params = s.params; h.vocabulary = s.vocabulary;
+        h.histories = s.histories; h.offsets = s.offsets; h.vocabulary = s.vocabulary;
         h.words = hist_words(s.vocabulary);
         h.cap = hist_cap(s.vocabulary, s.max_history);
         h.hb1 = c.take<uint32_t>(size_t(s.rows) * h.words);
         h.hlist = c.take<uint2>(size_t(s.rows) * h.cap);
         h.hhead = c.take<uint32_t>(size_t(s.rows) * 2);
-        if (!hist_in_lds(s.vocabulary, s.max_history))
-            h.tmp = c.take<uint32_t>(size_t(s.rows) * (2 * size_t(h.words) + size_t(h.cap)));
+        if (hist_lds(s.vocabulary, s.max_history) > kHistLdsWords)
+            h.tmp = c.take<uint32_t>(size_t(s.rows) * size_t(h.cap));
         a.hwords = h.words; a.hcap = h.cap;
     }
     if (!c.ok) return VI_ERR_WORKSPACE;
     if (hist) {
-        const dim3 rows(s.rows), block(kT);
-        if (h.tmp) hipLaunchKernelGGL((history_view_kernel<false, kHistLong>), rows, block, 0, stream, h);
-        else if (s.max_history <= kHistShort * kT) hipLaunchKernelGGL((history_view_kernel<true, kHistShort>), rows, block, 0, stream, h);
-        else hipLaunchKernelGGL((history_view_kernel<true, kHistLong>), rows, block, 0, stream, h);
+        if (h.tmp) hipLaunchKernelGGL((history_view_kernel<kHistLdsBits, kHistLong>), dim3(s.rows), dim3(kT), 0, stream, h);
+        else if (hist_lds(s.vocabulary, s.max_history) <= kHistLdsHalf) launch_history_view<kHistLdsHalf>(h, s.rows, s.max_history, stream);
+        else launch_history_view<kHistLdsWords>(h, s.rows, s.max_history, stream);
         if (launch_status() != VI_OK) return VI_ERR_LAUNCH;
     }
     for (int r0 = 0; r0 < s.rows; r0 += chunk) {
