@@ -5,7 +5,7 @@ The stream route serves the 16-bit full-route rows (temperature > 0, top_k 0 or
 oracle's except where a cumulative-mass boundary lies within 1e-6 of the drawn
 uniform or of a cut; support sizes, finite counts and flags equal
 outside exempt rows; Philox uniforms bit-exact; support mass within 1e-6.
-Cases: vocabularies from 64 to 248,320 and part boundaries (65,528 tokens),
+Cases: vocabularies from 64 to 248,320 and part boundaries (parts of up to 65,504 tokens),
 one to 128 rows (one to sixteen parts per row), caps above 64, min-p, top-p,
 ties, non-finite and empty rows, signed zeros, logits outside the fast
 division's range, temperatures whose z overflows, repetition / presence /

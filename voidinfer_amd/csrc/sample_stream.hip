@@ -5,9 +5,11 @@
 // (tokens, uniforms, stats, recording into penalty states, on request the
 // filtered distribution) and verification's (the distributions' bounds).
 // (Rows with an odd vocabulary, probabilities or bounds had kernels of their own,
-// which named the support's end by ranks: verification of 8 lanes x 16 drafts over
-// 248,320 tokens, bf16 and fp16, takes 134 us this way and 232 that way;
-// 56 x 66,181 bf16 26 and 54.)
+// which named the support's end by ranks.  This way / that way, us per call:
+// verification of 8 lanes x 16 drafts over 248,320 tokens, bf16 and fp16, 127 / 229;
+// 24 x 65,537 fp16 with probabilities 68 / 93; 56 x 66,181 bf16, odd, no penalties
+// 29.7 / 28.3; 2 x 248,319 bf16, odd, 500-token histories 37.6 / 33.3: few odd rows
+// pay for the history view's launch.)
 //
 // Key fact: bf16 / fp16 logits, and penalized logits stored back in the same
 // dtype, take one of 65,536 bit patterns, and z = x' * (1/T) is a strictly
@@ -16,7 +18,7 @@
 // patterns; every truncation and the draw are prefix sums over the occupied
 // patterns in key order, with one exp per occupied pattern, not per token.
 //
-// Stream launch (stream_kernel).  A row is cut into P parts of at most 65,528
+// Stream launch (stream_kernel).  A row is cut into P parts of at most 65,504
 // tokens, so a part's count of one pattern fits 16 bits.  Persistent
 // workgroups of 1024 threads (one per CU: the histogram takes 128 KB of LDS)
 // take the parts of their XCD's rows in a fixed order, with the next part's
@@ -134,7 +136,7 @@ struct StreamArgs {
     FullBound* bounds;         // [rows] (or null): the rows' filtered distributions
     int draw_every;            // rows whose token is drawn: every one (1), every n-th (row % n == n - 1), none (0)
     int row0;                  // row 0's number in the call (a call of very many rows takes several launches)
-    // the parts' tables: header (occupied-group bitmap, highest valid key) and
+    // the parts' tables: header (the occupied groups' bitmaps, by sign) and
     // the occupied groups' 32 words at their place
     uint32_t* ppub;            // [rows * parts][kPub]
     uint4* pwords;             // [rows * parts][kGroups][8]
@@ -1564,9 +1566,10 @@ __global__ __launch_bounds__(kT) void history_view_kernel(HistArgs h) {
 // are listed over all its rounds and penalized one per lane with count 1 (where
 // they lie, nearly every wave would run the penalty for nearly every logit of a
 // lane); the tokens seen more than once are written again by repeat_probs_kernel.
-// (24 / 128 x 151,936 bf16, 2,048-token histories: 11.7 / 38.3 us with two rounds,
-// 11.0 / 40.5 with one, 14.0 / 40.4 with four, and 3.9 / 4.8 for the repeats; 24 rows took 48.6 us with eight logits per thread, each slice's
-// penalties rebuilt in LDS and end-key ranks counted.)
+// (24 x 151,936 bf16, 2,048-token histories: 12.4 us, and 4.6 for the repeats; 48.6 with
+// eight logits per thread, each slice's penalties rebuilt in LDS and end-key ranks
+// counted.  Two rounds: with a cheaper exponential, 24 / 128 rows took 11.7 / 38.3 us,
+// 11.0 / 40.5 with one round, 14.0 / 40.4 with four.)
 constexpr int kPT = 256;                          // threads
 constexpr int kPRounds = 2;
 constexpr int kPChunk = kPT * kPRounds * 4;       // logits per workgroup

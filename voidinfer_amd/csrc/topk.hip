@@ -94,7 +94,7 @@ struct TopkArgs {
     float* probs;
     int64_t probs_stride;
     vi_sample_stats* stats;
-    int full_rows_unsupported;  // fp32 logits: rows outside the top-k route fail
+    int full_rows_unsupported;  // rows outside the top-k route fail (no full-vocabulary route takes the shape)
     int pres_words;         // dynamic LDS words for the slice's history-presence bitmap (0: none)
     int hist_counts;        // the dynamic words are the slice's history counts, one per token, counted
                             // from the histories by every workgroup of the row (no hash)
@@ -2058,10 +2058,9 @@ vi_status launch_sample(const SampleArgs& s, void* ws, size_t ws_bytes, hipStrea
         a.pstate = s.pstate; a.pl = s.playout; a.record = s.record;
         a.tokens = s.tokens; a.uniforms = s.uniforms; a.probs = s.probs; a.probs_stride = s.probs_stride;
         a.stats = s.stats;
-        // fp32 logits / unaligned rows: full-route rows fail loudly in the top-k launch
-        a.full_rows_unsupported = (full_ok && (s.route_mask & VI_ROUTE_FULL)) ? 0 : (full_ok ? 0 : 1);
-        st = launch_mode<kModeSample>(a, s.dtype, s.rows, plan.slices,
-                                      topk_stream);
+        // a vocabulary past the full routes' limit: their rows fail loudly in the top-k launch
+        a.full_rows_unsupported = full_ok ? 0 : 1;
+        st = launch_mode<kModeSample>(a, s.dtype, s.rows, plan.slices, topk_stream);
         if (st != VI_OK && !side) return st;
     }
     if (full_run) {
